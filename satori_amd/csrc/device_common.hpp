@@ -12,6 +12,7 @@ namespace satori {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Loads through the global address space (global_load_* rather than flat_*): every pointer the kernels

@@ -1,30 +1,38 @@
-// Many-position FP32-activation product for Q8_0 and Q4_0 on the matrix cores (gfx950 bf16 MFMA): the
+// Several-position FP32-activation product for Q8_0 and Q4_0 on the matrix cores (gfx950 bf16 MFMA): the
 // batched form of QuantizedMatVec.ExecuteBatch for the legacy formats (ExecuteBatchFloat / ExecuteBatchRows,
 // src/Satori.Core/QuantizedMatVec.cs:221-347), with the arithmetic of the scalar reference per block
 // (QuantizedMatVec.ExecuteScalar, QuantizedMatVec.cs:45-78: sum = q . x over the block's 32 weights, then
-// total += Scale * sum), so the weights are read once per 32-position tile instead of once per position.
+// total += Scale * sum), so the weights are read once per position tile instead of once per position.
 //
-// Exact operands. A block's codes q are small integers (Q8_0: -128..127; Q4_0: -8..7), exact in bf16. Each
-// activation x is split into three bf16 parts x = hi + lo + lolo, each the next 8 significant bits cut by
-// truncation (x - hi and (x - hi) - lo are exact in FP32, and the last part has at most 8 significant bits).
-// bf16 has FP32's exponent range, but a part below 2^-126 would be a bf16 subnormal: its bits below 2^-133 do
-// not fit and the matrix cores may flush it. So each position is first lifted by an exact power of two 2^k
-// (k >= 0) that brings its largest |x| into [2^64, 2^65). Every nonzero bit of a lifted x then weighs at least
-// 2^(-149 + k); in a position whose largest |x| is below 2^42 (k >= 23) every nonzero part is a normal bf16,
-// so the split is exact for every finite element, subnormals included. In a position with a larger |x| a
-// part can be subnormal only for an element below 2^-174 of the largest. From 2^64 on k = 0, so a product
-// that overflows in the reference overflows here too. An infinite or NaN x keeps k = 0 for its position and
-// keeps itself as hi (a NaN as the canonical quiet NaN) with zero lo and lolo, so q * x gives the IEEE
-// result of the single product. Every q * part product is exact in FP32 (at most 16 significant bits), the
-// sums of a lifted position stay below 2^120, and the block sum sum_k q_k x_k is three bf16 MFMA chains
-// accumulating in FP32. Only the FP32 additions round, in an order of their own, and the final scaling by
-// 2^-k rounds once where the result is subnormal: within 1e-5 * sum |w x| + n * 2^-149 of the reference,
-// like every FP32 path here.
+// Exact operands. A block's codes q are small integers (Q8_0: -128..127; Q4_0: -8..7, used as 16 q), exact in
+// bf16. Each activation x is split into three bf16 parts x = hi + lo + lolo, each the next 8 significant bits
+// cut by truncation (x - hi and (x - hi) - lo are exact in FP32, and the last part has at most 8 significant
+// bits). bf16 has FP32's exponent range, but a part below 2^-126 would be a bf16 subnormal: its bits below
+// 2^-133 do not fit and the matrix cores may flush it. So every x is first lifted by 2^24: every bit of a
+// lifted FP32 number, subnormals included, weighs at least 2^-125, and the split is exact for every finite x.
+// Every q * part product is exact in FP32 (at most 16 significant bits), and the block sum sum_k q_k x_k is
+// three bf16 MFMA chains accumulating in FP32. Only the FP32 additions round, in an order of their own, and the
+// final scaling by 2^-24 rounds once where the result is subnormal: within 1e-5 * sum |w x| + n * 2^-149 of
+// the reference, like every FP32 path here. A lifted sum stays below 2^118 while |x| < 2^40 (2^26 blocks of the
+// largest code and scale); a position holding a larger, infinite or NaN activation is flagged while it is
+// split, and its outputs are computed by a plain FP32 loop instead (finish_flagged), which overflows and
+// propagates where the reference does.
 //
-// Three launches: fbatch_lift_kernel finds each position's lifting exponent, fbatch_pack_kernel splits the
-// lifted activations into a workspace in MFMA first-operand order, and fbatch_kernel runs the product: waves
-// of 32-row x 32-position tiles, four row tiles per workgroup sharing the split activations staged in LDS a
-// round of W blocks at a time, one block of the round per way.
+// Launches. fbatch_kernel: a workgroup of eight waves walks (row group, position unit) tiles of 64 RH rows x 32 TP
+// positions, WAYS = 8 / RH blocks a round: each wave owns 64 rows x 32 TP positions of one of the round's blocks, and
+// the ways' sums are added at the end of the tile. The tiles' rounds are dealt to one workgroup per CU in equal
+// contiguous ranges (the chip is full and ends together whatever the shape: 4096 x 4096 over 256 positions has 64
+// tiles, over 12 positions 32); a tile cut between workgroups goes through partial sums in the workspace, added by
+// fbatch_fixup_kernel. Up to 64 positions (one position unit) the activations are split by the workgroups that
+// use them (FUSED, 128 rows and four ways); more positions are split once by fbatch_pack_kernel into the workspace,
+// since every row group would split them again, and take 256 rows and two ways: twice the rows halve the parts'
+// bytes a workgroup reads, which then bound it (128 rows: 1.3 GB through L2 in 94 us at 11008 x 4096 Q4_0 over 256
+// positions; 256 rows 0.83 GB).
+// Measured, whole call in a queue of calls (us, before: one 32 x 32 tile per wave and block, its workgroups one
+// per 128 rows and position tile): 256 positions 11008 x 4096 Q4_0 152 -> 83, 4096 x 4096 Q8_0 64 -> 41, 256 x 14336
+// Q8_0 195 -> 27; 64 positions 4096 x 4096 Q8_0 62 -> 18; 12 positions (the single-position kernel) 29 -> 14.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -34,164 +42,97 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kTile = 32;      // rows and positions per wave tile
+constexpr int kTile = 32;                              // rows and positions of one matrix-core tile
+constexpr int kThreads = 256;                          // of the pack and fix-up kernels
 constexpr int kPartBytes = 1024;                       // one part of one K step of one (block, tile)
 constexpr int kBlockTileBytes = 3 * 2 * kPartBytes;    // 3 parts x 2 K steps of 16 columns
+constexpr float kLift = 0x1p24f;
+constexpr int kLiftExponent = 24;
+constexpr uint32_t kFlagBits = 0x5F80u;                // a lifted part of 2^64: |x| from 2^40 on (infinite, NaN) is flagged
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// Workspace: for 32-column block b and 32-position tile t, 6 KB at (b * tiles + t) * 6144: part s (0: hi,
-// 1: lo, 2: lolo), K step st (columns 32b + 16st .. + 15) at (2s + st) * 1024, lane l = 32h + p holding the
-// 8 bf16 of position 32t + p, columns 32b + 16st + 8h .. + 7. Positions past the last are zero. After the
-// blocks x tiles records: one int32 lifting exponent k per position (tiles x 32 of them, zero past the last).
-
-// The exponent k lifting the largest |x| of a position into [2^64, 2^65), from the largest magnitude's FP32
-// bits: 0 for a zero or non-finite position, and for magnitudes of 2^64 and more.
-__device__ __forceinline__ int lift_exponent(uint32_t max_bits) {
-    if (max_bits == 0u || max_bits >= 0x7F800000u) return 0;
-    const int e = max_bits >= 0x00800000u ? static_cast<int>(max_bits >> 23) - 127  // normal: floor(log2)
-                                          : (31 - __clz(static_cast<int>(max_bits))) - 149;  // subnormal
-    return e >= 64 ? 0 : 64 - e;
+// Workspace of the packed form: for 32-column block b and 32-position tile t, 6 KB at (b * tiles + t) * 6144:
+// part s (0: hi, 1: lo, 2: lolo), K step st at (2s + st) * 1024, lane l = 32h + p holding the 8 bf16 of position
+// 32t + p at columns 32b + slot_column(st, h) .. + 7. Positions past the last are zero. Then one word per (block,
+// tile, K step): the tile's flagged positions in that slot's columns. Then the partial sums.
+//
+// The columns of a block are dealt to the K steps so that a lane's codes are contiguous: Q8_0 lane half h
+// holds bytes 16h .. 16h + 15 of the record, Q4_0 bytes 8h .. 8h + 7 (low nibbles in step 0, high in step 1).
+template <int FORMAT>
+__device__ __forceinline__ int slot_column(int st, int h) {
+    return FORMAT == kQ8_0 ? 16 * h + 8 * st : 16 * st + 8 * h;
 }
 
-// One workgroup per position tile slot (32 per tile): the lifting exponent of position p (0 past the last).
-// Rows of 16-byte-aligned activations are read in 16-byte pieces, four per thread in flight.
-__global__ __launch_bounds__(256) void fbatch_lift_kernel(const float* __restrict__ x, int columns, int positions,
-                                                          int* __restrict__ lift) {
-    __shared__ uint32_t wave_max[4];
-    const int p = blockIdx.x;
-    uint32_t m = 0u;
-    if (p < positions) {
-        const float* row = x + static_cast<int64_t>(p) * columns;
-        uint32_t m1 = 0u, m2 = 0u, m3 = 0u;
-        const auto mag = [](uint32_t bits) { return bits & 0x7FFFFFFFu; };
-        if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) {  // rows are 128-byte multiples: all aligned
-            const int pieces = columns >> 2;
-            int i = threadIdx.x;
-            for (; i + 768 < pieces; i += 1024) {
-                const u32x4 a = *(const SATORI_GLOBAL u32x4*)(row + 4 * i);
-                const u32x4 b = *(const SATORI_GLOBAL u32x4*)(row + 4 * (i + 256));
-                const u32x4 c = *(const SATORI_GLOBAL u32x4*)(row + 4 * (i + 512));
-                const u32x4 d = *(const SATORI_GLOBAL u32x4*)(row + 4 * (i + 768));
+// Eight activations lifted and split into their bf16 parts, packed in pairs; true when one must be flagged.
+__device__ __forceinline__ bool split8(const float (&v)[8], u32x4 (&part)[3]) {
+    u16x2 largest = {0, 0};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    m = max(m, mag(a[e]));
-                    m1 = max(m1, mag(b[e]));
-                    m2 = max(m2, mag(c[e]));
-                    m3 = max(m3, mag(d[e]));
-                }
-            }
-            for (; i < pieces; i += 256) {
-                const u32x4 a = *(const SATORI_GLOBAL u32x4*)(row + 4 * i);
+    for (int e = 0; e < 8; e += 2) {
+        uint32_t p[3][2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) m = max(m, mag(a[e]));
-            }
-        } else {
-            for (int c = threadIdx.x; c < columns; c += 256) m = max(m, mag(__float_as_uint(load_f32(row + c))));
+        for (int i = 0; i < 2; ++i) {
+            const float x = __fmul_rn(v[e + i], kLift);
+            p[0][i] = __float_as_uint(x);
+            const float r = __fsub_rn(x, __uint_as_float(p[0][i] & 0xFFFF0000u));  // exact
+            p[1][i] = __float_as_uint(r);
+            p[2][i] = __float_as_uint(__fsub_rn(r, __uint_as_float(p[1][i] & 0xFFFF0000u)));  // at most 8 bits
         }
-        m = max(max(m, m1), max(m2, m3));  // magnitudes order like their bits; NaN bits exceed every finite
-    }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off)));
-    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        lift[p] = lift_exponent(max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3])));
-}
-
-// The three bf16 parts of x (bit patterns in the low 16 bits).
-__device__ __forceinline__ void split3(float x, uint32_t& hi, uint32_t& lo, uint32_t& lolo) {
-    const uint32_t b = __float_as_uint(x);
-    if ((b & 0x7F800000u) == 0x7F800000u) {  // infinite or NaN
-        hi = (b & 0x007FFFFFu) ? (0x7FC0u | ((b >> 16) & 0x8000u)) : (b >> 16);
-        lo = lolo = 0u;
-        return;
+        for (int s = 0; s < 3; ++s) part[s][e >> 1] = __builtin_amdgcn_perm(p[s][1], p[s][0], 0x07060302u);
+        largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, part[0][e >> 1] & 0x7FFF7FFFu));
     }
-    const float h = __uint_as_float(b & 0xFFFF0000u);
-    const float r = __fsub_rn(x, h);  // exact: the bits of x below its top eight
-    const uint32_t rb = __float_as_uint(r);
-    const float l = __uint_as_float(rb & 0xFFFF0000u);
-    const float ll = __fsub_rn(r, l);  // exact, at most eight significant bits
-    hi = b >> 16;
-    lo = rb >> 16;
-    lolo = __float_as_uint(ll) >> 16;
+    return max(largest[0], largest[1]) >= kFlagBits;
 }
 
-// One thread per (block, position tile, K step, lane): the 8 activations of its operand slot, split.
-__global__ __launch_bounds__(256) void fbatch_pack_kernel(const float* __restrict__ x, int columns, int positions,
-                                                          int tiles, uint8_t* __restrict__ workspace,
-                                                          const int* __restrict__ lift) {
-    const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+__device__ __forceinline__ void load8(const float* src, float (&v)[8]) {
+    const u32x4 a = load16_a4(reinterpret_cast<const uint8_t*>(src));
+    const u32x4 b = load16_a4(reinterpret_cast<const uint8_t*>(src + 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = __uint_as_float(a[e]);
+        v[4 + e] = __uint_as_float(b[e]);
+    }
+}
+
+// One wave per (block, position tile, K step), lane by lane the 8 activations of its operand slot, split.
+template <int FORMAT>
+__global__ __launch_bounds__(kThreads) void fbatch_pack_kernel(const float* __restrict__ x, int columns, int positions,
+                                                               int tiles, uint8_t* __restrict__ parts,
+                                                               uint32_t* __restrict__ flags) {
+    const int64_t item = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     const int blocks = columns / 32;
-    if (item >= static_cast<int64_t>(blocks) * tiles * 128) return;
+    if (item >= static_cast<int64_t>(blocks) * tiles * 128) return;  // whole waves
     const int lane = static_cast<int>(item & 63), st = static_cast<int>((item >> 6) & 1);
     const int64_t bt = item >> 7;  // b * tiles + t
     const int b = static_cast<int>(bt / tiles), t = static_cast<int>(bt - static_cast<int64_t>(b) * tiles);
     const int p = t * kTile + (lane & 31);
-    const int c0 = 32 * b + 16 * st + 8 * (lane >> 5);
-    uint32_t part[3][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-    if (p < positions) {
-        const float* src = x + static_cast<int64_t>(p) * columns + c0;
-        const int k = lift[p];
-        float v[8];
-        if ((reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-            const u32x4 a = *(const SATORI_GLOBAL u32x4*)(src), c = *(const SATORI_GLOBAL u32x4*)(src + 4);
+    float v[8];
+    load8(x + static_cast<int64_t>(min(p, positions - 1)) * columns + 32 * b + slot_column<FORMAT>(st, lane >> 5), v);
+    if (p >= positions)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = __uint_as_float(a[e]);
-                v[4 + e] = __uint_as_float(c[e]);
-            }
-        } else {
+        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+    u32x4 part[3];
+    const uint64_t flagged = __ballot(split8(v, part));
+    uint8_t* dst = parts + bt * kBlockTileBytes + st * kPartBytes + 16 * lane;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = load_f32(src + e);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            uint32_t h, l, ll;
-            split3(__builtin_amdgcn_ldexpf(v[e], k), h, l, ll);  // exact: the lifted value is at most 2^65
-            const int shift = 16 * (e & 1);
-            part[0][e >> 1] |= h << shift;
-            part[1][e >> 1] |= l << shift;
-            part[2][e >> 1] |= ll << shift;
-        }
-    }
-    uint8_t* dst = workspace + bt * kBlockTileBytes + st * kPartBytes + 16 * lane;
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-        *reinterpret_cast<u32x4*>(dst + 2 * s * kPartBytes) = u32x4{part[s][0], part[s][1], part[s][2], part[s][3]};
+    for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(dst + 2 * s * kPartBytes) = part[s];
+    if (lane == 0) flags[2 * bt + st] = static_cast<uint32_t>(flagged) | static_cast<uint32_t>(flagged >> 32);
 }
 
 // Two small integers as a pair of bf16 (exact: at most 8 significant bits): the high halves of their FP32
-// patterns, q0 low, joined by one byte permute.
-__device__ __forceinline__ uint32_t pack_bf16(int q0, int q1) {
-    return __builtin_amdgcn_perm(__float_as_uint(static_cast<float>(q1)), __float_as_uint(static_cast<float>(q0)),
+// patterns, byte i low, joined by one byte permute.
+__device__ __forceinline__ uint32_t pack_bytes(uint32_t w, int i) {
+    return __builtin_amdgcn_perm(__float_as_uint(sbyte_to_float(w, i + 1)), __float_as_uint(sbyte_to_float(w, i)),
                                  0x07060302u);
 }
 
-// The lane's second operand (8 codes of its row) for K step st of a block, from the device layout: Q8_0
-// records are the 32 signed bytes; Q4_0 records hold q - 8 per nibble (byte j: low nibble weight j, high
-// nibble weight j + 16), so step 0 takes low nibbles and step 1 high nibbles of bytes 8h .. 8h + 7.
+// Pair k % 4 of the lane's second operand (8 codes of its row) for K step k / 4 of a block: Q8_0 from its 16
+// signed bytes, Q4_0 from its 8 nibble bytes (each nibble q - 8 in two's complement) as the bytes 16 (q - 8).
 template <int FORMAT>
-__device__ __forceinline__ bf16x8 codes_operand(const uint32_t (&raw)[4], int st) {
-    uint32_t d[4];
-    if constexpr (FORMAT == kQ8_0) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t w = raw[2 * st + k];
-            d[2 * k] = pack_bf16(static_cast<int8_t>(w), static_cast<int8_t>(w >> 8));
-            d[2 * k + 1] = pack_bf16(static_cast<int8_t>(w >> 16), static_cast<int8_t>(w >> 24));
-        }
-    } else {
-        const int shift = 4 * st;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t w = raw[k];
-            auto nib = [&](int byte) {
-                return __builtin_amdgcn_sbfe(static_cast<int>(w), 8 * byte + shift, 4);  // q - 8, sign-extended
-            };
-            d[2 * k] = pack_bf16(nib(0), nib(1));
-            d[2 * k + 1] = pack_bf16(nib(2), nib(3));
-        }
-    }
-    return __builtin_bit_cast(bf16x8, u32x4{d[0], d[1], d[2], d[3]});
+__device__ __forceinline__ uint32_t code_pair(const uint32_t (&raw)[4], int k) {
+    if constexpr (FORMAT == kQ8_0) return pack_bytes(raw[k >> 1], 2 * (k & 1));
+    const uint32_t w = raw[k >> 1 & 1];
+    return pack_bytes((k < 4 ? w << 4 : w) & 0xF0F0F0F0u, 2 * (k & 1));
 }
 
 __device__ __forceinline__ f32x16 mfma_bf16(const bf16x8& a, const bf16x8& b, const f32x16& c) {
@@ -199,203 +140,537 @@ __device__ __forceinline__ f32x16 mfma_bf16(const bf16x8& a, const bf16x8& b, co
 }
 
 struct FbatchArgs {
-    const uint8_t* w;          // device layout (code records, then FP16 scales)
-    const uint8_t* workspace;  // split activations (fbatch_pack_kernel)
-    const int* lift;           // per position: the exponent its activations were lifted by
-    float* y;                  // [positions][rows]
+    const uint8_t* w;       // device layout (code records, then FP16 scales)
+    const float* x;         // [positions][columns]
+    const uint8_t* parts;   // packed form: split activations
+    const uint32_t* flags;  // packed form: flagged positions per (block, tile, K step)
+    float* partial;         // two slots per workgroup: the cut tiles at the ends of its range
+    uint32_t* slot_flags;   // fused form: flagged positions found by a piece (TP words a slot)
+    uint32_t* tile_flags;   // fused form: flagged positions of a tile that was not cut (TP words a tile)
+    float* y;               // [positions][rows]
     int rows, blocks, positions, tiles;
+    int units;              // position units: ceil(tiles / TP)
+    int rounds;             // rounds per tile: ceil(blocks / 2)
+    int total;              // tiles x rounds
+    int workgroups;         // ranges: the first total % workgroups hold total / workgroups + 1 rounds, the others one less
+    int share, longer;      // total / workgroups, total % workgroups
 };
 
-// Workgroup u of the padded grid: units (row group of four row tiles, position tile), position tiles fastest,
-// consecutive units on one XCD (workgroup ids are dealt to the eight XCDs in turn), so the position tiles
-// that share a row group's weights read them through one L2. W ways per row tile: a round stages W
-// consecutive blocks' split activations once for the workgroup, and way w of each row tile computes the
-// round's block w, so the four row tiles share every staged byte and the workgroup keeps 4 W waves busy.
-// Each way sums its own blocks; the ways' sums are added once at the end, in way order.
-template <int FORMAT, int W>
-__global__ __launch_bounds__(256 * W) void fbatch_kernel(FbatchArgs a) {
+// Floats of one partial slot: [row half][row tile][position tile][output / 4][lane][output % 4].
+constexpr int slot_floats(int TP, int RH) { return 2 * RH * TP * 1024; }
+
+// First round of range i of the launch, and the range that holds round r.
+__device__ __forceinline__ int range_start(const FbatchArgs& a, int i) { return a.share * i + min(i, a.longer); }
+__device__ __forceinline__ int range_of(const FbatchArgs& a, int r) {
+    const int in_longer = a.longer * (a.share + 1);
+    return r < in_longer ? r / (a.share + 1) : a.longer + (r - in_longer) / a.share;
+}
+
+// Outputs of the flagged positions of one 32-row x 32-position tile, by 256 threads: eight per row, each the plain
+// FP32 block sums (QuantizedMatVec.cs:45-78) of every eighth block, their totals then added in order.
+template <int FORMAT>
+__device__ void finish_flagged(const FbatchArgs& a, int row0, int p0, uint32_t mask, float* totals) {
     constexpr int kRecord = FORMAT == kQ8_0 ? 32 : 16;
-    constexpr int kThreads = 256 * W;
-    constexpr int kRoundBytes = W * kBlockTileBytes;
-    constexpr int kChunks = kRoundBytes / 16;                                // 16-byte pieces staged per round
-    constexpr int kLoads = (kChunks + kThreads - 1) / kThreads;
-    constexpr int kSumBytes = (W - 1) * 4 * 16 * 64 * 4;                    // the ways' sums at the end
-    __shared__ uint8_t lds[2 * kRoundBytes > kSumBytes ? 2 * kRoundBytes : kSumBytes];  // two rounds' buffers
+    const int tid = threadIdx.x, row = row0 + (tid & 31), share = tid >> 5;
+    const int64_t count = static_cast<int64_t>(a.rows) * a.blocks;
+    const int64_t first = static_cast<int64_t>(min(row, a.rows - 1)) * a.blocks;
+    for (; mask; mask &= mask - 1u) {
+        const int p = p0 + __builtin_ctz(mask);
+        if (p >= a.positions) break;
+        if (tid < 256) {
+            float total = 0.0f;
+            for (int b = share; b < a.blocks; b += 8) {
+                const uint8_t* rec = a.w + (first + b) * kRecord;
+                const float* xb = a.x + static_cast<int64_t>(p) * a.blocks * 32 + 32 * b;
+                const u32x4 lo = load16_a4(rec);
+                const u32x4 hi = FORMAT == kQ8_0 ? load16_a4(rec + 16) : lo;
+                const float scale = half_bits_to_float(load2_a2(a.w + count * kRecord + (first + b) * 2));
+                float sum = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 32; ++j) {
+                    float q;
+                    if constexpr (FORMAT == kQ8_0)
+                        q = sbyte_to_float(j < 16 ? lo[j >> 2] : hi[(j >> 2) - 4], j & 3);
+                    else  // bytes 16 (q - 8), the low nibbles first
+                        q = 0.0625f * sbyte_to_float((j < 16 ? lo[j >> 2] << 4 : lo[(j >> 2) - 4]) & 0xF0F0F0F0u, j & 3);
+                    sum = __fadd_rn(sum, __fmul_rn(q, load_f32(xb + j)));
+                }
+                total = __fadd_rn(total, __fmul_rn(scale, sum));
+            }
+            totals[tid] = total;
+        }
+        __syncthreads();
+        if (tid < 32 && row < a.rows) {
+            float total = totals[tid];
+            for (int i = 1; i < 8; ++i) total = __fadd_rn(total, totals[tid + 32 * i]);
+            store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, total);
+        }
+        __syncthreads();
+    }
+}
 
-    const int per_xcd = gridDim.x >> 3;
-    const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    const int groups = (a.rows + 4 * kTile - 1) / (4 * kTile);
-    if (u >= groups * a.tiles) return;  // whole workgroup
-    const int group = u / a.tiles, t = u - group * a.tiles;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5;
-    const int rt = wave & 3, way = wave >> 2;
-    const int row = (group * 4 + rt) * kTile + (lane & 31);
-    const int row_c = row < a.rows ? row : a.rows - 1;  // rows past the last compute on a live row, store nothing
+// What bounds it: the matrix cores at many positions (6 MFMAs of 32 cycles per 32 x 32 tile and block), then the
+// staged activations' way from L2 (a 128-row tile reads 6 KB of parts per 32 positions and block); at few
+// positions the weights from HBM. A wave's 64-row x 64-position tile reuses each LDS read of the parts for two row
+// tiles and each converted code for two position tiles, so that neither the LDS (3.5 KB a tile and block) nor
+// the vector ALU (16 FMAs and 12-15 conversions) is ahead of the matrix cores.
+// Ranges are dealt so that consecutive ones, which share rows of weights, run on one XCD (workgroup ids go
+// round-robin over the eight).
+template <int FORMAT, int TP, bool FUSED, int RH, int WAYS>
+__global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a) {
+    constexpr int kThreads = 64 * RH * WAYS, kGroupRows = 64 * RH;
+    static_assert(FUSED ? 2 * TP % RH == 0 : WAYS == 2, "staging passes");
+    constexpr int kAhead = FUSED && TP == 1 ? 2 : 1;  // rounds in registers on their way into the LDS
+    constexpr int kRecord = FORMAT == kQ8_0 ? 32 : 16;
+    constexpr int kPieces = FORMAT == kQ8_0 ? 2 : 1;                 // 16-byte pieces of a record
+    constexpr int kPlane = kGroupRows * 16 + 16;                     // one piece of every row, padded off its banks
+    constexpr int kUnitBytes = TP * kBlockTileBytes;
+    constexpr int kXBytes = WAYS * kUnitBytes;
+    constexpr int kRoundBytes = kXBytes + WAYS * kPieces * kPlane;
+    constexpr int kSlots = 2 * TP / RH;                              // fused form: operand slots per thread
+    constexpr int kScaleRounds = 8 / WAYS;                           // rounds whose scales are staged together
+    constexpr int kXLoads = kXBytes / 16 / kThreads;                 // packed form: pieces per thread
+    __shared__ __align__(16) uint8_t lds[2 * kRoundBytes];
+    __shared__ __align__(16) uint8_t lds_scales[2 * kGroupRows * 16];
+    __shared__ uint32_t lds_flags[TP];
+
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    const int rh = (tid >> 6) % RH, way = (tid >> 6) / RH;
+    const int per_xcd = a.workgroups >> 3;
+    const int range = (a.workgroups & 7) == 0 ? (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
+    const int end = range_start(a, range + 1);
     const int blocks = a.blocks;
-    const int64_t count = static_cast<int64_t>(a.rows) * blocks;
-    const uint8_t* records = a.w + static_cast<int64_t>(row_c) * blocks * kRecord + 8 * h;
-    const uint8_t* scales = a.w + count * kRecord + static_cast<int64_t>(row_c) * blocks * 2;
-    const uint8_t* parts = a.workspace + static_cast<int64_t>(t) * kBlockTileBytes;
-    const int64_t part_stride = static_cast<int64_t>(a.tiles) * kBlockTileBytes;  // block b to b + 1
+    const uint8_t* scales = a.w + static_cast<int64_t>(a.rows) * blocks * kRecord;
 
-    // Staging of round k (blocks W k .. W k + W - 1): thread i copies the 16-byte pieces i, i + threads, ...
-    // Piece c of a round lies in block W k + c_blk of the round; its address steps by W blocks a round (an
-    // addition, not a 64-bit multiply), and a block past the last reads the last one instead (unused).
-    u32x4 st_regs[kLoads];
-    const uint8_t* st_ptr[kLoads];
-    const uint8_t* st_last[kLoads];
-    int st_blk[kLoads];
+    for (int at = range_start(a, range); at < end;) {
+        const int tile = at / a.rounds, r0 = at - tile * a.rounds, r1 = min(a.rounds, r0 + (end - at));
+        const int group = tile / a.units, t0 = (tile - group * a.units) * TP;  // row group, first position tile
+        const int row0 = group * kGroupRows;
+
+        // ---- staging: this thread's pieces of a round (blocks 2r and 2r + 1; a second block past the last reads the
+        // first again, and is not computed). Addresses are a uniform base per round and a fixed 32-bit offset (a
+        // payload is at most 2^31 - 1 bytes). ----
+        u32x4 wregs[kAhead][kPieces];
+        uint32_t woff[kPieces];
+        constexpr int kRowPieces = WAYS * kPieces;  // of one row in a round: consecutive bytes
+        const int wblk = tid % kRowPieces / kPieces;
 #pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-        const int off = 16 * (threadIdx.x + kThreads * j);
-        st_blk[j] = off / kBlockTileBytes;
-        st_ptr[j] = parts + st_blk[j] * part_stride + off % kBlockTileBytes;
-        st_last[j] = parts + (blocks - 1) * part_stride + off % kBlockTileBytes;
-    }
-    auto stage_load = [&](int k) {
+        for (int j = 0; j < kPieces; ++j)
+            woff[j] = static_cast<uint32_t>(min(row0 + (tid + kThreads * j) / kRowPieces, a.rows - 1)) * blocks * kRecord +
+                      16 * (tid % kRowPieces);
+        const int wdst = kXBytes + tid % kRowPieces * kPlane + tid / kRowPieces * 16;
+        u32x4 xregs[kAhead][FUSED ? 2 * kSlots : kXLoads];
+        bool flagged[TP] = {};
+        const uint8_t* xsrc[TP];
+        if constexpr (FUSED) {  // slots (position tile, block, K step (tid / 64) % 2, lane), the threads' passes in that order
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            if (threadIdx.x + kThreads * j < kChunks) {
-                const uint8_t* src = W * k + st_blk[j] < blocks ? st_ptr[j] : st_last[j];
-                st_regs[j] = *(const SATORI_GLOBAL u32x4*)(src);
+            for (int j = 0; j < TP; ++j)
+                xsrc[j] = reinterpret_cast<const uint8_t*>(
+                    a.x + static_cast<int64_t>(min((t0 + j) * kTile + (lane & 31), a.positions - 1)) * blocks * 32 +
+                    slot_column<FORMAT>((tid >> 6) & 1, h));
+        }
+        auto slot_tile = [](int j) { return j * kThreads / 128 / WAYS; };
+        auto slot_block = [&](int j) { return (tid >> 7) + j * kThreads / 128 % WAYS; };
+        auto load_round = [&](int r, u32x4 (&wreg)[kPieces], u32x4 (&xreg)[FUSED ? 2 * kSlots : kXLoads]) {
+            const int last = blocks - 1 - WAYS * r;  // the round's last block
+            const uint8_t* wbase = a.w + static_cast<int64_t>(WAYS * r) * kRecord;
+            const uint32_t back = static_cast<uint32_t>(wblk - min(wblk, last)) * kRecord;
+#pragma unroll
+            for (int j = 0; j < kPieces; ++j) wreg[j] = *(const SATORI_GLOBAL u32x4*)(wbase + (woff[j] - back));
+            if constexpr (FUSED) {
+#pragma unroll
+                for (int j = 0; j < kSlots; ++j) {
+                    const int64_t b = WAYS * r + min(slot_block(j), last);
+                    xreg[2 * j] = load16_a4(xsrc[slot_tile(j)] + b * 128);
+                    xreg[2 * j + 1] = load16_a4(xsrc[slot_tile(j)] + b * 128 + 16);
+                }
+            } else {
+                // The unit's position tiles of a block are adjacent: piece c of the round is byte 16 (c % pieces) of
+                // block c / pieces.
+                constexpr int kPiecesX = kUnitBytes / 16;
+                const uint32_t stride = static_cast<uint32_t>(a.units) * kUnitBytes, second = last > 0 ? stride : 0u;
+                const uint8_t* base = a.parts + static_cast<int64_t>(WAYS * r) * stride + (t0 / TP) * kUnitBytes;
+#pragma unroll
+                for (int j = 0; j < kXLoads; ++j) {
+                    const int c = tid + kThreads * j;
+                    xreg[j] = *(const SATORI_GLOBAL u32x4*)(base + (c < kPiecesX ? 16u * c : 16u * (c - kPiecesX) + second));
+                }
             }
-            st_ptr[j] += W * part_stride;
-        }
-    };
-    auto stage_store = [&](uint8_t* buf) {
+        };
+        auto store_round = [&](uint8_t* buf, const u32x4 (&wreg)[kPieces], const u32x4 (&xreg)[FUSED ? 2 * kSlots : kXLoads]) {
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) {
-            const int c = threadIdx.x + kThreads * j;
-            if (c < kChunks) *reinterpret_cast<u32x4*>(buf + 16 * c) = st_regs[j];
-        }
-    };
-    // The lane's codes and scale of block b (clamped to the last block, read and unused past it).
-    struct Weights {
-        uint32_t raw[4];
-        uint32_t scale;
-    };
-    auto load_weights = [&](int b, Weights& wgt) {
-        const int bc = min(b, blocks - 1);
-        const uint8_t* rec = records + bc * kRecord;  // within one row: 32-bit offsets
-        const uint64_t lo8 = load8_a8(rec);
-        wgt.raw[0] = static_cast<uint32_t>(lo8);
-        wgt.raw[1] = static_cast<uint32_t>(lo8 >> 32);
-        if constexpr (FORMAT == kQ8_0) {
-            const uint64_t hi8 = load8_a8(rec + 16);
-            wgt.raw[2] = static_cast<uint32_t>(hi8);
-            wgt.raw[3] = static_cast<uint32_t>(hi8 >> 32);
-        }
-        wgt.scale = load2_a2(scales + 2 * bc);
-    };
-
-    float acc[16];
+            for (int j = 0; j < kPieces; ++j)
+                *reinterpret_cast<u32x4*>(buf + wdst + j * (kThreads / kRowPieces) * 16) = wreg[j];
+            if constexpr (FUSED) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    // One block: total += Scale * sum (QuantizedMatVec.cs:74), the product and the sum rounded apart.
-    auto block = [&](const Weights& wgt, const uint8_t* sb) {
-        f32x16 d = {};
+                for (int j = 0; j < kSlots; ++j) {
+                    const int t = slot_tile(j);
+                    float v[8];  // (positions past the last are the last one again: computed, never stored)
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            const bf16x8 w = codes_operand<FORMAT>(wgt.raw, st);
+                    for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(xreg[2 * j + (e >> 2)][e & 3]);
+                    u32x4 part[3];
+                    flagged[t] |= split8(v, part);
+                    uint8_t* dst = buf + (slot_block(j) * TP + t) * kBlockTileBytes + ((tid >> 6) & 1) * kPartBytes + 16 * lane;
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {
-                const bf16x8 x = *reinterpret_cast<const bf16x8*>(sb + (2 * s + st) * kPartBytes + 16 * lane);
-                d = mfma_bf16(x, w, d);
+                    for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(dst + 2 * s * kPartBytes) = part[s];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < kXLoads; ++j) *reinterpret_cast<u32x4*>(buf + 16 * (tid + kThreads * j)) = xreg[j];
             }
-        }
-        const float scale = half_bits_to_float(wgt.scale);
+        };
+        // The rows' scales of eight blocks (four rounds) at a time, 16 bytes a row (2-byte aligned; up to 14 bytes past
+        // the last row's end, inside the payload's slack): one line read per row and four rounds, where two bytes a lane
+        // and round took half of the kernel's L2 requests.
+        u32x4 sreg;
+        const uint8_t* ssrc = scales + static_cast<uint32_t>(min(row0 + tid % kGroupRows, a.rows - 1)) * blocks * 2u;
+        auto load_scales = [&](int g) { sreg = *(const SATORI_GLOBAL u32x4_a2*)(ssrc + 16 * min(g, (blocks - 1) >> 3)); };
+        auto store_scales = [&](int g) {
+            if (tid < kGroupRows) *reinterpret_cast<u32x4*>(lds_scales + ((g & 1) * kGroupRows + tid) * 16) = sreg;
+        };
+
+        // ---- rounds: computed from one LDS buffer while the next round is stored into the other and the one after
+        // it is on its way into registers ----
+        float acc[2][TP][16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(scale, d[i]));
-    };
-
-    // Two LDS buffers: round k is computed from buffer k & 1 while round k + 1's parts, loaded during round
-    // k - 1, are stored into the other and round k + 2's are loaded; the weights run two rounds ahead too.
-    const int rounds = (blocks + W - 1) / W;
-    Weights w0, w1, w2;
-    stage_load(0);
-    stage_store(lds);
-    stage_load(1);
-    load_weights(way, w0);
-    load_weights(W + way, w1);
-    __syncthreads();  // round 0 staged
-    for (int k = 0; k < rounds; ++k) {
-        uint8_t* cur = lds + (k & 1) * kRoundBytes;
-        load_weights(W * (k + 2) + way, w2);  // clamped to the last block past the end
-        if (W * k + way < blocks) block(w0, cur + way * kBlockTileBytes);
-        if (k + 1 < rounds) {
-            stage_store(lds + ((k + 1) & 1) * kRoundBytes);  // its buffer was last read in round k - 1
-            if (k + 2 < rounds) stage_load(k + 2);
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int tp = 0; tp < TP; ++tp)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[rt][tp][i] = 0.0f;
+        load_scales(r0 / kScaleRounds);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (r0 + u < r1) load_round(r0 + u, wregs[u], xregs[u]);
+        store_scales(r0 / kScaleRounds);
+        store_round(lds, wregs[0], xregs[0]);
+        load_scales(r0 / kScaleRounds + 1);
+        if (r0 + kAhead < r1) load_round(r0 + kAhead, wregs[0], xregs[0]);
+        for (int base = r0; base < r1; base += kAhead)
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {  // round r + 1 waits in register set (u + 1) % kAhead
+            const int r = base + u;
+            if (r >= r1) break;
+            uint8_t* cur = lds + ((r - r0) & 1) * kRoundBytes;
+            uint8_t* other = lds + ((r - r0 + 1) & 1) * kRoundBytes;
+            __syncthreads();  // round r staged; the other buffer is no longer read
+            // This way's operands of its block, requested before the staging so that they arrive behind it.
+            const bool live = WAYS * r + way < blocks;  // (a way without a block only takes part in the staging)
+            const uint8_t* xcur = cur + way * kUnitBytes + 16 * lane;
+            float scale[2];
+            uint32_t raw[2][4];
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) {
+                const int row = 64 * rh + 32 * rt + (lane & 31);
+                scale[rt] = half_bits_to_float(*reinterpret_cast<const uint16_t*>(
+                    lds_scales + ((r / kScaleRounds & 1) * kGroupRows + row) * 16 + 2 * (r % kScaleRounds * WAYS + way)));
+                if (FORMAT == kQ4_0) scale[rt] *= 0.0625f;  // (codes 16 q)
+                if constexpr (FORMAT == kQ8_0) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(cur + kXBytes + (2 * way + h) * kPlane + 16 * row);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) raw[rt][e] = v[e];
+                } else {
+                    const uint2 v = *reinterpret_cast<const uint2*>(cur + kXBytes + way * kPlane + 16 * row + 8 * h);
+                    raw[rt][0] = v.x;
+                    raw[rt][1] = v.y;
+                }
+            }
+            bf16x8 xa[6];
+#pragma unroll
+            for (int s = 0; s < 6; ++s) xa[s] = *reinterpret_cast<const bf16x8*>(xcur + s * kPartBytes);
+            if (r + 1 < r1) {
+                if ((r + 1) % kScaleRounds == 0) {
+                    store_scales((r + 1) / kScaleRounds);
+                    load_scales((r + 1) / kScaleRounds + 1);
+                }
+                store_round(other, wregs[(u + 1) % kAhead], xregs[(u + 1) % kAhead]);
+            }
+            if (r + 1 + kAhead < r1) load_round(r + 1 + kAhead, wregs[(u + 1) % kAhead], xregs[(u + 1) % kAhead]);
+            if (!live) continue;  // (its barrier is the next round's: every wave takes the same number)
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
+            // One product chain per (row tile, position tile). Each step issues one MFMA and, in its shadow, part of
+            // the vector work beside it: the second row tile's conversions under the first chain, then the
+            // previous tile's FMAs; each position tile's parts are read while the last chain on the one before
+            // runs. (Left to the compiler, the conversions and FMAs ran between the chains: MFMA and vector
+            // time added up: the loop without its staging took 58 us at 11008 x 4096 Q4_0 over 256 positions, 44 at the
+            // rate a loop of MFMAs with as many vector instructions beside them reaches.)
+            u32x4 wop[2][2];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) wop[0][k >> 2][k & 3] = code_pair<FORMAT>(raw[0], k);
+            f32x16 prev;
+#pragma unroll
+            for (int k = 0; k < 2 * TP; ++k) {
+                const int rt = k & 1, tp = k >> 1;
+                f32x16 d = {};
+#pragma unroll
+                for (int s = 0; s < 6; ++s) {
+                    d = mfma_bf16(xa[s], __builtin_bit_cast(bf16x8, wop[rt][s & 1]), d);
+                    if (k == 0) {
+                        if (s < 4) {
+                            wop[1][s >> 1][2 * s & 3] = code_pair<FORMAT>(raw[1], 2 * s);
+                            wop[1][s >> 1][2 * s + 1 & 3] = code_pair<FORMAT>(raw[1], 2 * s + 1);
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = s < 1 ? 0 : 3 * s - 2 - (s == 1); i < (s < 1 ? 0 : 3 * s + 1); ++i)
+                            acc[rt ^ 1][(k - 1) >> 1][i] = __builtin_fmaf(scale[rt ^ 1], prev[i], acc[rt ^ 1][(k - 1) >> 1][i]);
+                    }
+                    if (rt == 1 && tp + 1 < TP)
+                        xa[s] = *reinterpret_cast<const bf16x8*>(xcur + (tp + 1) * kBlockTileBytes + s * kPartBytes);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                prev = d;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[1][TP - 1][i] = __builtin_fmaf(scale[1], prev[i], acc[1][TP - 1][i]);
         }
-        __syncthreads();  // round k + 1 staged, round k's buffer read
-        w0 = w1;
-        w1 = w2;
-    }
 
-    // The ways' sums, added in way order by way 0 (the loop's last barrier ends every read of the buffers).
-    if constexpr (W > 1) {
-        float* sums = reinterpret_cast<float*>(lds);  // [way - 1][row tile][output][lane]
+        // ---- the tile's sums: the ways' are added pairwise, then stored, or left as a partial.
+        // Four outputs (positions p .. p + 3 of a lane's row) are adjacent in the LDS and in a partial. ----
+        if (FUSED && tid < TP) lds_flags[tid] = 0u;
+        __syncthreads();
+        f32x4* sums = reinterpret_cast<f32x4*>(lds);
+        auto quad_at = [&](int rt, int tp, int q) { return (((rh * 2 + rt) * TP + tp) * 4 + q) * 64 + lane; };
         if (way > 0)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sums[(((way - 1) * 4 + rt) * 16 + i) * 64 + lane] = acc[i];
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int tp = 0; tp < TP; ++tp)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        sums[(way - 1) * (slot_floats(TP, RH) / 4) + quad_at(rt, tp, q)] =
+                            f32x4{acc[rt][tp][4 * q], acc[rt][tp][4 * q + 1], acc[rt][tp][4 * q + 2], acc[rt][tp][4 * q + 3]};
+        if constexpr (FUSED) {
+#pragma unroll
+            for (int j = 0; j < TP; ++j) {
+                const uint64_t f = __ballot(flagged[j]);
+                const uint32_t word = static_cast<uint32_t>(f) | static_cast<uint32_t>(f >> 32);
+                if (lane == 0 && word) atomicOr(&lds_flags[j], word);
+            }
+        }
         __syncthreads();
-        if (way > 0) return;
+        if (way == 0) {
+            const bool whole = r0 == 0 && r1 == a.rounds;
+            const int slot = 2 * range + (r0 == 0 ? 1 : 0);  // the range's first segment, or its last
+            f32x4* out = reinterpret_cast<f32x4*>(a.partial + static_cast<int64_t>(slot) * slot_floats(TP, RH));
 #pragma unroll
-        for (int w2 = 1; w2 < W; ++w2)
+            for (int rt = 0; rt < 2; ++rt) {
+                const int row = row0 + 64 * rh + 32 * rt + (lane & 31);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = __fadd_rn(acc[i], sums[(((w2 - 1) * 4 + rt) * 16 + i) * 64 + lane]);
+                for (int tp = 0; tp < TP; ++tp)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        f32x4 o[WAYS];
+                        o[0] = f32x4{acc[rt][tp][4 * q], acc[rt][tp][4 * q + 1], acc[rt][tp][4 * q + 2], acc[rt][tp][4 * q + 3]};
+#pragma unroll
+                        for (int w = 1; w < WAYS; ++w) o[w] = sums[(w - 1) * (slot_floats(TP, RH) / 4) + quad_at(rt, tp, q)];
+#pragma unroll
+                        for (int n = WAYS / 2; n > 0; n /= 2)
+#pragma unroll
+                            for (int w = 0; w < n; ++w)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) o[w][e] = __fadd_rn(o[w][e], o[w + n][e]);
+                        const f32x4 v = o[0];
+                        if (!whole) {
+                            out[quad_at(rt, tp, q)] = v;
+                            continue;
+                        }
+                        const int p = (t0 + tp) * kTile + 8 * q + 4 * h;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (row < a.rows && p + e < a.positions)
+                                store_f32(a.y + static_cast<int64_t>(p + e) * a.rows + row,
+                                          __builtin_amdgcn_ldexpf(v[e], -kLiftExponent));
+                    }
+            }
+            if (FUSED && tid < TP) (whole ? a.tile_flags + tile * TP : a.slot_flags + slot * TP)[tid] = lds_flags[tid];
+        }
+        __syncthreads();  // the sums and flags are read
+        at += r1 - r0;
     }
-    if (row >= a.rows) return;
+}
+
+// One workgroup per 32 x 32 tile of every (row group, position unit) tile: adds the pieces of a cut tile and computes
+// the flagged positions of any tile. Thread (g, wave q, lane) adds pieces g, g + G, ... of outputs 4q .. 4q + 3 of its
+// lane, four chains at a time, then the chains and the G sums in a fixed order: with many pieces (a few rows of many
+// columns) a single chain of their loads took longer than the product (256 x 14336 Q8_0 over 8 positions: 21.9 us
+// against 13.3) and rounded more.
+template <int FORMAT, int TP, bool FUSED, int RH, int G>
+__global__ __launch_bounds__(kThreads * G) void fbatch_fixup_kernel(FbatchArgs a) {
+    constexpr int kGroupRows = 64 * RH, kSubs = 2 * RH * TP;
+    __shared__ uint32_t lds_flags;
+    __shared__ float lds_totals[kThreads];
+    __shared__ f32x4 lds_sums[G > 1 ? (G - 1) * kThreads : 1];
+    const int tile = blockIdx.x / kSubs, sub = blockIdx.x - tile * kSubs;  // sub = (2 rh + rt) * TP + tp
+    const int first = range_of(a, tile * a.rounds), last = range_of(a, (tile + 1) * a.rounds - 1);
+    const int tid = threadIdx.x % kThreads, g = threadIdx.x / kThreads, q = tid >> 6, lane = tid & 63, h = lane >> 5;
+    const int group = tile / a.units, tp = sub % TP, t = (tile - group * a.units) * TP + tp;
+    const int row0 = group * kGroupRows + 32 * (sub / TP);
+    const int row = row0 + (lane & 31);
+    const bool cut = first != last;
+    // The piece that starts the tile is its range's last segment, the others their range's first.
+    auto slot_of = [&](int i) { return 2 * i + (i == first ? 1 : 0); };
+    f32x4 sum[4] = {};  // one chain per piece in flight
+    if (cut)
+        for (int i0 = first + g; i0 <= last; i0 += 4 * G) {  // four pieces' loads in flight
+            f32x4 v[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int p = t * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
-        // Undo the position's lifting: exact unless the result is subnormal, where it rounds once.
-        if (p < a.positions)
-            store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, __builtin_amdgcn_ldexpf(acc[i], -a.lift[p]));
+            for (int j = 0; j < 4; ++j)
+                v[j] = *(const SATORI_GLOBAL f32x4*)(a.partial + static_cast<int64_t>(slot_of(min(i0 + j * G, last))) * slot_floats(TP, RH) +
+                                                     ((sub * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (i0 + j * G <= last)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) sum[j][k] = __fadd_rn(sum[j][k], v[j][k]);
+        }
+    f32x4 acc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = __fadd_rn(__fadd_rn(sum[0][k], sum[1][k]), __fadd_rn(sum[2][k], sum[3][k]));
+    if (threadIdx.x == 0) lds_flags = 0u;
+    if (G > 1 && g > 0) lds_sums[(g - 1) * kThreads + tid] = acc;
+    __syncthreads();
+    uint32_t word = 0u;
+    if constexpr (FUSED) {
+        if (!cut)
+            word = a.tile_flags[tile * TP + tp];
+        else
+            for (int i = first + threadIdx.x; i <= last; i += kThreads * G) word |= a.slot_flags[slot_of(i) * TP + tp];
+    } else {
+        for (int i = threadIdx.x; i < 2 * a.blocks; i += kThreads * G)
+            word |= a.flags[2 * (static_cast<int64_t>(i >> 1) * a.tiles + t) + (i & 1)];
     }
+    if (word) atomicOr(&lds_flags, word);
+    __syncthreads();
+    const uint32_t flagged = lds_flags;
+    if (cut && g == 0) {
+#pragma unroll
+        for (int j = 0; j < G - 1; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] = __fadd_rn(acc[k], lds_sums[j * kThreads + tid][k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 8 * q + 4 * h + k, p = t * kTile + i;
+            if (row < a.rows && p < a.positions && !((flagged >> i) & 1u))
+                store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, __builtin_amdgcn_ldexpf(acc[k], -kLiftExponent));
+        }
+    }
+    if (flagged) finish_flagged<FORMAT>(a, row0, t * kTile, flagged, lds_totals);
+}
+
+// How a launch is cut, for the device's CU count.
+struct FbatchPlan {
+    int TP, RH, ways;
+    bool fused;
+    int tiles, units, rounds, total, workgroups;
+    size_t flags_offset, partial_offset, slot_flags_offset, tile_flags_offset, bytes;
+};
+
+FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
+    FbatchPlan p{};
+    const int blocks = columns / 32;
+    p.tiles = (positions + kTile - 1) / kTile;
+    p.TP = p.tiles > 1 ? 2 : 1;
+    p.fused = p.tiles <= 2;
+    p.RH = p.fused ? 2 : 4;
+    p.ways = 8 / p.RH;
+    p.units = (p.tiles + p.TP - 1) / p.TP;
+    p.tiles = p.units * p.TP;  // whole units: the packed form's last tile may be all zero
+    p.rounds = (blocks + p.ways - 1) / p.ways;
+    // (Below 2^31 for every payload of at most 2^31 - 1 bytes: a round of a tile is 64 columns of 128 rows or more.)
+    p.total = (rows + 64 * p.RH - 1) / (64 * p.RH) * p.units * p.rounds;
+    int n = std::min(p.total, cus);  // one workgroup of eight waves per CU
+    if (n >= 8) n -= n % 8;
+    p.workgroups = n;
+    const size_t parts = p.fused ? 0 : static_cast<size_t>(blocks) * p.tiles * kBlockTileBytes;
+    p.flags_offset = parts;
+    p.partial_offset = parts + (p.fused ? 0 : (static_cast<size_t>(blocks) * p.tiles * 8 + 255) / 256 * 256);
+    p.slot_flags_offset = p.partial_offset + static_cast<size_t>(p.workgroups) * 2 * slot_floats(p.TP, p.RH) * sizeof(float);
+    p.tile_flags_offset = p.slot_flags_offset + static_cast<size_t>(p.workgroups) * 2 * p.TP * 4;
+    p.bytes = p.tile_flags_offset + static_cast<size_t>(p.total / p.rounds) * p.TP * 4;
+    return p;
+}
+
+int device_cus() {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
+        return 256;
+    return cus;
+}
+
+template <int FORMAT, int TP, bool FUSED, int RH, int WAYS>
+hipError_t launch_product(const FbatchArgs& a, hipStream_t stream) {
+    fbatch_kernel<FORMAT, TP, FUSED, RH, WAYS><<<static_cast<unsigned>(a.workgroups), 64 * RH * WAYS, 0, stream>>>(a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const unsigned grid = static_cast<unsigned>(a.total / a.rounds) * 2 * RH * TP;
+    if (a.rounds > 4 * a.share)  // more than about five pieces a tile
+        fbatch_fixup_kernel<FORMAT, TP, FUSED, RH, 4><<<grid, 4 * kThreads, 0, stream>>>(a);
+    else
+        fbatch_fixup_kernel<FORMAT, TP, FUSED, RH, 1><<<grid, kThreads, 0, stream>>>(a);
+    return hipGetLastError();
+}
+
+template <int FORMAT>
+hipError_t launch_format(FbatchArgs a, const FbatchPlan& p, uint8_t* workspace, hipStream_t stream) {
+    if (p.fused) return p.TP == 1 ? launch_product<FORMAT, 1, true, 2, 4>(a, stream) : launch_product<FORMAT, 2, true, 2, 4>(a, stream);
+    const int64_t items = static_cast<int64_t>(a.blocks) * p.tiles * 128;
+    if ((items + kThreads - 1) / kThreads > INT32_MAX) return hipErrorInvalidValue;
+    uint32_t* flags = reinterpret_cast<uint32_t*>(workspace + p.flags_offset);
+    fbatch_pack_kernel<FORMAT><<<static_cast<unsigned>((items + kThreads - 1) / kThreads), kThreads, 0, stream>>>(
+        a.x, a.blocks * 32, a.positions, p.tiles, workspace, flags);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    a.parts = workspace;
+    a.flags = flags;
+    return launch_product<FORMAT, 2, false, 4, 2>(a, stream);
 }
 
 }  // namespace
 
-// From one whole position tile on. Below it the product runs few workgroups (row groups x one tile) and is
-// latency-bound: measured at 8-32 positions, 4096x4096 Q8_0 takes 56 us against 21-52 us for the
-// single-position kernel per position, 11008x4096 Q4_0 44 us against 40-150 us.
-int fbatch_min_positions() { return 32; }
+// From 32 positions on always; below, where the weights the single-position kernel would read again outweigh the second
+// launch. Measured against that kernel (us, FP32 activations): 4096 x 4096 Q8_0 14 at any count to 32, against 10 at 2
+// positions, 16 at 4, 29 at 12; 11008 x 4096 Q4_0 23 against 16 at 2, 24 at 4, 39 at 8; 1135 x 3808 Q4_0 11 against
+// 9.4 at 8, 15 at 16; 4096 x 1024 Q4_0 10 against 8.4 at 16, 13 at 31; 512 x 1024 8.5 against 3.8 at 31.
+bool fbatch_pays(int rows, int columns, int positions) {
+    if (positions >= kTile) return true;
+    return positions >= 4 && static_cast<int64_t>(rows) * columns * (positions - 1) >= 72000000;
+}
 
-size_t fbatch_workspace_bytes(int columns, int positions) {
-    const int tiles = (positions + kTile - 1) / kTile;
-    return static_cast<size_t>(columns / 32) * tiles * kBlockTileBytes + static_cast<size_t>(tiles) * kTile * 4;
+size_t fbatch_workspace_bytes(int rows, int columns, int positions) {
+    // The largest of this and every smaller position count, so that a buffer made for one call serves the smaller
+    // ones (each of the three forms grows with its positions).
+    const int cus = device_cus();
+    size_t bytes = fbatch_plan(rows, columns, positions, cus).bytes;
+    for (int limit : {kTile, 2 * kTile})
+        if (positions > limit) bytes = std::max(bytes, fbatch_plan(rows, columns, limit, cus).bytes);
+    return bytes;
 }
 
 hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* workspace, float* y, int rows,
                               int columns, int positions, hipStream_t stream) {
     if (rows <= 0 || positions <= 0 || columns <= 0) return hipSuccess;
     if ((format != kQ8_0 && format != kQ4_0) || columns % 32 != 0) return hipErrorInvalidValue;
-    const int blocks = columns / 32;
-    const int tiles = (positions + kTile - 1) / kTile;
-    const int64_t items = static_cast<int64_t>(blocks) * tiles * 128;
-    if ((items + 255) / 256 > INT32_MAX) return hipErrorInvalidValue;
-    int* lift = reinterpret_cast<int*>(workspace + static_cast<size_t>(blocks) * tiles * kBlockTileBytes);
-    fbatch_lift_kernel<<<static_cast<unsigned>(tiles * kTile), 256, 0, stream>>>(x, columns, positions, lift);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    fbatch_pack_kernel<<<static_cast<unsigned>((items + 255) / 256), 256, 0, stream>>>(x, columns, positions, tiles,
-                                                                                      workspace, lift);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int64_t units = static_cast<int64_t>((rows + 4 * kTile - 1) / (4 * kTile)) * tiles;
-    const int64_t grid = (units + 7) / 8 * 8;
-    if (grid > INT32_MAX) return hipErrorInvalidValue;
-    const FbatchArgs a{w, workspace, lift, y, rows, blocks, positions, tiles};
-    // Ways per row tile: as many (4, 2, 1) as keep every workgroup resident at once (two workgroups of 16
-    // waves, four of 8 or eight of 4 per CU), so no second wave of workgroups trails the first.
-    const int W = units <= 512 ? 4 : (units <= 1024 ? 2 : 1);
-    auto go = [&](auto kernel, int w_) { kernel<<<static_cast<unsigned>(grid), 256 * w_, 0, stream>>>(a); };
-    if (format == kQ8_0) {
-        if (W == 4) go(fbatch_kernel<kQ8_0, 4>, 4); else if (W == 2) go(fbatch_kernel<kQ8_0, 2>, 2); else go(fbatch_kernel<kQ8_0, 1>, 1);
-    } else {
-        if (W == 4) go(fbatch_kernel<kQ4_0, 4>, 4); else if (W == 2) go(fbatch_kernel<kQ4_0, 2>, 2); else go(fbatch_kernel<kQ4_0, 1>, 1);
-    }
-    return hipGetLastError();
+    const FbatchPlan p = fbatch_plan(rows, columns, positions, device_cus());
+    FbatchArgs a{};
+    a.w = w;
+    a.x = x;
+    a.y = y;
+    a.partial = reinterpret_cast<float*>(workspace + p.partial_offset);
+    a.slot_flags = reinterpret_cast<uint32_t*>(workspace + p.slot_flags_offset);
+    a.tile_flags = reinterpret_cast<uint32_t*>(workspace + p.tile_flags_offset);
+    a.rows = rows;
+    a.blocks = columns / 32;
+    a.positions = positions;
+    a.tiles = p.tiles;
+    a.units = p.units;
+    a.rounds = p.rounds;
+    a.total = p.total;
+    a.workgroups = p.workgroups;
+    a.share = p.total / p.workgroups;
+    a.longer = p.total % p.workgroups;
+    return format == kQ8_0 ? launch_format<kQ8_0>(a, p, workspace, stream) : launch_format<kQ4_0>(a, p, workspace, stream);
 }
 
 }  // namespace satori

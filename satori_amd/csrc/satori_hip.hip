@@ -91,6 +91,7 @@ struct satori_hip_context {
     bool live = true;
     int matrices = 0;
     satori::DeviceBuffer x, y, q8k;
+    satori::DeviceBuffer batch;                      // partial sums of short Q8_0 / Q4_0 batches on the context stream
     satori::DeviceBuffer upload_stage, upload_flag;  // packed payloads on their way into the device layouts
     // Split-attention partials (grouped attention over long prefixes), one buffer per stream the attention
     // runs on, so attentions on different streams never share one; attentions on one stream run in order.
@@ -227,31 +228,58 @@ LaunchShape launch_shape(const Shape& s, int positions, int rows_max) {
 
 bool is_k(const Shape& s) { return s.format == SATORI_HIP_Q4_K || s.format == SATORI_HIP_Q6_K; }
 
-// Enqueue one FP32-activation product: x [positions][C] -> y [positions][R], all device pointers. Q8_0 and
-// Q4_0 over fbatch_min_positions() positions or more run on the matrix cores, 256 positions per launch pair,
-// with the split activations in the matrix's activation buffer (executions of one matrix that overlap in
-// time race on it).
-void enqueue_float(satori_hip_matrix* m, const float* x, int positions, float* y, hipStream_t stream) {
-    const Shape& s = m->shape;
-    if ((s.format == SATORI_HIP_Q8_0 || s.format == SATORI_HIP_Q4_0) && positions >= fbatch_min_positions()) {
-        constexpr int kChunk = 256;
-        const size_t need = fbatch_workspace_bytes(s.columns, std::min(positions, kChunk));
-        if (m->context->capturing && m->q8k.bytes < need)
+// The matrix's activation buffer of at least `need` bytes for a many-position product, refused where it may not
+// grow: while capturing, and while a captured step holds the current one.
+void* reserve_activations(satori_hip_matrix* m, size_t need) {
+    if (m->q8k.bytes < need) {
+        if (m->context->capturing)
             fail(SATORI_HIP_E_INVALID_OPERATION,
                  "Run this many-position product once before capturing it (its workspace is allocated on first use).");
-        if (m->steps > 0 && m->q8k.bytes < need)  // a captured step holds the current buffer
+        if (m->steps > 0)
             fail(SATORI_HIP_E_INVALID_OPERATION,
                  "The workspace of this matrix cannot grow while a captured step launches it: destroy the step, "
                  "or run the largest product before capturing.");
         m->q8k.reserve(need);
-        for (int p0 = 0; p0 < positions; p0 += kChunk) {
-            const int n = std::min(kChunk, positions - p0);
-            check_hip(launch_gemv_fbatch(m->payload, s.format, x + static_cast<int64_t>(p0) * s.columns,
-                                         static_cast<uint8_t*>(m->q8k.ptr), y + static_cast<int64_t>(p0) * s.rows,
-                                         s.rows, s.columns, n, stream),
-                      "matrix-core gemv launch");
+    }
+    return m->q8k.ptr;
+}
+
+// Workspace of a Q8_0 / Q4_0 batch on the matrix cores, or null where a call of fewer than 32 positions may not
+// allocate or hold one (it then takes the single-position kernel, which needs none). Below 32 positions a call on
+// the context stream uses the context's buffer, so a matrix's first call allocates nothing (hipMalloc took 25 us
+// beside a 14 us product). No graph holds that buffer: a captured step may hold the matrix's own (which then cannot
+// grow), a capture the caller makes of a stream itself holds none.
+void* batch_workspace(satori_hip_matrix* m, int positions, size_t need, hipStream_t stream) {
+    satori_hip_context* c = m->context;
+    if (positions >= 32) return reserve_activations(m, need);
+    if (c->capturing && stream == c->stream) return m->q8k.bytes >= need ? m->q8k.ptr : nullptr;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
+    if (stream == c->stream) {
+        c->batch.reserve(need);
+        return c->batch.ptr;
+    }
+    if (m->q8k.bytes < need && (m->steps > 0 || c->capturing)) return nullptr;
+    return reserve_activations(m, need);
+}
+
+// Enqueue one FP32-activation product: x [positions][C] -> y [positions][R], all device pointers. Q8_0 and
+// Q4_0 over as many positions as fbatch_pays says run on the matrix cores, 256 positions at a time.
+void enqueue_float(satori_hip_matrix* m, const float* x, int positions, float* y, hipStream_t stream) {
+    const Shape& s = m->shape;
+    if ((s.format == SATORI_HIP_Q8_0 || s.format == SATORI_HIP_Q4_0) && fbatch_pays(s.rows, s.columns, positions)) {
+        constexpr int kChunk = 256;
+        const size_t need = fbatch_workspace_bytes(s.rows, s.columns, std::min(positions, kChunk));
+        if (void* workspace = batch_workspace(m, positions, need, stream)) {
+            for (int p0 = 0; p0 < positions; p0 += kChunk) {
+                const int n = std::min(kChunk, positions - p0);
+                check_hip(launch_gemv_fbatch(m->payload, s.format, x + static_cast<int64_t>(p0) * s.columns,
+                                             static_cast<uint8_t*>(workspace), y + static_cast<int64_t>(p0) * s.rows,
+                                             s.rows, s.columns, n, stream),
+                          "matrix-core gemv launch");
+            }
+            return;
         }
-        return;
     }
     MatDesc d{m->payload, x, y, s.rows, 0};
     const LaunchShape l = launch_shape(s, positions, s.rows);
@@ -289,17 +317,9 @@ const uint8_t* ensure_planes(satori_hip_matrix* m, hipStream_t stream) {
 void enqueue_kint(satori_hip_matrix* m, const float* x, int positions, float* y, hipStream_t stream) {
     const Shape& s = m->shape;
     if (positions >= kmfma_min_positions()) {
-        const size_t need = kmfma_workspace_bytes(s.blocks, positions);
-        if (m->context->capturing && m->q8k.bytes < need)
-            fail(SATORI_HIP_E_INVALID_OPERATION,
-                 "Run this many-position product once before capturing it (its workspace is allocated on first use).");
-        if (m->steps > 0 && m->q8k.bytes < need)  // a captured step holds the current buffer
-            fail(SATORI_HIP_E_INVALID_OPERATION,
-                 "The workspace of this matrix cannot grow while a captured step launches it: destroy the step, "
-                 "or run the largest product before capturing.");
+        uint8_t* workspace = static_cast<uint8_t*>(reserve_activations(m, kmfma_workspace_bytes(s.blocks, positions)));
         const uint8_t* planes = ensure_planes(m, stream);
-        m->q8k.reserve(need);
-        check_hip(launch_gemv_kmfma(planes, s.format, x, static_cast<uint8_t*>(m->q8k.ptr), y, s.rows, s.blocks,
+        check_hip(launch_gemv_kmfma(planes, s.format, x, workspace, y, s.rows, s.blocks,
                                     s.row_bytes, positions, stream),
                   "matrix-core gemv launch");
         return;
@@ -809,6 +829,7 @@ int satori_hip_context_destroy(satori_hip_context* c) {
         c->x.release();
         c->y.release();
         c->q8k.release();
+        c->batch.release();
         c->upload_stage.release();
         c->upload_flag.release();
         for (auto& entry : c->attention) entry.second.release();

@@ -988,6 +988,66 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
     m.dispose()
 
 
+@pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
+@pytest.mark.parametrize("rows,columns,positions", [(1, 64, 32), (63, 32, 40), (129, 96, 65), (257, 4128, 129),
+                                                    (8200, 2080, 6), (513, 9056, 17), (4097, 4128, 31)])
+def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
+    # The edges of the matrix-core batch: row groups of 128 (up to 64 positions) and 256 rows with one row more
+    # or less, odd block counts, rounds past the last block, tiles cut into many partial sums, and counts below 32
+    # on matrices large enough for it. The first and last positions hold an activation from which the split
+    # activations give way to plain FP32 sums (2^40), and one just below it; the bound is that of
+    # test_legacy_matrix_core_batch, on the FP64 product.
+    g = rng(515 + rows + columns + positions)
+    w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
+    data = S.quantize_weights(w, rows, columns, fmt)
+    x = g.standard_normal((positions, columns)).astype(np.float32)
+    x[0, columns - 1] = np.float32(2.0 ** 40)
+    x[1, 0] = np.nextafter(np.float32(2.0 ** 40), np.float32(0))
+    x[positions - 1, columns // 2] = np.float32(-2.0 ** 60)
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        y = np.full((positions, rows), np.nan, np.float32)
+        m.execute_batch(x.reshape(-1), positions, y.reshape(-1))
+    wq = O.decode_matrix(data, rows, columns, int(fmt)).astype(np.float64)
+    xf = x.astype(np.float64)
+    bound = np.abs(xf) @ np.abs(wq).T * 1e-5 + (columns + columns // 32 + 2) * TINY
+    exact = xf @ wq.T
+    for p in range(positions):
+        assert_within(y[p], exact[p], bound[p], f"position {p}")
+
+
+def test_legacy_batch_captured_before_it_ran(context):
+    # A batch of fewer than 32 positions that would use the workspace is captured without one (nothing may be
+    # allocated then), replays within the FP32 bound, and the same matrix then runs eagerly with a workspace.
+    rows, columns, positions = 8200, 2080, 6
+    g = rng(99)
+    w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
+    data = S.quantize_weights(w, rows, columns, BQ.Q8_0)
+    x = g.standard_normal((positions, columns)).astype(np.float32)
+    wq = O.decode_matrix(data, rows, columns, int(BQ.Q8_0)).astype(np.float64)
+    exact = x.astype(np.float64) @ wq.T
+    bound = np.abs(x.astype(np.float64)) @ np.abs(wq).T * 1e-5
+    dx, dy = context.alloc(x.nbytes), context.alloc(4 * positions * rows)
+    context.upload(dx, x)
+    y = np.zeros((positions, rows), np.float32)
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, BQ.Q8_0)) as m:
+        context.capture_begin()
+        m.execute_batch_device(dx, positions, dy)
+        step = context.capture_end()
+        for _ in range(3):
+            context.upload(dy, np.zeros_like(y))
+            step.execute()
+            context.synchronize()
+            context.download(y, dy)
+            assert np.all(np.abs(y - exact) <= bound)
+        m.execute_batch_device(dx, positions, dy)  # while the step lives: still no workspace
+        assert np.all(np.abs(context.download(y, dy) - exact) <= bound)
+        step.dispose()
+        m.execute_batch_device(dx, positions, dy)
+        assert np.all(np.abs(context.download(y, dy) - exact) <= bound)
+    context.free(dx)
+    context.free(dy)
+
+
 def _tiny_positions(g, positions, columns, mixed):
     """Activation rows of tiny magnitude (NumericalCorpus.cs:24-27 carries 1e-30, subnormal and 1e-38 cases):
     N(0,1) scaled to 1e-36 and 1e-38, FP32 subnormals, TINY alternating, normal elements mixed with 1e-38 and
