@@ -81,8 +81,10 @@ __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
     return v;
 }
 
-// `lane` is the lane within the wave (0..63); all 16 lanes of its row must be active together.
-__device__ __forceinline__ Q8KRow16 q8k_quantize_row16(const float (&v)[16], int lane) {
+// The general form, for rows that hold a NaN or whose largest magnitude occurs with both signs (or is zero): the
+// row's first index with the largest magnitude decides the sign. `lane` is the lane within the wave (0..63); all 16
+// lanes of its row must be active together.
+__device__ __forceinline__ Q8KRow16 q8k_quantize_row16_general(const float (&v)[16], int lane) {
     uint32_t key = 0;
     float first = 0.0f;  // the lane's first element of maximal magnitude (strict >: the lowest index wins)
 #pragma unroll
@@ -117,6 +119,48 @@ __device__ __forceinline__ Q8KRow16 q8k_quantize_row16(const float (&v)[16], int
         r.packed[i >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(n)) << (8 * (i & 3));
     }
     r.group_sum = sum;
+    r.scale = __fdiv_rn(1.0f, inverse);
+    return r;
+}
+
+// The largest value of a 16-lane row in every lane of it, NaN if any is (DPP rotations within the row).
+template <bool MAX>
+__device__ __forceinline__ float row_extreme_f32(float v) {
+    auto op = [](float a, float b) { return MAX ? __builtin_elementwise_maximum(a, b) : __builtin_elementwise_minimum(a, b); };
+    v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xF, 0xF, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xF, 0xF, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false)));
+    v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false)));
+    return v;
+}
+
+// The quantizer is vector-ALU bound wherever every workgroup repeats it (the integer products): 16 NaN-propagating
+// maxima and minima find the largest magnitude and its sign, unless the two extremes are equal in magnitude (then,
+// and with a NaN, the general form). Where they are not, every product is in -127..127, so the shifted float's low
+// byte is the code (NearestInteger's clamp and sign extension do nothing) and the codes are summed by dot products.
+__device__ __forceinline__ Q8KRow16 q8k_quantize_row16(const float (&v)[16], int lane) {
+    float hi = v[0], lo = v[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) {
+        hi = __builtin_elementwise_maximum(hi, v[i]);
+        lo = __builtin_elementwise_minimum(lo, v[i]);
+    }
+    hi = row_extreme_f32<true>(hi);
+    lo = row_extreme_f32<false>(lo);
+    if (__ballot(!(hi > -lo || hi < -lo))) return q8k_quantize_row16_general(v, lane);
+    const float inverse = __fdiv_rn(-127.0f, hi > -lo ? hi : lo);
+    Q8KRow16 r;
+    r.group_sum = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        uint32_t s[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = __float_as_uint(__fadd_rn(__fmul_rn(inverse, v[4 * w + e]), 12582912.0f));
+        const uint32_t low = __builtin_amdgcn_perm(s[1], s[0], 0x0C0C0400u);   // bytes s0, s1, 0, 0
+        const uint32_t high = __builtin_amdgcn_perm(s[3], s[2], 0x04000C0Cu);  // bytes 0, 0, s2, s3
+        r.packed[w] = low | high;
+        r.group_sum = __builtin_amdgcn_sdot4(static_cast<int>(r.packed[w]), 0x01010101, r.group_sum, false);
+    }
     r.scale = __fdiv_rn(1.0f, inverse);
     return r;
 }

@@ -1015,6 +1015,50 @@ def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
         assert_within(y[p], exact[p], bound[p], f"position {p}")
 
 
+def _q8k_special_row(columns):
+    """Blocks whose Q8_K quantization takes its special cases: the largest magnitude with both signs (either first), a
+    NaN beside it (quiet, with a payload, alone), infinities, zeros of both signs, subnormals and a plain block."""
+    g = rng(31337)
+    x = g.standard_normal((columns // 256, 256)).astype(np.float32)
+    x[0, [40, 41]] = [9.0, -9.0]
+    x[1, [200, 7]] = [9.0, -9.0]
+    x[2, [3, 250]] = [np.nan, 8.0]
+    x[3, 17] = np.uint32(0x7FC00123).view(np.float32)
+    x[4] = np.nan
+    x[5, 100] = np.inf
+    x[6, [5, 90]] = [-np.inf, np.inf]
+    x[7] = 0.0
+    x[8] = -0.0
+    x[9] = (x[9] * 1e-41).astype(np.float32)
+    x[10] = (x[10] * 1e-37).astype(np.float32)
+    return x
+
+
+@pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
+@pytest.mark.parametrize("rows,positions", [(40, 1), (3000, 3), (3001, 11), (64, 17)])
+def test_k_quantizer_special_blocks_in_every_product(context, fmt, rows, positions):
+    # The activation quantizer inside the single-position, few-position and matrix-core integer products, on rows whose
+    # blocks take its special cases, against the oracle's quantizer and integer product, bit for bit; one block at a
+    # time (the others plain), so that a NaN or infinity of one does not hide another.
+    columns = 12 * 256
+    special = _q8k_special_row(columns)
+    g = rng(404 + rows)
+    w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
+    data = S.quantize_weights(w, rows, columns, fmt)
+    x = g.standard_normal((12, columns)).astype(np.float32)
+    for b in range(12):
+        x[b, 256 * b:256 * (b + 1)] = special[b]
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        for p0 in range(0, 12, positions):
+            batch = x[np.arange(p0, p0 + positions) % 12]
+            y = np.zeros((positions, rows), np.float32)
+            m.execute_batch(np.ascontiguousarray(batch).reshape(-1), positions, y.reshape(-1))
+            for i in range(positions):
+                ref = O.qk_matvec_quantized_avx2(data, rows, columns, int(fmt), O.q8k_quantize_row(batch[i]))
+                same = (y[i].view(np.uint32) == ref.view(np.uint32)) | (np.isnan(y[i]) & np.isnan(ref))
+                assert np.all(same), f"row {(p0 + i) % 12}"
+
+
 def test_legacy_batch_captured_before_it_ran(context):
     # A batch of fewer than 32 positions that would use the workspace is captured without one (nothing may be
     # allocated then), replays within the FP32 bound, and the same matrix then runs eagerly with a workspace.
