@@ -72,6 +72,12 @@ __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4(static_cast<int>(a), static_cast<int>(b), c, false);
 }
 
+// Two int16 products and a sum, exact.
+__device__ __forceinline__ int sdot2(uint32_t a, uint32_t b, int c) {
+    typedef short s16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, a), __builtin_bit_cast(s16x2, b), c, false);
+}
+
 struct ActTile {
     uint32_t* codes;   // [blocks][64] dwords
     int16_t* sums;     // [blocks][16]
@@ -480,6 +486,187 @@ __global__ __launch_bounds__(kThreads) void gemv_kint_kernel(KintMembers inline_
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The same product over a few positions (2 to 15). A workgroup owns a tile of rows of one member at up to
+// kMultiPositions positions: it quantizes those positions' rows, then unpacks every (row, block) pair's weights
+// once for all of them. What bounds the product at these sizes is the vector ALU (unpacking, the quantization every
+// workgroup repeats) and one latency chain, not HBM; a launch slice per position repeated all of it per position.
+// One workgroup of 512 threads per CU keeps the repeated quantization to one per CU. Each output is formed exactly
+// as gemv_kint_kernel forms it.
+// ------------------------------------------------------------------------------------------------
+constexpr int kMultiThreads = 512;
+constexpr int kMultiPositions = 8;
+constexpr int kMultiLdsBytes = 144 * 1024;
+
+template <int FORMAT, bool INLINE>
+__global__ __launch_bounds__(kMultiThreads) void gemv_kint_multi_kernel(KintMembers inline_members,
+                                                                         const MatDesc* __restrict__ group,
+                                                                         LaunchShape s, int per) {
+    constexpr int G = 4;  // lanes per (row, block) pair
+    constexpr int kSlots = kMultiThreads / G, kRows16 = kMultiThreads / 16;
+    constexpr int kDepth = 2;  // pairs whose payload is in flight
+    using Raw = typename std::conditional<FORMAT == kQ4_K, Q4KRaw, Q6KRaw>::type;
+    const MatDesc m = INLINE ? inline_members.m[blockIdx.y] : group[blockIdx.y];
+    const int row_begin = blockIdx.x * s.rows_per_wg;
+    if (row_begin >= m.rows) return;
+    const int rows = min(s.rows_per_wg, m.rows - row_begin);
+    const int first = blockIdx.z * per, np = min(per, s.positions - first);
+    const int nb = s.blocks, K = s.chunk_blocks;
+    const int tid = threadIdx.x, lane = tid & 63, c = lane % G, j16 = tid & 15;
+
+    // Per position: codes, scales and group sums of K blocks (as gemv_kint_kernel); then the terms, [position][row][block].
+    extern __shared__ uint32_t smem[];
+    auto act_of = [&](int pp) {
+        uint32_t* base = smem + pp * (kActDwords * K);
+        return ActTile{base, reinterpret_cast<int16_t*>(base + (kCodeStride + 1) * K),
+                       reinterpret_cast<float*>(base + kCodeStride * K)};
+    };
+    float* terms = reinterpret_cast<float*>(smem + np * (kActDwords * K));
+
+    auto load_pair = [&](int b0, int kb, int p, Raw& r) {
+        const int row = row_begin + p / kb, b = b0 + p % kb;
+        if constexpr (FORMAT == kQ4_K)
+            q4k_load(m.w + static_cast<int64_t>(row) * s.row_bytes + b * 144, c, r);
+        else
+            q6k_load_quarter(m.w, static_cast<int64_t>(m.rows) * nb, static_cast<int64_t>(row) * nb + b, c, r);
+    };
+    auto load_x = [&](int b0, int kb, int item, f32x4 (&x4)[4]) {  // 16 values of (position, block) `item`
+        const int pp = item / kb, b = b0 + item % kb;
+        const float* src = m.x + static_cast<int64_t>(first + pp) * s.columns + 256 * b + 16 * j16;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const u32x4 raw = load16_a4(reinterpret_cast<const uint8_t*>(src + 4 * q));
+            x4[q] = f32x4{__uint_as_float(raw[0]), __uint_as_float(raw[1]), __uint_as_float(raw[2]),
+                          __uint_as_float(raw[3])};
+        }
+    };
+
+    float acc[2] = {0.0f, 0.0f};  // sums t = tid, tid + threads of rows * np: row t % rows of position t / rows, in block order
+    const int p0 = tid / G;
+    for (int b0 = 0; b0 < nb; b0 += K) {
+        const int kb = min(K, nb - b0), pairs = rows * kb, items = np * kb;
+        // The first activations, then the first pairs' weights; a 16-lane row per (position, block), 32 at a time.
+        // (Two or four blocks side by side per row measured 5-40% slower: the quantization is bound by its instructions.)
+        int item = tid >> 4;
+        f32x4 x4[4];
+        load_x(b0, kb, min(item, items - 1), x4);
+        Raw buf[kDepth];
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) load_pair(b0, kb, min(p0 + i * kSlots, pairs - 1), buf[i]);
+        for (; item < items; item += kRows16) {
+            float v[16];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * q + e] = x4[q][e];
+            if (item + kRows16 < items) load_x(b0, kb, item + kRows16, x4);
+            const Q8KRow16 qr = q8k_quantize_row16(v, lane);
+            const ActTile act = act_of(item / kb);
+            const int bl = item % kb;
+            *reinterpret_cast<u32x4*>(act.codes + kCodeStride * bl + 4 * j16) =
+                u32x4{qr.packed[0], qr.packed[1], qr.packed[2], qr.packed[3]};
+            act.sums[16 * bl + j16] = static_cast<int16_t>(qr.group_sum);
+            if (j16 == 0) act.scales[bl] = qr.scale;
+        }
+        __syncthreads();  // activations of the chunk staged
+        for (int base = p0; base < pairs; base += kDepth * kSlots) {
+#pragma unroll
+            for (int i = 0; i < kDepth; ++i) {
+                const int p = base + i * kSlots;
+                if (p < pairs) {
+                    const int bl = p % kb;
+                    if constexpr (FORMAT == kQ4_K) {
+                        const Raw& r = buf[i];
+                        int s0, m0, s1, m1;
+                        q4k_scale_min(2 * c, r.head, s0, m0);
+                        q4k_scale_min(2 * c + 1, r.head, s1, m1);
+                        const uint32_t mm0 = m0 * 0x10001u, mm1 = m1 * 0x10001u;
+                        uint32_t lo[8], hi[8];
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            lo[w] = r.qs0[w] & 0x0F0F0F0Fu;
+                            lo[4 + w] = r.qs1[w] & 0x0F0F0F0Fu;
+                            hi[w] = (r.qs0[w] >> 4) & 0x0F0F0F0Fu;
+                            hi[4 + w] = (r.qs1[w] >> 4) & 0x0F0F0F0Fu;
+                        }
+                        const float d = half_bits_to_float(r.head[0] & 0xFFFFu), dmin = half_bits_to_float(r.head[0] >> 16);
+                        for (int pp = 0; pp < np; ++pp) {
+                            const ActTile act = act_of(pp);
+                            const uint32_t* codes = act.codes + kCodeStride * bl + 16 * c;
+                            int dl = 0, dh = 0;
+#pragma unroll
+                            for (int q = 0; q < 2; ++q) {
+                                const u32x4 l = *reinterpret_cast<const u32x4*>(codes + 4 * q);
+                                const u32x4 h = *reinterpret_cast<const u32x4*>(codes + 8 + 4 * q);
+#pragma unroll
+                                for (int w = 0; w < 4; ++w) {
+                                    dl = sdot4(lo[4 * q + w], l[w], dl);
+                                    dh = sdot4(hi[4 * q + w], h[w], dh);
+                                }
+                            }
+                            const uint2 sums = *reinterpret_cast<const uint2*>(act.sums + 16 * bl + 4 * c);
+                            const int dot = group_sum_last_int<G>(__mul24(s0, dl) + __mul24(s1, dh));
+                            const int mins = group_sum_last_int<G>(sdot2(sums.x, mm0, sdot2(sums.y, mm1, 0)));
+                            const float a = act.scales[bl];
+                            float term = 0.0f;  // zero activation block: skipped (QuantizedKAvx2Kernel.cs:86)
+                            if (a != 0.0f)
+                                term = __fsub_rn(__fmul_rn(__fmul_rn(d, a), static_cast<float>(dot)),
+                                                 __fmul_rn(__fmul_rn(dmin, a), static_cast<float>(mins)));
+                            if (c == G - 1) terms[pp * pairs + p] = term;
+                        }
+                    } else {
+                        const Raw& r = buf[i];
+                        const int h = c >> 1, t = c & 1;
+                        uint32_t q[4][4];
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            const uint32_t a = r.qla[w], bq = r.qlb[w], hb = r.qh[w];
+                            q[0][w] = (a & 0x0F0F0F0Fu) | ((hb << 4) & 0x30303030u);
+                            q[1][w] = (bq & 0x0F0F0F0Fu) | ((hb << 2) & 0x30303030u);
+                            q[2][w] = ((a >> 4) & 0x0F0F0F0Fu) | (hb & 0x30303030u);
+                            q[3][w] = ((bq >> 4) & 0x0F0F0F0Fu) | ((hb >> 2) & 0x30303030u);
+                        }
+                        const float d = q6k_d(r);
+                        for (int pp = 0; pp < np; ++pp) {
+                            const ActTile act = act_of(pp);
+                            const uint32_t* codes = act.codes + kCodeStride * bl + 32 * h + 4 * t;
+                            const u32x4 sums = *reinterpret_cast<const u32x4*>(act.sums + 16 * bl + 8 * h);  // pair k: t = 0, 1
+                            int total = 0;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                const u32x4 x = *reinterpret_cast<const u32x4*>(codes + 8 * k);
+                                int dot = 0;
+#pragma unroll
+                                for (int w = 0; w < 4; ++w) dot = sdot4(q[k][w], x[w], dot);
+                                total += __mul24(static_cast<int8_t>(r.sc >> (8 * k)),
+                                                 dot - 32 * static_cast<int16_t>(sums[k] >> (16 * t)));
+                            }
+                            const int dot = group_sum_last_int<G>(total);
+                            const float a = act.scales[bl];
+                            const float term = a != 0.0f ? __fmul_rn(__fmul_rn(a, d), static_cast<float>(dot)) : 0.0f;
+                            if (c == G - 1) terms[pp * pairs + p] = term;
+                        }
+                    }
+                    if (p + kDepth * kSlots < pairs) load_pair(b0, kb, p + kDepth * kSlots, buf[i]);
+                }
+            }
+        }
+        __syncthreads();  // the chunk's terms are in LDS
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int t = tid + k * kMultiThreads;
+            if (t < rows * np)
+                for (int b = 0; b < kb; ++b) acc[k] = __fadd_rn(acc[k], terms[(t / rows) * pairs + (t % rows) * kb + b]);
+        }
+        if (b0 + K < nb) __syncthreads();  // every thread is done with this chunk's activations and terms
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int t = tid + k * kMultiThreads;
+        if (t < rows * np) store_f32(m.y + static_cast<int64_t>(first + t / rows) * m.rows + row_begin + t % rows, acc[k]);
+    }
+}
+
 }  // namespace
 
 hipError_t launch_q8k_quantize(const float* x, int columns, int positions, uint8_t* out, hipStream_t stream) {
@@ -560,8 +747,63 @@ hipError_t launch_kint(const MatDesc* members, const MatDesc* device_members, in
 
 }  // namespace
 
+namespace {
+
+constexpr int kMultiRows = 128;  // two sums per thread at kMultiPositions
+
+int multi_slices(int positions) { return (positions + kMultiPositions - 1) / kMultiPositions; }
+
+// Whether the positions share a workgroup: where a launch slice per position would be bound by its throughput (about
+// 24 M weights x positions), and a slice's positions are not so long that quantizing all of them in every workgroup
+// costs more than reading the weights again. Measured (us, a slice per position against this): 4096 x 4096 Q4_K 7.2
+// and 5.2 at 2 positions, 10.4 and 7.5 at 5, 22.0 and 14.6 at 15; 1536 x 8960 8.4 and 7.1 at 2, 16.9 and 13.1 at 5,
+// but 16.3 and 20.6 at 8 (280 blocks a workgroup); 512 x 1024 4.4 and 5.0 at 8; 256 x 14336 8.7 and 11.3 at 5. Short
+// rows at many positions leave each pair few blocks to share (8960 x 1536 12.5 and 12.8 at 8, 1536 x 1536 6.1 and 7.0 at
+// 12; 3000 x 2048 11.0 and 7.7 at 15).
+bool multi_pays(int64_t rows, int blocks, int positions) {
+    const int slices = multi_slices(positions);
+    return rows * blocks * 256 * positions >= 24000000 && (positions + slices - 1) / slices * blocks <= 180 &&
+           (blocks >= 8 || positions <= 6);
+}
+
+// In slices of at most kMultiPositions positions, with one workgroup per CU over all slices.
+hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_members, int count, LaunchShape s,
+                             hipStream_t stream) {
+    const int slices = multi_slices(s.positions);
+    const int per = (s.positions + slices - 1) / slices;
+    int64_t rows = 0;
+    for (int i = 0; i < count; ++i) rows += members[i].rows;
+    const int64_t tile = (rows * slices + 255) / 256;
+    s.rows_per_wg = static_cast<int>(tile < 4 ? 4 : tile > kMultiRows ? kMultiRows : tile);
+    const int per_block = per * (kActDwords + s.rows_per_wg) * static_cast<int>(sizeof(uint32_t));
+    s.chunk_blocks = s.blocks < kMultiLdsBytes / per_block ? s.blocks : kMultiLdsBytes / per_block;
+    const dim3 grid((s.rows_max + s.rows_per_wg - 1) / s.rows_per_wg, count, slices);
+    const size_t lds = static_cast<size_t>(per_block) * s.chunk_blocks;
+    KintMembers inline_members{};
+    const bool in_arguments = count <= kKintInlineMembers;
+    if (in_arguments)
+        for (int i = 0; i < count; ++i) inline_members.m[i] = members[i];
+    auto go = [&](auto kernel) {
+        kernel<<<grid, kMultiThreads, lds, stream>>>(inline_members, device_members, s, per);
+        return hipGetLastError();
+    };
+    if (s.format == kQ4_K)
+        return in_arguments ? go(gemv_kint_multi_kernel<kQ4_K, true>) : go(gemv_kint_multi_kernel<kQ4_K, false>);
+    if (s.format == kQ6_K)
+        return in_arguments ? go(gemv_kint_multi_kernel<kQ6_K, true>) : go(gemv_kint_multi_kernel<kQ6_K, false>);
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
 hipError_t launch_gemv_kint(const MatDesc* members, const MatDesc* device_members, int count, LaunchShape s,
                             hipStream_t stream) {
+    if (count > 0 && s.rows_max > 0 && s.positions > 1) {
+        if (count > kKintInlineMembers && !device_members) return hipErrorInvalidValue;
+        int64_t rows = 0;
+        for (int i = 0; i < count; ++i) rows += members[i].rows;
+        if (multi_pays(rows, s.blocks, s.positions)) return launch_kint_multi(members, device_members, count, s, stream);
+    }
     return launch_kint<kInputPlain>(members, device_members, count, s, InputTransform{}, stream);
 }
 
