@@ -281,7 +281,8 @@ hipError_t launch_attention_inputs(float* q, const float* q_bias, const float* k
                                    const float* v, const float* v_bias, float* v_out, int heads, int kv_heads,
                                    int head_dim, int position, double base, int rotary, hipStream_t stream);
 // Grouped attention over `tokens` cached positions. Up to 32 tokens one workgroup per head; longer prefixes
-// are split over several workgroups per head (attention_splits) whose FP64 partials go to `scratch`
+// are split over several workgroups (attention_splits per head, or the shared form's splits, whose workgroups serve
+// several query heads of one key/value head: heads of 32, 64, 96 or 128 lanes) whose FP64 partials go to `scratch`
 // (attention_scratch_bytes: the bytes for `tokens`, which also cover every shorter prefix of these heads).
 // attention_supported is false only where one split's exponentials and staged query would not fit the LDS
 // (more than 134 million tokens).
@@ -300,7 +301,8 @@ hipError_t launch_attention_decode(float* q, const float* q_bias, const float* k
                                    const double* rope, float* out, double* partials, hipStream_t stream);
 // RoPE sines and cosines of positions 0 .. positions - 1: row p = rotary / 2 sines, then the cosines (doubles).
 hipError_t launch_rope_table(int positions, int rotary, double base, double* table, hipStream_t stream);
-// Partials one call of `tokens` tokens writes (0 when one workgroup per head needs none).
+// Partials of attention_splits(tokens) splits (0 when one workgroup per head needs none), what the no-allocation entry
+// point is refused by; the shared form takes as many splits as fit kStaticAttentionBytes.
 size_t attention_partials_bytes(int query_heads, int head_dim, int tokens);
 // The no-allocation attention's partials: a file-scope device array of kStaticAttentionBytes per device. Its
 // device address on the current device (call with that device current; the address differs per device).

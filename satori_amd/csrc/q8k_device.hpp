@@ -138,6 +138,8 @@ __device__ __forceinline__ float row_extreme_f32(float v) {
 // maxima and minima find the largest magnitude and its sign, unless the two extremes are equal in magnitude (then,
 // and with a NaN, the general form). Where they are not, every product is in -127..127, so the shifted float's low
 // byte is the code (NearestInteger's clamp and sign extension do nothing) and the codes are summed by dot products.
+// About 100 instructions a block where the general form takes 300: one position of 1536 x 8960 Q4_K 6.9 -> 6.1 us, of
+// 256 x 14336 6.9 -> 6.3, of 4096 x 4096 5.0 -> 4.8.
 __device__ __forceinline__ Q8KRow16 q8k_quantize_row16(const float (&v)[16], int lane) {
     float hi = v[0], lo = v[0];
 #pragma unroll

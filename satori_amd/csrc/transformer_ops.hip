@@ -10,6 +10,7 @@
 // place. The row decode and Add are FP32 expressions of the reference and agree bit for bit.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -815,6 +816,330 @@ __global__ __launch_bounds__(kSplitThreads) void attention_combine_kernel(const 
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The split attention for heads of 32, 64, 96 or 128 lanes whose key/value head serves at most eight query heads:
+// workgroup (key/value head, subgroup of its query heads, split) computes the split's scores, softmax terms and unnormalised
+// sums for all of those query heads at once. What bounds these launches is one chain of latencies and, in it, the FP64
+// conversions: each key and value element is loaded and converted once instead of once per query head, so a split
+// can be 32 tokens (one pass of loads, all issued at kernel start) where a workgroup per query head needed 128 to
+// keep the launch's workgroups few. The products of two FP32 values are exact in FP64, so the dot products' FMAs
+// round as a product and an addition. Measured on 12 / 2 heads of 128 lanes, the attention's two launches one pass after
+// another (us; before: a workgroup per query head): 300 tokens 10.0 -> 8.0, 1,500 12.8 -> 9.1, 4,096 14.5 -> 11.3 (split
+// 11.3 -> 7.6), 20,000 39.1 -> 21.2; 8 / 8 heads of 128 at 4,096 14.9 -> 12.7, 48 / 8 26.6 -> 17.9, 1 / 1 of 64 lanes at
+// 100 9.2 -> 7.2.
+// ------------------------------------------------------------------------------------------------
+constexpr int kSharedThreads = 256;
+constexpr int kSharedHeads = 8;        // query heads per key/value head
+constexpr int kSharedTile = 32;        // tokens per pass
+constexpr int kSharedMaxTokens = 256;  // tokens of one split (its softmax terms in LDS)
+constexpr int kSharedCombineThreads = 512;
+
+// Sum over each aligned group of 8 lanes, in every lane of it (DPP quad permutes and the half-row mirror).
+__device__ __forceinline__ double octet_sum(double v) {
+    auto move = [](double x, auto ctrl) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, x);
+        const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), decltype(ctrl)::value, 0xF, 0xF, false);
+        const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), decltype(ctrl)::value, 0xF, 0xF, false);
+        return __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
+    };
+    v = v + move(v, std::integral_constant<int, 0xB1>{});   // lane ^ 1
+    v = v + move(v, std::integral_constant<int, 0x4E>{});   // lane ^ 2
+    return v + move(v, std::integral_constant<int, 0x141>{});  // the other quad of the eight
+}
+
+// DP: lanes of a head per thread of a token (head_dim / 8). NG: query heads computed side by side (the key/value
+// head's, rounded up; one past the last repeats the last and is not stored), so that their chains of FP64 operations
+// overlap: one head after another took 3 us longer per launch at six heads.
+template <bool INPUTS, int DP, int NG>
+__global__ __launch_bounds__(kSharedThreads) void attention_shared_kernel(const float* __restrict__ q, const float* k,
+                                                                          const float* v, int query_heads,
+                                                                          int kv_heads, int tokens, int per, int splits,
+                                                                          int group, double* __restrict__ partial,
+                                                                          DecodeInputs in,
+                                                                          float* k_cache, float* v_cache) {
+    constexpr int HD = 8 * DP;
+    constexpr int kQStride = DP + 2;                               // a thread's query lanes in LDS, padded off its banks
+    constexpr int kValueGroups = kSharedThreads / HD;              // token groups of the value sums
+    constexpr int kValueTokens = kSharedTile / kValueGroups;       // tokens of a pass per group
+    constexpr int kQueryLoads = (NG * HD + kSharedThreads - 1) / kSharedThreads;
+    extern __shared__ double lds[];
+    const int subgroups = query_heads / kv_heads / group;
+    const int unit = blockIdx.x / splits, split = blockIdx.x - unit * splits;
+    const int kv_head = unit / subgroups, sub = unit - kv_head * subgroups, head0 = unit * group;
+    const int t0 = min(split * per, tokens), t1 = min(tokens, t0 + per), count = t1 - t0;
+    const int64_t kv_width = static_cast<int64_t>(kv_heads) * HD;
+    const int tid = threadIdx.x, token = tid >> 3, part = tid & 7;
+    double* qd = lds;                                              // [group][8][kQStride]
+    double* es = qd + group * 8 * kQStride;                        // [group][per]
+    double* sums = es + group * per;                               // [kValueGroups - 1][group][HD]
+    float* ks_new = reinterpret_cast<float*>(sums + (kValueGroups - 1) * group * HD);  // the new row (INPUTS)
+    float* vs_new = ks_new + HD;
+    const bool has_new = INPUTS && t0 <= in.position && in.position < t1;
+
+    // Every load the first pass needs: the key lanes of this thread's token, the value lane of its tokens (rows past the
+    // split's last, and the new row, read a valid row and are not used), the query lanes.
+    const float* kbase = k + kv_head * HD + part * DP;
+    const float* vbase = v + kv_head * HD + tid % HD;
+    const int vgroup = tid / HD;                                   // (HD 96: the last 64 threads have no value lane)
+    const int last_row = INPUTS ? max(0, min(t1 - 1, in.position - 1)) : t1 - 1;
+    float kr[DP], vr[kValueTokens];
+    auto load_keys = [&](int t) {
+        const uint8_t* src = reinterpret_cast<const uint8_t*>(kbase + min(t, last_row) * kv_width);
+#pragma unroll
+        for (int i = 0; i < DP; i += 4) {
+            const u32x4 raw = load16_a4(src + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kr[i + e] = __uint_as_float(raw[e]);
+        }
+    };
+    auto load_values = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < kValueTokens; ++i) vr[i] = load_f32(vbase + min(t + vgroup * kValueTokens + i, last_row) * kv_width);
+    };
+    if (count > 0) {
+        load_keys(t0 + token);
+        load_values(t0);
+    }
+    const int pairs = in.rotary / 2;
+    float qx[kQueryLoads], qy[kQueryLoads], qxb[kQueryLoads], qyb[kQueryLoads];
+    double sn[kQueryLoads], cs[kQueryLoads];
+    const int lane = tid % HD;                                     // (of the new row: threads below HD)
+    // The lane pair a rotated lane is formed from (one lane past the rotation).
+    auto pair_of = [&](int l, bool& rot, int& kk, int& ia, int& ib) {
+        rot = l < in.rotary;
+        kk = rot ? (l < pairs ? l : l - pairs) : 0;
+        ia = rot ? kk : l;
+        ib = rot ? kk + pairs : l;
+    };
+#pragma unroll
+    for (int n = 0; n < kQueryLoads; ++n) {
+        const int i = min(tid + n * kSharedThreads, group * HD - 1);
+        const int base = (head0 + i / HD) * HD, l = i % HD;
+        if constexpr (INPUTS) {
+            bool rot;
+            int kk, ia, ib;
+            pair_of(l, rot, kk, ia, ib);
+            qx[n] = load_f32(q + base + ia);
+            qy[n] = load_f32(q + base + ib);
+            qxb[n] = in.q_bias ? load_f32(in.q_bias + base + ia) : 0.0f;
+            qyb[n] = in.q_bias ? load_f32(in.q_bias + base + ib) : 0.0f;
+            if (in.rope) {
+                sn[n] = in.rope[kk];
+                cs[n] = in.rope[pairs + kk];
+            }
+        } else {
+            qx[n] = load_f32(q + base + l);
+        }
+    }
+    // The new row's operands, in the workgroups whose split holds it.
+    float nkx = 0.0f, nky = 0.0f, nkxb = 0.0f, nkyb = 0.0f, nv = 0.0f, nvb = 0.0f;
+    double nsn = 0.0, ncs = 0.0;
+    if (INPUTS && has_new && tid < HD) {
+        bool rot;
+        int kk, ia, ib;
+        pair_of(lane, rot, kk, ia, ib);
+        const int kb = kv_head * HD;
+        nkx = load_f32(in.k_new + kb + ia);
+        nky = load_f32(in.k_new + kb + ib);
+        nv = load_f32(in.v_new + kb + lane);
+        if (in.k_bias) {
+            nkxb = load_f32(in.k_bias + kb + ia);
+            nkyb = load_f32(in.k_bias + kb + ib);
+        }
+        if (in.v_bias) nvb = load_f32(in.v_bias + kb + lane);
+        if (in.rope) {
+            nsn = in.rope[kk];
+            ncs = in.rope[pairs + kk];
+        }
+    }
+    // Biased, then rotated, as attention_inputs_kernel forms the lane.
+    auto transform = [&](int l, float x, float y, float xb, float yb, bool bias, double s, double c) {
+        bool rot;
+        int kk, ia, ib;
+        pair_of(l, rot, kk, ia, ib);
+        const float xv = bias ? __fadd_rn(x, xb) : x, yv = bias ? __fadd_rn(y, yb) : y;
+        if (!rot) return xv;
+        if (!in.rope) rope_angle(kk, in.position, in.base, in.rotary, s, c);
+        float a, b;
+        rope_apply(xv, yv, s, c, a, b);
+        return l < pairs ? a : b;
+    };
+#pragma unroll
+    for (int n = 0; n < kQueryLoads; ++n) {
+        const int i = tid + n * kSharedThreads, h = i / HD, l = i % HD;
+        if (i >= group * HD) break;
+        float value = qx[n];
+        if constexpr (INPUTS) {
+            value = transform(l, qx[n], qy[n], qxb[n], qyb[n], in.q_bias != nullptr, sn[n], cs[n]);
+            if (split == 0)  // the rotated query, for the combine launch to store in place
+                reinterpret_cast<float*>(partial + static_cast<int64_t>(query_heads) * splits * (2 + HD))
+                    [(head0 + h) * HD + l] = value;
+        }
+        qd[(h * 8 + l / DP) * kQStride + l % DP] = value;
+    }
+    if (INPUTS && has_new && tid < HD) {
+        const int64_t at = in.position * kv_width + kv_head * HD + lane;
+        const float kj = transform(lane, nkx, nky, nkxb, nkyb, in.k_bias != nullptr, nsn, ncs);
+        const float vj = in.v_bias ? __fadd_rn(nv, nvb) : nv;
+        ks_new[lane] = kj;
+        vs_new[lane] = vj;
+        if (sub == 0) {
+            store_f32(k_cache + at, kj);
+            store_f32(v_cache + at, vj);
+        }
+    }
+    __syncthreads();
+
+    // Scores: eight threads per token, each its DP lanes of every head in lane order, the eight parts then added.
+    const double scale = 1.0 / __dsqrt_rn(static_cast<double>(HD));
+    for (int base = t0; base < t1; base += kSharedTile) {
+        const int t = base + token;
+        double kd[DP];
+#pragma unroll
+        for (int i = 0; i < DP; ++i) kd[i] = INPUTS && t == in.position ? ks_new[part * DP + i] : kr[i];
+        if (base + kSharedTile < t1) load_keys(t + kSharedTile);
+        double dot[NG];
+#pragma unroll
+        for (int h = 0; h < NG; ++h) dot[h] = 0.0;
+#pragma unroll
+        for (int i = 0; i < DP; ++i)
+#pragma unroll
+            for (int h = 0; h < NG; ++h)
+                dot[h] = __builtin_fma(qd[(min(h, group - 1) * 8 + part) * kQStride + i], kd[i], dot[h]);
+#pragma unroll
+        for (int h = 0; h < NG; ++h) dot[h] = octet_sum(dot[h]);
+#pragma unroll
+        for (int h = 0; h < NG; ++h)
+            if (part == h && h < group && t < t1) es[h * per + t - t0] = dot[h] * scale;
+    }
+    __syncthreads();
+
+    // Softmax terms: 32 lanes per head. A split whose scores are all -infinity contributes nothing (its terms are 0).
+    {
+        const int h = tid >> 5, l = tid & 31;
+        if (h < group) {
+            double m = -INFINITY, total = 0.0;
+            for (int t = l; t < count; t += 32) m = fmax(m, es[h * per + t]);
+#pragma unroll
+            for (int o = 16; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+            for (int t = l; t < count; t += 32) {
+                const double score = es[h * per + t];
+                const double e = score == -INFINITY ? 0.0 : exp(score - m);
+                es[h * per + t] = e;
+                total = total + e;
+            }
+#pragma unroll
+            for (int o = 16; o > 0; o >>= 1) total = total + __shfl_xor(total, o, 64);
+            const int t = count + l;  // the last pass's tokens past the end: term 0
+            if (t < (count + kSharedTile - 1) / kSharedTile * kSharedTile) es[h * per + t] = 0.0;
+            if (l == 0) {
+                double* out = partial + (static_cast<int64_t>(head0 + h) * splits + split) * (2 + HD);
+                out[0] = m;
+                out[1] = total;
+            }
+        }
+    }
+    __syncthreads();
+
+    // Unnormalised sums: thread (token group, lane) over its tokens of every pass, for every head.
+    double acc[NG];
+#pragma unroll
+    for (int h = 0; h < NG; ++h) acc[h] = 0.0;
+    const bool value_thread = vgroup < kValueGroups;
+    for (int base = t0; base < t1; base += kSharedTile) {
+        const int first = base + vgroup * kValueTokens;
+        double vd[kValueTokens];
+#pragma unroll
+        for (int i = 0; i < kValueTokens; ++i) {
+            float value = INPUTS && first + i == in.position ? vs_new[lane] : vr[i];
+            value = first + i < t1 ? value : 0.0f;  // (its term is 0 too)
+            vd[i] = value;
+        }
+        if (base + kSharedTile < t1) load_values(base + kSharedTile);
+        if (value_thread) {
+            const double* e = es + (first - t0);
+#pragma unroll
+            for (int i = 0; i < kValueTokens; ++i)
+#pragma unroll
+                for (int h = 0; h < NG; ++h) acc[h] = __builtin_fma(e[min(h, group - 1) * per + i], vd[i], acc[h]);
+        }
+    }
+    if (value_thread && vgroup > 0)
+#pragma unroll
+        for (int h = 0; h < NG; ++h)
+            if (h < group) sums[((vgroup - 1) * group + h) * HD + lane] = acc[h];
+    __syncthreads();
+    if (vgroup == 0)
+#pragma unroll
+        for (int h = 0; h < NG; ++h) {
+            if (h >= group) break;
+            double total = acc[h];
+#pragma unroll
+            for (int g = 0; g < kValueGroups - 1; ++g) total = total + sums[(g * group + h) * HD + lane];
+            partial[(static_cast<int64_t>(head0 + h) * splits + split) * (2 + HD) + 2 + lane] = total;
+        }
+}
+
+// Combines the splits of attention_shared_kernel: one workgroup per head and 32 lanes of it, sixteen shares of the
+// splits each summed by 32 threads (16 loads in flight), the shares then added in order. At most 512 splits (one per
+// thread for the maximum and the total); the same formulas as attention_combine_kernel.
+template <bool INPUTS>
+__global__ __launch_bounds__(kSharedCombineThreads) void attention_shared_combine_kernel(const double* __restrict__ partial,
+                                                                                        int splits, int head_dim,
+                                                                                        float* __restrict__ out, float* q) {
+    constexpr int kShares = kSharedCombineThreads / 32, kWaves = kSharedCombineThreads / 64, kFlight = 16;
+    __shared__ double weight[kSharedCombineThreads];
+    __shared__ double lane_part[kSharedCombineThreads];
+    __shared__ double red[2 * kWaves];
+    const int head = blockIdx.x, tid = threadIdx.x, j = 32 * blockIdx.y + (tid & 31), share = tid >> 5;
+    const int64_t stride = 2 + head_dim;
+    const double* p = partial + static_cast<int64_t>(head) * splits * stride;
+    const int each = (splits + kShares - 1) / kShares, s0 = min(splits, share * each), s1 = min(splits, s0 + each);
+    const int own = min(tid, splits - 1);
+    const double m_s = p[own * stride], l_s = p[own * stride + 1];
+    double o[kFlight];
+#pragma unroll
+    for (int i = 0; i < kFlight; ++i) o[i] = p[min(s0 + i, splits - 1) * stride + 2 + j];
+    if (INPUTS && tid < 32)  // the query rotated in place: split 0 left it after the partials
+        q[head * head_dim + j] = reinterpret_cast<const float*>(
+            partial + static_cast<int64_t>(gridDim.x) * splits * stride)[head * head_dim + j];
+    double m = tid < splits ? m_s : -INFINITY;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) m = fmax(m, __shfl_xor(m, s, 64));
+    if ((tid & 63) == 0) red[tid >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < kWaves; ++i) m = fmax(m, red[i]);
+    const double w = tid < splits && l_s > 0 ? exp(m_s - m) : 0.0;
+    weight[tid] = w;
+    double total = tid < splits ? w * l_s : 0.0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) total = total + __shfl_xor(total, s, 64);
+    if ((tid & 63) == 0) red[kWaves + (tid >> 6)] = total;
+    __syncthreads();
+    total = red[kWaves];
+#pragma unroll
+    for (int i = 1; i < kWaves; ++i) total = total + red[kWaves + i];
+    double sum = 0.0;
+    for (int s = s0; s < s1; s += kFlight) {
+        if (s > s0)
+#pragma unroll
+            for (int i = 0; i < kFlight; ++i) o[i] = p[min(s + i, splits - 1) * stride + 2 + j];
+#pragma unroll
+        for (int i = 0; i < kFlight; ++i)
+            if (s + i < s1) sum = __builtin_fma(weight[s + i], o[i], sum);
+    }
+    lane_part[tid] = sum;
+    __syncthreads();
+    if (tid < 32) {
+        double lane_sum = lane_part[tid];
+#pragma unroll
+        for (int i = 1; i < kShares; ++i) lane_sum = lane_sum + lane_part[tid + 32 * i];
+        out[head * head_dim + j] = static_cast<float>(lane_sum / total);
+    }
+}
+
 __device__ __forceinline__ uint32_t byte_at(const uint8_t* p) { return *(const SATORI_GLOBAL uint8_t*)(p); }
 __device__ __forceinline__ uint32_t half_bits_at(const uint8_t* p) { return byte_at(p) | (byte_at(p + 1) << 8); }
 
@@ -942,9 +1267,11 @@ int attention_splits(int tokens) {
 
 size_t attention_scratch_bytes(int query_heads, int head_dim, int tokens) {
     const int splits = std::max(kMinSplits, attention_splits(tokens));
-    // The partials, then the rotated query of the fused decode form.
-    return static_cast<size_t>(query_heads) * splits * (2 + head_dim) * sizeof(double) +
-           static_cast<size_t>(query_heads) * head_dim * sizeof(float);
+    // The partials, then the rotated query of the fused decode form; at least what any prefix takes in the shared form,
+    // whose splits are more.
+    const size_t bytes = static_cast<size_t>(query_heads) * splits * (2 + head_dim) * sizeof(double) +
+                         static_cast<size_t>(query_heads) * head_dim * sizeof(float);
+    return head_dim % 32 == 0 && head_dim <= 128 ? std::max(bytes, kStaticAttentionBytes) : bytes;
 }
 
 namespace {
@@ -1007,6 +1334,65 @@ bool decode_fusable(int tokens, int head_dim) {
 
 }  // namespace
 
+namespace {
+
+// Splits of the shared form, or 0 where it does not apply: 32 tokens each (one pass of the workgroup: a token's key by
+// eight threads), at most 512 workgroups over the key/value heads (two per CU; more would run in a second round) and,
+// for the no-allocation entry point, partials within its buffer; at most kSharedMaxTokens tokens a split, what a
+// split's terms take of the LDS. Past that, and for other heads, the general split attention.
+int shared_splits(int query_heads, int kv_heads, int head_dim, int tokens) {
+    if (tokens <= 32 || head_dim % 32 != 0 || head_dim > 128 || query_heads / kv_heads > kSharedHeads) return 0;
+    const int64_t fit = static_cast<int64_t>(kStaticAttentionBytes - static_cast<size_t>(query_heads) * head_dim * sizeof(float)) /
+                        (static_cast<int64_t>(query_heads) * (2 + head_dim) * static_cast<int64_t>(sizeof(double)));
+    const int most = static_cast<int>(std::min<int64_t>({512 / kv_heads, kSharedCombineThreads, fit}));
+    if (most < 1) return 0;
+    int per = std::max(kSharedTile, (tokens + most - 1) / most);
+    per = (per + kSharedTile - 1) / kSharedTile * kSharedTile;  // whole passes
+    if (per > kSharedMaxTokens) return 0;
+    return (tokens + per - 1) / per;
+}
+
+template <bool INPUTS>
+hipError_t launch_shared(const float* q, float* q_out, const float* k, const float* v, int query_heads, int kv_heads,
+                         int head_dim, int tokens, int splits, float* out, double* partials, const DecodeInputs& in,
+                         float* k_cache, float* v_cache, hipStream_t stream) {
+    const int per = ((tokens + splits - 1) / splits + kSharedTile - 1) / kSharedTile * kSharedTile;
+    // Query heads per workgroup: all of the key/value head's once their splits fill the chip (512 workgroups, two per
+    // CU); a shorter prefix divides them evenly over more workgroups, each of whose chains is then shorter (12 / 2 heads
+    // of 128 lanes at 300 tokens 10.7 -> 8.0 us, 48 / 8 10.6 -> 8.6; at 1,500, two heads a workgroup, 10.7 -> 9.1).
+    const int all = query_heads / kv_heads, dp = head_dim / 8;
+    int group = all;
+    for (int n : {4, 2, 1})
+        if (n < all && all % n == 0 && kv_heads * splits * (all / n) <= 512) group = n;
+    const size_t lds = sizeof(double) * (static_cast<size_t>(group) * (8 * (dp + 2) + per) +
+                                         static_cast<size_t>(kSharedThreads / head_dim - 1) * group * head_dim) +
+                       sizeof(float) * 2 * head_dim;
+    auto go = [&](auto kernel) {
+        kernel<<<kv_heads * splits * (all / group), kSharedThreads, lds, stream>>>(
+            q, k, v, query_heads, kv_heads, tokens, per, splits, group, partials, in, k_cache, v_cache);
+    };
+    auto pick = [&](auto lanes) {
+        constexpr int DP = decltype(lanes)::value;
+        if (group == 1) go(attention_shared_kernel<INPUTS, DP, 1>);
+        else if (group == 2) go(attention_shared_kernel<INPUTS, DP, 2>);
+        else if (group <= 4) go(attention_shared_kernel<INPUTS, DP, 4>);
+        else if (group <= 6) go(attention_shared_kernel<INPUTS, DP, 6>);
+        else go(attention_shared_kernel<INPUTS, DP, 8>);
+    };
+    switch (head_dim) {
+        case 32: pick(std::integral_constant<int, 4>{}); break;
+        case 64: pick(std::integral_constant<int, 8>{}); break;
+        case 96: pick(std::integral_constant<int, 12>{}); break;
+        case 128: pick(std::integral_constant<int, 16>{}); break;
+        default: return hipErrorInvalidValue;
+    }
+    attention_shared_combine_kernel<INPUTS><<<dim3(query_heads, head_dim / 32), kSharedCombineThreads, 0, stream>>>(
+        partials, splits, head_dim, out, q_out);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_rope_table(int positions, int rotary, double base, double* table, hipStream_t stream) {
     const int64_t n = static_cast<int64_t>(positions) * (rotary / 2);
     if (n <= 0) return hipSuccess;
@@ -1020,6 +1406,12 @@ hipError_t launch_attention_decode(float* q, const float* q_bias, const float* k
                                    const double* rope, float* out, double* partials, hipStream_t stream) {
     const int tokens = position + 1;
     const int64_t kv_width = static_cast<int64_t>(kv_heads) * head_dim;
+    if (const int splits = shared_splits(query_heads, kv_heads, head_dim, tokens)) {
+        if (!partials) return hipErrorInvalidValue;
+        const DecodeInputs in{q_bias, k_new, k_bias, v_new, v_bias, rope, position, rotary, base};
+        return launch_shared<true>(q, q, k_cache, v_cache, query_heads, kv_heads, head_dim, tokens, splits, out, partials,
+                                   in, k_cache, v_cache, stream);
+    }
     if (!decode_fusable(tokens, head_dim)) {  // the two launches it stands for
         hipError_t e = launch_attention_inputs(q, q_bias, k_new, k_bias, k_cache + position * kv_width, v_new, v_bias,
                                                v_cache + position * kv_width, query_heads, kv_heads, head_dim,
@@ -1053,6 +1445,9 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, int 
         return hipGetLastError();
     }
     if (!partials) return hipErrorInvalidValue;
+    if (const int n = shared_splits(query_heads, kv_heads, head_dim, tokens))
+        return launch_shared<false>(q, nullptr, k, v, query_heads, kv_heads, head_dim, tokens, n, out, partials,
+                                    DecodeInputs{}, nullptr, nullptr, stream);
     const int per = (tokens + splits - 1) / splits;
     const int grid = split_grid(query_heads, kv_heads, splits);
     const size_t lds = split_lds_bytes(per, head_dim);

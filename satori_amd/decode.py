@@ -30,7 +30,8 @@ from . import DeviceOps, HipContext, HipGroup, HipQuantizedMatrix, HipStep
 
 
 def decode_attention_launches(tokens: int, head_dim: int) -> int:
-    """Launches of satori_hip_attention_decode over `tokens` cached tokens, by the library's rule: up to 32
+    """Launches of satori_hip_attention_decode over `tokens` cached tokens for heads outside the shared form
+    (shares_attention, which always takes 2 past 32 tokens), by the library's rule: up to 32
     tokens, the attention inputs and the one-workgroup attention (2); beyond, the split attention over
     max(min(32, ceil(tokens / 32)), min(64, ceil(tokens / 128)), ceil(tokens / 2048)) workgroups per head,
     with the inputs inside it (split + combine: 2) while the head fits one workgroup's lanes (at most 256)
@@ -41,6 +42,17 @@ def decode_attention_launches(tokens: int, head_dim: int) -> int:
     per = -(-tokens // splits)
     fits = per * 8 + 3 * head_dim * 4 + 256 * 8 <= 64 * 1024
     return 2 if head_dim <= 256 and per <= 80 and fits else 3
+
+
+def shares_attention(tokens: int, heads: int, kv_heads: int, head_dim: int) -> bool:
+    """Whether the library attends with one workgroup per key/value head and split for all of its query heads (the
+    inputs of a decoded position always inside it): heads of 32, 64, 96 or 128 lanes, at most eight per key/value
+    head, past 32 tokens, while splits of at most 256 tokens suffice."""
+    if tokens <= 32 or head_dim % 32 or head_dim > 128 or heads // kv_heads > 8:
+        return False
+    fit = ((4 << 20) - 4 * heads * head_dim) // (heads * (2 + head_dim) * 8)
+    most = min(512 // kv_heads, 512, fit)
+    return most >= 1 and -(-(-(-tokens // most)) // 32) * 32 <= 256
 
 
 @dataclass
@@ -209,7 +221,9 @@ class DeviceDecoder:
         split = position is not None and position + 1 > 32
         extra = len(self.layers) if split else 0
         if folded:  # q/k/v, the decode attention, o, gate/up (and SwiGlu), down; add + RmsNorm to Q8_K, output
-            attention = decode_attention_launches(position + 1 if position is not None else 1, self.cfg.head_dim)
+            tokens, c = position + 1 if position is not None else 1, self.cfg
+            attention = (2 if shares_attention(tokens, c.heads, c.kv_heads, c.head_dim)
+                         else decode_attention_launches(tokens, c.head_dim))
             return 1 + (4 + attention) * len(self.layers) + 2
         if fused:
             return 2 + 9 * len(self.layers) + 1 + extra

@@ -495,3 +495,61 @@ def test_attention_decode_equals_inputs_then_attention(context, position, heads,
     finally:
         for p in buffers:
             context.free(p)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,tokens", [
+    (1, 1, 32, 33), (2, 1, 64, 63), (6, 2, 96, 64), (4, 1, 128, 65),   # the edges of one 32-token split
+    (5, 1, 128, 97), (35, 5, 32, 255), (48, 8, 96, 257), (64, 8, 64, 300),  # 1 .. 8 query heads, divided and whole
+    (12, 2, 128, 2079), (7, 1, 128, 16385),   # two and three heads a workgroup; 64 tokens a split, its last partial
+    (16, 2, 128, 8129), (3, 3, 96, 40000)])   # all eight heads a workgroup; 256 tokens a split
+def test_attention_shared_by_query_heads(context, heads, kv_heads, head_dim, tokens):
+    # One workgroup per key/value head and split for several of its query heads: within one unit in the last place of
+    # the oracle (sums in FP64, one rounding to FP32), the decode form with the same bits as its two calls, a whole
+    # split of scores of -infinity contributing nothing, and a NaN key reaching exactly its key/value head's outputs.
+    g = rng(heads * 100003 + head_dim * 7 + tokens)
+    kw, position = kv_heads * head_dim, tokens - 1
+    q = np.abs(g.standard_normal(heads * head_dim)).astype(np.float32)
+    k = (g.standard_normal((tokens, kw)) * 0.3).astype(np.float32)
+    v = g.standard_normal((tokens, kw)).astype(np.float32)
+    out = np.zeros(heads * head_dim, np.float32)
+    for masked in (False, True):
+        if masked:
+            k[:min(300, tokens - 1)] = -np.inf
+        S.TransformerOps.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens, out, context)
+        _within_ulp(out, O.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens),
+                    f"masked {masked}")
+    k[position, :head_dim] = np.nan
+    S.TransformerOps.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens, out, context)
+    assert np.array_equal(np.isnan(out), np.arange(out.size) < heads // kv_heads * head_dim)
+
+    k = (g.standard_normal((tokens, kw)) * 0.3).astype(np.float32)
+    qb, kb, vb = ((g.standard_normal(n) * 0.1).astype(np.float32) for n in (q.size, kw, kw))
+    ops, buffers, results = S.DeviceOps(context), [], []
+
+    def dev(arr):
+        p = context.alloc(arr.nbytes)
+        context.upload(p, arr)
+        buffers.append(p)
+        return p
+
+    try:
+        for form in range(3):  # the two calls; one call without and with the table
+            dq, dk, dv, dck, dcv, dout = dev(q), dev(k[position]), dev(v[position]), dev(k), dev(v), dev(out)
+            table = context.alloc(8 * tokens * 32)
+            buffers.append(table)
+            ops.rope_table(tokens, 32, 1e4, table)
+            if form == 0:
+                ops.attention_inputs(dq, dev(qb), dk, dev(kb), dck + 4 * position * kw, dv, dev(vb),
+                                     dcv + 4 * position * kw, heads, kv_heads, head_dim, position, 1e4, 32)
+                ops.grouped_attention(dq, dck, dcv, heads, kv_heads, head_dim, tokens, dout)
+            else:
+                ops.attention_decode(dq, dev(qb), dk, dev(kb), dv, dev(vb), dck, dcv, heads, kv_heads, head_dim, position,
+                                     1e4, 32, dout, table if form == 2 else 0)
+            results.append([context.download(np.zeros(n, np.float32), p).view(np.uint32) for p, n in
+                            ((dout, q.size), (dq, q.size), (dck, k.size), (dcv, v.size))])
+        for other in results[1:]:
+            for name, a, b in zip(("output", "query", "keys", "values"), results[0], other):
+                assert np.array_equal(a, b), name
+    finally:
+        for p in buffers:
+            context.free(p)
