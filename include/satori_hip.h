@@ -371,7 +371,7 @@ int satori_hip_attention_inputs(satori_hip_context* context, float* query, const
  * token-major [tokens][kv_heads * head_dim]. The scores live on the device (no scratch argument). Prefixes
  * longer than 32 tokens are split over several workgroups per head, whose partial sums go to a workspace the
  * context keeps per stream: it is allocated by the first split attention on that stream and grows with the
- * prefix (at least 4 MiB for heads of 32, 64, 96 or 128 lanes); attentions on different streams never share one. While capturing, and while captured steps use the
+ * prefix (4 MiB at least); attentions on different streams never share one. While capturing, and while captured steps use the
  * context stream's workspace, a call that would have to grow it fails with SATORI_HIP_E_INVALID_OPERATION. */
 int satori_hip_grouped_attention(satori_hip_context* context, const float* query, const float* keys,
                                  const float* values, int query_heads, int kv_heads, int head_dim, int tokens,

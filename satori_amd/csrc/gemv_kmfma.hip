@@ -534,6 +534,219 @@ __global__ __launch_bounds__(256, S == 1 ? 3 : 2) void kmfma_kernel(KmfmaArgs a)
     }
 }
 
+// ---- Few row tiles x position tiles: four ways, each its own blocks' operands ----
+// With few tiles the launch is bound by each workgroup's chain of rounds (block loads, staging, two barriers), not by
+// the matrix cores, and by what one CU can draw from the L2. A workgroup is then one row tile x position tile whose
+// four waves each load their own block's weights and codes straight into registers, a step of the next block's as
+// soon as this block's step has read its own (no other wave reads them, so LDS staging would only add barriers);
+// only the terms pass through LDS, double-buffered, one barrier a round that leaves the loads in flight. Lanes of
+// positions past the last read the last one's bytes, so that up to 16 positions fetch half a tile's lines. Measured
+// (us a pass with the pack launch, before -> now): Q4_K 4096 x 4096 at 16 positions 13.3 -> 10.0, 1536 x 8960 at 16
+// 23.2 -> 15.7 and at 64 23.5 -> 17.2, 256 x 14336 at 64 36.8 -> 25.0; Q6_K 4096 x 4096 at 32 15.3 -> 11.3, 1536 x 8960
+// at 64 26.1 -> 16.7. Eight ways were no faster (25.2 for 256 x 14336: the CU's draw from the L2, not the rounds).
+// A block's packed activations in one lane's registers: its codes of every K step, its group sums, the scales of its
+// 16 positions.
+struct CodeRegs {
+    i32x4 c[8];
+    u32x4 sums;
+    u32x4 scales[4];
+};
+
+struct Record {
+    const uint8_t *codes, *sums, *scales;  // this lane's bytes of block 0
+    int64_t codes_step, sums_step, scales_step;
+};
+
+__device__ __forceinline__ i32x4 load_codes(const Record& a, int b, int j) {
+    return *(const SATORI_GLOBAL i32x4*)(a.codes + b * a.codes_step + 1024 * j);
+}
+template <bool SUMS>
+__device__ __forceinline__ void load_rest(const Record& a, int b, CodeRegs& r) {
+    if (SUMS) r.sums = *(const SATORI_GLOBAL u32x4*)(a.sums + b * a.sums_step);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r.scales[q] = *(const SATORI_GLOBAL u32x4*)(a.scales + b * a.scales_step + 32 * q);
+}
+
+// Four codes (a byte each, at most 15) times a factor of at most 7: products of at most 105, so no byte carries.
+__device__ __forceinline__ int times(uint32_t codes, uint32_t factor) {
+    uint32_t product;  // (both 16-bit halves times the factor's low half)
+    __asm__("v_pk_mul_lo_u16 %0, %1, %2 op_sel_hi:[1,0]" : "=v"(product) : "v"(codes), "v"(factor));
+    return static_cast<int>(product);
+}
+
+// The terms of block_terms from registers, refilled with block `nb` of the lane's row and tile as soon as read. Q4_K:
+// the scale s_j = 8 s_hi + s_lo of sub-block j multiplied into its codes as two int8 planes (q s_hi, q s_lo <= 105),
+// so that Dot = 8 sum (q s_hi) c + sum (q s_lo) c is two MFMA chains, each step's planes made in the shadow of the
+// step before.
+__device__ __forceinline__ void way_terms(Q4KRegs& w, const uint8_t* next, CodeRegs& r, const Record& a, int nb, int lane,
+                                          float (&term)[16]) {
+    const int h = lane >> 5;
+    const float d = half_bits_to_float(w.head[0] & 0xFFFFu), dmin = half_bits_to_float(w.head[0] >> 16);
+    // Scales (mins) 0..3 and 4..7, a byte each (Q4KCodec.GetScaleMin).
+    const uint32_t s03 = w.head[1] & 0x3F3F3F3Fu;
+    const uint32_t s47 = (w.head[3] & 0x0F0F0F0Fu) | ((w.head[1] >> 2) & 0x30303030u);
+    const uint32_t m03 = w.head[2] & 0x3F3F3F3Fu;
+    const uint32_t m47 = ((w.head[3] >> 4) & 0x0F0F0F0Fu) | ((w.head[2] >> 2) & 0x30303030u);
+    const uint32_t mine = h ? m47 : m03;
+    w.head = load16_a4(next);
+    // MinProduct = sum over the 16 group sums g of m_(g / 2) * sum_g: one FP16 product (|sum_g| <= 2032,
+    // m <= 63, |total| < 2^21).
+    f16x8 mw;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mw[e] = static_cast<_Float16>(byte_to_float(mine, e / 2));
+    const f32x16 mins = mfma_f16(__builtin_bit_cast(f16x8, r.sums), mw);
+    u32x4 sc[4] = {r.scales[0], r.scales[1], r.scales[2], r.scales[3]};
+    load_rest<true>(a, nb, r);
+    auto expand = [&](int j, i32x4& wh, i32x4& wl) {
+        const uint32_t six = (j < 4 ? s03 : s47) >> (8 * (j & 3));
+        const uint32_t s_lo = six & 7u, s_hi = (six >> 3) & 7u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t q = (w.qs[j >> 1][e] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+            wh[e] = times(q, s_hi);
+            wl[e] = times(q, s_lo);
+        }
+        if (j & 1) w.qs[j >> 1] = load16_a4(next + 16 + 32 * (j >> 1) + 16 * h);
+    };
+    i32x16 hi = {}, lo = {};
+    i32x4 wh, wl;
+    expand(0, wh, wl);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        i32x4 nh, nl;
+        if (j + 1 < 8) expand(j + 1, nh, nl);
+        hi = mfma32(r.c[j], wh, hi);
+        lo = mfma32(r.c[j], wl, lo);
+        r.c[j] = load_codes(a, nb, j);
+        if (j + 1 < 8) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
+            wh = nh;
+            wl = nl;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 4 * q + e;
+            const float scale = __uint_as_float(sc[q][e]);
+            // mins[i] is the exact integer MinProduct, i.e. its float conversion.
+            term[i] = __fsub_rn(__fmul_rn(__fmul_rn(d, scale), static_cast<float>(hi[i] * 8 + lo[i])),
+                                __fmul_rn(__fmul_rn(dmin, scale), mins[i]));
+        }
+}
+
+__device__ __forceinline__ void way_terms(PlaneRegs& w, const uint8_t* next, CodeRegs& r, const Record& a, int nb, int lane,
+                                          float (&term)[16]) {
+    const float d = w.d;
+    w.d = load_plane_d(next, lane);
+    u32x4 sc[4] = {r.scales[0], r.scales[1], r.scales[2], r.scales[3]};
+    load_rest<false>(a, nb, r);
+    i32x16 hi = {}, lo = {};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        hi = mfma32(r.c[j], w.w[0][j], hi);
+        lo = mfma32(r.c[j], w.w[1][j], lo);
+        r.c[j] = load_codes(a, nb, j);
+        w.w[0][j] = load_plane(next, 0, j, lane);
+        w.w[1][j] = load_plane(next, 1, j, lane);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 4 * q + e;
+            term[i] = __fmul_rn(__fmul_rn(__uint_as_float(sc[q][e]), d), static_cast<float>(hi[i] * 128 + lo[i]));
+        }
+}
+
+template <int FORMAT>
+__global__ __launch_bounds__(256, 2) void kmfma_ways_kernel(KmfmaArgs a) {
+    constexpr int S = 4;
+    __shared__ f32x4 terms[2 * S * 4 * 64];  // [round parity][way][quad][lane]
+    const int per_xcd = gridDim.x >> 3;
+    int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    int mi = 0;
+    while (mi + 1 < a.count && u >= a.units[mi]) u -= a.units[mi++];
+    if (u >= a.units[mi]) return;  // whole workgroup
+    const KmfmaMember& m = a.m[mi];
+    const int rows = m.rows, blocks = a.blocks, tiles = a.tiles;
+    const int rt = u / tiles, t = u - rt * tiles;
+    const int way = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5;
+    const int row = rt * kTile + (lane & 31), rounds = (blocks + S - 1) / S;
+    const int from = 16 * (32 * h + min(lane & 31, a.positions - t * kTile - 1));
+    const Record rec = {m.workspace + static_cast<int64_t>(t) * 8192 + from,
+                        m.workspace + kmfma_sums_offset(blocks, tiles) + static_cast<int64_t>(t) * 1024 + from,
+                        m.workspace + kmfma_scales_offset(blocks, tiles) + static_cast<int64_t>(t) * 128 + 16 * h,
+                        static_cast<int64_t>(tiles) * 8192, static_cast<int64_t>(tiles) * 1024,
+                        static_cast<int64_t>(tiles) * 128};
+    using Weights = std::conditional_t<FORMAT == kQ4_K, Q4KRegs, PlaneRegs>;
+    constexpr int kBlockBytes = FORMAT == kQ4_K ? 144 : kPlaneRecord;
+    const uint8_t* weights = FORMAT == kQ4_K ? m.w + static_cast<int64_t>(min(row, rows - 1)) * m.row_bytes
+                                             : m.w + static_cast<int64_t>(rt) * blocks * kPlaneRecord;
+    Weights w;
+    CodeRegs r;
+    {
+        const int b = min(way, blocks - 1);
+        const uint8_t* block = weights + static_cast<int64_t>(b) * kBlockBytes;
+        if constexpr (FORMAT == kQ4_K)
+            load_weights(weights, b, h, w);
+        else
+            load_planes(block, lane, w);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r.c[j] = load_codes(rec, b, j);
+        load_rest<FORMAT == kQ4_K>(rec, b, r);
+    }
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // way w adds up quad w of the lane's outputs
+    for (int k = 0; k < rounds; ++k) {
+        const int b = k * S + way, nb = min(b + S, blocks - 1);
+        float term[16];
+        way_terms(w, weights + static_cast<int64_t>(nb) * kBlockBytes, r, rec, nb, lane, term);
+        f32x4* buf = terms + (k & 1) * (S * 4 * 64);
+        const bool past = b >= blocks;  // its terms are zeros (a sum that starts at +0 is never -0)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = past ? 0.0f : term[4 * q + e];
+            buf[(way * 4 + q) * 64 + lane] = v;
+        }
+        // This round's terms are in LDS; the other half is written next round, and this one only after that round's
+        // barrier, so one barrier a round is enough. Global loads stay in flight over it.
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+        // The round's terms of each owned output, added in block order.
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const f32x4 v = buf[(s * 4 + way) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = __fadd_rn(acc[e], v[e]);
+        }
+    }
+    if (row >= rows) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int p = t * kTile + 8 * way + 4 * h + e;
+        if (p < a.positions) store_f32(m.y + static_cast<int64_t>(p) * rows + row, acc[e]);
+    }
+}
+
+template <int FORMAT>
+void launch_ways(KmfmaArgs& a, hipStream_t stream) {
+    int total = 0;
+    for (int i = 0; i < a.count; ++i) {
+        a.units[i] = (a.m[i].rows + kTile - 1) / kTile * a.tiles;
+        total += a.units[i];
+    }
+    kmfma_ways_kernel<FORMAT><<<(total + 7) / 8 * 8, 256, 0, stream>>>(a);
+}
+
 template <int FORMAT, int S>
 void launch_split(KmfmaArgs& a, hipStream_t stream) {
     int total = 0;
@@ -559,18 +772,32 @@ template <int FORMAT>
 void launch_format(KmfmaArgs& a, hipStream_t stream) {
     long wave_tiles = 0;
     for (int i = 0; i < a.count; ++i) wave_tiles += static_cast<long>((a.m[i].rows + kTile - 1) / kTile) * a.tiles;
-    // Weight planes: at most two ways, whose 256-VGPR budget holds two plane sets (four ways would spill).
+    // Four ways: the kernel without staging; for the weight planes, whose bytes bound it from there on, only while each
+    // tile has a CU (280 tiles of 8960 x 1536: 12.1 against 11.0 us; 256 of 4096 x 4096: 12.1 against 15.5).
     const int split = choose_split(wave_tiles, a.blocks);
-    switch (FORMAT == kQ6_K ? std::min(split, 2) : split) {
-        case 1: launch_split<FORMAT, 1>(a, stream); break;
-        case 2: launch_split<FORMAT, 2>(a, stream); break;
-        default: launch_split<FORMAT, 4>(a, stream); break;
-    }
+    if (split == 4 && (FORMAT == kQ4_K || wave_tiles <= 256)) return launch_ways<FORMAT>(a, stream);
+    if (split == 1)
+        launch_split<FORMAT, 1>(a, stream);
+    else
+        launch_split<FORMAT, 2>(a, stream);
 }
 
 }  // namespace
 
-int kmfma_min_positions() { return 16; }
+// Where the matrix-core product beats the integer kernels, in rows x blocks x positions: its two launches and chain of
+// rounds (10 us for 4096 x 4096, 8 for 1536 x 1536, whatever the positions up to 32) against their time per product.
+// Crossings measured, Q4_K: 14336 x 4096 4.2 positions, 4096 x 4096 7.7, 8960 x 1536 5.5 to 7, 1536 x 8960 9, 256 x 14336
+// about 50, 1024 x 1024 about 40; Q6_K, whose integer kernels take longer a product, from 0.75 of that. Tiles past one
+// per CU take their time in proportion. Q6_K from 16 positions on: its product reads the weight planes, which fewer
+// positions do not build. Gained (us): 14336 x 4096 at 11 positions 31.5 -> 16.1, 4096 x 4096 at 12
+// 13.5 -> 10.0, 1024 x 1024 at 16 7.2 -> 4.8, 256 x 14336 at 16 35.8 -> 11.8.
+bool kmfma_pays(int format, int64_t rows, int blocks, int positions) {
+    if (positions < (format == kQ6_K ? kKmfmaHeldPositions : 4)) return false;
+    const int64_t tiles = (rows + kTile - 1) / kTile * ((positions + kTile - 1) / kTile);
+    int64_t line = std::min<int64_t>(60000 + 28000 * static_cast<int64_t>(blocks), 560000);
+    if (format == kQ6_K) line = line * 4 / 5;
+    return rows * blocks * positions * 256 >= line * std::max<int64_t>(tiles, 256);
+}
 
 size_t kmfma_workspace_bytes(int blocks, int positions) {
     const int tiles = (positions + kTile - 1) / kTile;

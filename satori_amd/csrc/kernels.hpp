@@ -208,7 +208,7 @@ hipError_t launch_gemv_kint_swiglu(const MatDesc* members, LaunchShape shape, co
 
 // Integer K-format product (Q4_K or Q6_K) over `positions` positions on the matrix cores: quantizes the FP32
 // activations x ([positions][blocks * 256]) to Q8_K into `workspace` (kmfma_workspace_bytes), then the
-// product; outputs bit-exact with launch_gemv_kint's. Used from kmfma_min_positions() positions on. `w` is
+// product; outputs bit-exact with launch_gemv_kint's. Used where kmfma_pays says so (rows: all members'). `w` is
 // the resident payload for Q4_K (row_bytes per row) and the matrix's weight planes for Q6_K.
 hipError_t launch_gemv_kmfma(const uint8_t* w, int format, const float* x, uint8_t* workspace, float* y, int rows,
                              int blocks, int64_t row_bytes, int positions, hipStream_t stream);
@@ -283,7 +283,8 @@ hipError_t launch_attention_inputs(float* q, const float* q_bias, const float* k
 // Grouped attention over `tokens` cached positions. Up to 32 tokens one workgroup per head; longer prefixes
 // are split over several workgroups (attention_splits per head, or the shared form's splits, whose workgroups serve
 // several query heads of one key/value head: heads of 32, 64, 96 or 128 lanes) whose FP64 partials go to `scratch`
-// (attention_scratch_bytes: the bytes for `tokens`, which also cover every shorter prefix of these heads).
+// (attention_scratch_bytes, the general form's bytes for `tokens`, which also cover every shorter prefix of these heads,
+// and at least kStaticAttentionBytes, what the shared form takes of it for any prefix).
 // attention_supported is false only where one split's exponentials and staged query would not fit the LDS
 // (more than 134 million tokens).
 hipError_t launch_attention(const float* q, const float* k, const float* v, int query_heads, int kv_heads,
@@ -318,7 +319,10 @@ hipError_t launch_scale_check(const uint8_t* payload, int64_t blocks, int format
 // on `stream`; either side may be pinned host memory from hipHostMalloc.
 constexpr size_t kKernelCopyMaxBytes = size_t(1) << 20;
 hipError_t launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t stream);
-int kmfma_min_positions();
+// Positions from which a K-format product holds its own workspace (and a Q6_K matrix its planes) once it has run,
+// whichever kernel it takes.
+constexpr int kKmfmaHeldPositions = 16;
+bool kmfma_pays(int format, int64_t rows, int blocks, int positions);
 
 // Blocks of the activation row the integer product stages in LDS at once (with the block terms of the
 // workgroup's rows); wider rows are processed in chunks of this many blocks, in block order.

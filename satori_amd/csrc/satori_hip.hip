@@ -94,8 +94,15 @@ struct satori_hip_context {
     satori::DeviceBuffer batch;                      // partial sums of short Q8_0 / Q4_0 batches on the context stream
     satori::DeviceBuffer upload_stage, upload_flag;  // packed payloads on their way into the device layouts
     // Split-attention partials (grouped attention over long prefixes), one buffer per stream the attention
-    // runs on, so attentions on different streams never share one; attentions on one stream run in order.
-    std::vector<std::pair<hipStream_t, satori::DeviceBuffer>> attention;
+    // runs on, so attentions on different streams never share one; attentions on one stream run in order. `granted`
+    // is what calls have been let have, by attention_scratch_bytes; the buffer is at least kStaticAttentionBytes, which
+    // any call of the shared form fits, so that it never has to grow for one within the grant.
+    struct AttentionBuffer {
+        hipStream_t stream;
+        satori::DeviceBuffer buffer;
+        size_t granted;
+    };
+    std::vector<AttentionBuffer> attention;
     int attention_steps = 0;         // live captured steps whose graph uses the context stream's buffer
     bool captured_attention = false; // the capture in progress enqueued a split attention
     // The device address of the no-allocation attention's partials on this context's device (the file-scope
@@ -244,23 +251,25 @@ void* reserve_activations(satori_hip_matrix* m, size_t need) {
     return m->q8k.ptr;
 }
 
-// Workspace of a Q8_0 / Q4_0 batch on the matrix cores, or null where a call of fewer than 32 positions may not
-// allocate or hold one (it then takes the single-position kernel, which needs none). Below 32 positions a call on
-// the context stream uses the context's buffer, so a matrix's first call allocates nothing (hipMalloc took 25 us
-// beside a 14 us product). No graph holds that buffer: a captured step may hold the matrix's own (which then cannot
-// grow), a capture the caller makes of a stream itself holds none.
+// The context's buffer for a matrix-core product of few positions, or null where it may not be used: on another stream
+// than the context's (calls there may overlap) and in any capture (no graph holds it). A call there takes a kernel
+// that needs no workspace, as it does for a matrix's first call: a buffer of the matrix's own took 25 us of hipMalloc
+// beside a 14 us product.
+uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t stream) {
+    if (stream != c->stream || c->capturing) return nullptr;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
+    c->batch.reserve(need);
+    return static_cast<uint8_t*>(c->batch.ptr);
+}
+
+// Workspace of a Q8_0 / Q4_0 batch on the matrix cores, or null where a call of fewer than 32 positions has none. A
+// captured step may hold the matrix's own buffer (which then cannot grow).
 void* batch_workspace(satori_hip_matrix* m, int positions, size_t need, hipStream_t stream) {
     satori_hip_context* c = m->context;
     if (positions >= 32) return reserve_activations(m, need);
     if (c->capturing && stream == c->stream) return m->q8k.bytes >= need ? m->q8k.ptr : nullptr;
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
-    if (stream == c->stream) {
-        c->batch.reserve(need);
-        return c->batch.ptr;
-    }
-    if (m->q8k.bytes < need && (m->steps > 0 || c->capturing)) return nullptr;
-    return reserve_activations(m, need);
+    return small_batch_workspace(c, need, stream);
 }
 
 // Enqueue one FP32-activation product: x [positions][C] -> y [positions][R], all device pointers. Q8_0 and
@@ -311,16 +320,25 @@ const uint8_t* ensure_planes(satori_hip_matrix* m, hipStream_t stream) {
     return static_cast<const uint8_t*>(m->planes.ptr);
 }
 
-// Enqueue the Q8_K integer product. Few positions: one kernel that quantizes the activations itself; many:
-// quantize all positions into the matrix's Q8_K buffer, then the matrix-core product (same outputs). The
-// buffer belongs to the matrix, so many-position executions of one matrix that overlap in time race.
+// Enqueue the Q8_K integer product. Where kmfma_pays: quantize all positions into a Q8_K buffer, then the matrix-core
+// product; else one kernel that quantizes the activations itself (same outputs). From kKmfmaHeldPositions on the
+// buffer belongs to the matrix, so executions of that many positions of one matrix that overlap in time race, and it
+// is held with the weight planes whichever product runs, so that what has run once can be captured at any such count
+// of no more positions.
 void enqueue_kint(satori_hip_matrix* m, const float* x, int positions, float* y, hipStream_t stream) {
     const Shape& s = m->shape;
-    if (positions >= kmfma_min_positions()) {
-        uint8_t* workspace = static_cast<uint8_t*>(reserve_activations(m, kmfma_workspace_bytes(s.blocks, positions)));
-        const uint8_t* planes = ensure_planes(m, stream);
-        check_hip(launch_gemv_kmfma(planes, s.format, x, workspace, y, s.rows, s.blocks,
-                                    s.row_bytes, positions, stream),
+    const bool pays = kmfma_pays(s.format, s.rows, s.blocks, positions);
+    const bool held = positions >= kKmfmaHeldPositions;
+    uint8_t* workspace = nullptr;
+    const uint8_t* weights = m->payload;
+    if (held || pays) {
+        const size_t need = kmfma_workspace_bytes(s.blocks, positions);
+        workspace = held ? static_cast<uint8_t*>(reserve_activations(m, need))
+                         : small_batch_workspace(m->context, need, stream);
+        if (held) weights = ensure_planes(m, stream);
+    }
+    if (pays && workspace) {
+        check_hip(launch_gemv_kmfma(weights, s.format, x, workspace, y, s.rows, s.blocks, s.row_bytes, positions, stream),
                   "matrix-core gemv launch");
         return;
     }
@@ -614,7 +632,7 @@ void enqueue_group(satori_hip_group* g, hipStream_t st) {
 }
 
 // Enqueues one K-format group over `positions` positions (inputs [positions][columns], outputs
-// [positions][rows]): the integer kernel below kmfma_min_positions(), else the matrix-core product, with the
+// [positions][rows]): the integer kernel, or where kmfma_pays the matrix-core product, with the
 // Q8_K pack of each distinct input pointer done once and up to kKmfmaMaxMembers members per launch.
 void enqueue_group_batch(satori_hip_group* g, int positions, hipStream_t st) {
     const Shape& s = g->shape;
@@ -622,11 +640,14 @@ void enqueue_group_batch(satori_hip_group* g, int positions, hipStream_t st) {
         fail(SATORI_HIP_E_NOT_SUPPORTED, "An input transform applies to one-position group launches only.");
     if (g->output.activated)
         fail(SATORI_HIP_E_NOT_SUPPORTED, "An output transform applies to one-position group launches only.");
-    if (positions < kmfma_min_positions()) {
+    int64_t rows = 0;
+    for (const MatDesc& d : g->host) rows += d.rows;
+    const bool pays = kmfma_pays(s.format, rows, s.blocks, positions), held = positions >= kKmfmaHeldPositions;
+    auto integer = [&] {
         check_hip(launch_gemv_kint(g->host.data(), g->descriptors, g->count, launch_shape(s, positions, g->rows_max), st),
                   "integer gemv launch");
-        return;
-    }
+    };
+    if (!pays && !held) return integer();
     std::vector<const float*> inputs;
     std::vector<size_t> slot(g->count);
     for (int i = 0; i < g->count; ++i) {
@@ -635,10 +656,10 @@ void enqueue_group_batch(satori_hip_group* g, int positions, hipStream_t st) {
         if (it == inputs.end()) inputs.push_back(g->host[i].x);
     }
     const size_t per = kmfma_workspace_bytes(s.blocks, positions);
-    if (g->context->capturing && g->batch.bytes < per * inputs.size())
+    if (held && g->context->capturing && g->batch.bytes < per * inputs.size())
         fail(SATORI_HIP_E_INVALID_OPERATION,
              "Run this many-position product once before capturing it (its workspace is allocated on first use).");
-    if (g->steps > 0 && g->batch.bytes < per * inputs.size())  // a captured step holds the current buffer
+    if (held && g->steps > 0 && g->batch.bytes < per * inputs.size())  // a captured step holds the current buffer
         fail(SATORI_HIP_E_INVALID_OPERATION,
              "The workspace of this group cannot grow while a captured step replays it: destroy the step, "
              "or run the largest product before capturing.");
@@ -649,10 +670,16 @@ void enqueue_group_batch(satori_hip_group* g, int positions, hipStream_t st) {
         for (satori_hip_matrix* m : g->members)
             if (m->payload == g->host[i].w) owner = m;
         if (!owner) fail(SATORI_HIP_E_INVALID_OPERATION, "Group member not found.");
-        planes[i] = ensure_planes(owner, st);
+        planes[i] = held ? ensure_planes(owner, st) : owner->payload;  // (fewer positions: Q4_K)
     }
-    g->batch.reserve(per * inputs.size());
-    uint8_t* ws = static_cast<uint8_t*>(g->batch.ptr);
+    uint8_t* ws = nullptr;
+    if (held) {  // whichever product runs (enqueue_kint)
+        g->batch.reserve(per * inputs.size());
+        ws = static_cast<uint8_t*>(g->batch.ptr);
+    } else {
+        ws = small_batch_workspace(g->context, per * inputs.size(), st);
+    }
+    if (!pays || !ws) return integer();
     for (size_t k = 0; k < inputs.size(); ++k)
         check_hip(launch_kmfma_pack(s.format, inputs[k], s.blocks, positions, ws + k * per, st), "Q8_K pack launch");
     for (int i0 = 0; i0 < g->count; i0 += kKmfmaMaxMembers) {
@@ -832,7 +859,7 @@ int satori_hip_context_destroy(satori_hip_context* c) {
         c->batch.release();
         c->upload_stage.release();
         c->upload_flag.release();
-        for (auto& entry : c->attention) entry.second.release();
+        for (auto& entry : c->attention) entry.buffer.release();
         c->attention.clear();
         c->host_x.release();
         c->host_y.release();
@@ -1960,21 +1987,25 @@ double* attention_workspace(satori_hip_context* c, hipStream_t st, int query_hea
     if (attention_splits(tokens) <= 1) return nullptr;
     const size_t need = attention_scratch_bytes(query_heads, head_dim, tokens);
     auto it = std::find_if(c->attention.begin(), c->attention.end(),
-                           [&](const std::pair<hipStream_t, DeviceBuffer>& e) { return e.first == st; });
-    if (c->capturing && (it == c->attention.end() || it->second.bytes < need))
+                           [&](const satori_hip_context::AttentionBuffer& e) { return e.stream == st; });
+    if (c->capturing && (it == c->attention.end() || it->granted < need))
         fail(SATORI_HIP_E_INVALID_OPERATION,
              "Run an attention of these heads and tokens once before capturing it (its workspace is allocated "
              "on first use).");
     if (it == c->attention.end()) {
-        c->attention.emplace_back(st, DeviceBuffer{});
+        c->attention.push_back({st, DeviceBuffer{}, 0});
         it = c->attention.end() - 1;
     }
-    DeviceBuffer& buffer = it->second;
-    if (st == c->stream && c->attention_steps > 0 && buffer.bytes < need)  // captured steps hold it
+    DeviceBuffer& buffer = it->buffer;
+    if (st == c->stream && c->attention_steps > 0 && it->granted < need)  // captured steps hold it
         fail(SATORI_HIP_E_INVALID_OPERATION,
              "The attention workspace cannot grow while captured steps use it: destroy them, or run the "
              "longest attention before capturing.");
-    buffer.reserve(need);
+    if (it->granted < need) {
+        it->granted = 0;
+        buffer.reserve(std::max(need, kStaticAttentionBytes));
+        it->granted = need;
+    }
     if (c->capturing && st == c->stream) c->captured_attention = true;
     return static_cast<double*>(buffer.ptr);
 }

@@ -1267,11 +1267,9 @@ int attention_splits(int tokens) {
 
 size_t attention_scratch_bytes(int query_heads, int head_dim, int tokens) {
     const int splits = std::max(kMinSplits, attention_splits(tokens));
-    // The partials, then the rotated query of the fused decode form; at least what any prefix takes in the shared form,
-    // whose splits are more.
-    const size_t bytes = static_cast<size_t>(query_heads) * splits * (2 + head_dim) * sizeof(double) +
-                         static_cast<size_t>(query_heads) * head_dim * sizeof(float);
-    return head_dim % 32 == 0 && head_dim <= 128 ? std::max(bytes, kStaticAttentionBytes) : bytes;
+    // The partials, then the rotated query of the fused decode form.
+    return static_cast<size_t>(query_heads) * splits * (2 + head_dim) * sizeof(double) +
+           static_cast<size_t>(query_heads) * head_dim * sizeof(float);
 }
 
 namespace {
@@ -1338,7 +1336,8 @@ namespace {
 
 // Splits of the shared form, or 0 where it does not apply: 32 tokens each (one pass of the workgroup: a token's key by
 // eight threads), at most 512 workgroups over the key/value heads (two per CU; more would run in a second round) and,
-// for the no-allocation entry point, partials within its buffer; at most kSharedMaxTokens tokens a split, what a
+// partials within kStaticAttentionBytes, the no-allocation entry point's buffer and the least of any other; at most
+// kSharedMaxTokens tokens a split, what a
 // split's terms take of the LDS. Past that, and for other heads, the general split attention.
 int shared_splits(int query_heads, int kv_heads, int head_dim, int tokens) {
     if (tokens <= 32 || head_dim % 32 != 0 || head_dim > 128 || query_heads / kv_heads > kSharedHeads) return 0;

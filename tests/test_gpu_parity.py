@@ -1059,6 +1059,61 @@ def test_k_quantizer_special_blocks_in_every_product(context, fmt, rows, positio
                 assert np.all(same), f"row {(p0 + i) % 12}"
 
 
+@pytest.mark.parametrize("fmt,rows,blocks,positions", [
+    (BQ.Q4_K, 4111, 16, 9), (BQ.Q4_K, 4111, 16, 7),     # either side of the line below 16 positions
+    (BQ.Q4_K, 1300, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
+    (BQ.Q4_K, 33, 3, 40), (BQ.Q4_K, 33, 1, 256),        # small products from 16 positions on
+    (BQ.Q6_K, 3001, 6, 16), (BQ.Q6_K, 1300, 4, 50), (BQ.Q6_K, 200, 9, 40)])
+def test_k_batch_kernel_choice(context, fmt, rows, blocks, positions):
+    # The matrix-core product of few tiles and the integer kernels, each where the other ran before: the bits of
+    # single-position products, from a matrix and from a group of two. Captured before it ran, a call of fewer than 16
+    # positions takes the integer kernel and one of more is refused; after it ran, it is captured. Replays give the
+    # same bits.
+    columns = 256 * blocks
+    g = rng(rows + positions)
+    x = g.standard_normal((positions, columns)).astype(np.float32)
+    x[positions // 2, :256] = 0.0
+    data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
+    want = np.zeros((positions, rows), np.float32)
+    got = np.zeros_like(want)
+    dx, dy, dz = context.alloc(x.nbytes), context.alloc(want.nbytes), context.alloc(want.nbytes)
+    context.upload(dx, x)
+
+    def same(p):
+        return np.array_equal(context.download(got, p).view(np.uint32), want.view(np.uint32))
+
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        for i in range(positions):
+            m.execute_batch(x[i], 1, want[i])
+        group = S.HipGroup(context, [m, m], [dx, dx], [dy, dz], True)
+        for run in (lambda: m.execute_batch_device(dx, positions, dy), lambda: group.execute_batch(positions)):
+            for ran in (False, True):
+                context.capture_begin()
+                try:
+                    if positions >= 16 and not ran:
+                        with pytest.raises(S.InvalidOperationException):
+                            run()
+                    else:
+                        run()
+                finally:
+                    step = context.capture_end()
+                if positions < 16 or ran:
+                    for _ in range(3):
+                        context.upload(dy, np.full_like(want, np.nan))
+                        step.execute()
+                        context.synchronize()
+                        assert same(dy), f"replay {ran}"
+                step.dispose()
+                context.upload(dy, np.full_like(want, np.nan))
+                run()
+                context.synchronize()
+                assert same(dy), f"eager {ran}"
+        assert same(dz)
+        group.dispose()
+    for p in (dx, dy, dz):
+        context.free(p)
+
+
 def test_legacy_batch_captured_before_it_ran(context):
     # A batch of fewer than 32 positions that would use the workspace is captured without one (nothing may be
     # allocated then), replays within the FP32 bound, and the same matrix then runs eagerly with a workspace.
