@@ -23,14 +23,14 @@
 // the ways' sums are added at the end of the tile. The tiles' rounds are dealt to one workgroup per CU in equal
 // contiguous ranges (the chip is full and ends together whatever the shape: 4096 x 4096 over 256 positions has 64
 // tiles, over 12 positions 32); a tile cut between workgroups goes through partial sums in the workspace, added by
-// fbatch_fixup_kernel. Up to 64 positions (one position unit) the activations are split by the workgroups that
-// use them (FUSED, 128 rows and four ways); more positions are split once by fbatch_pack_kernel into the workspace,
-// since every row group would split them again, and take 256 rows and two ways: twice the rows halve the parts'
+// fbatch_fixup_kernel. Up to 64 positions, and in smaller products, the activations are split by the workgroups that
+// use them (FUSED, 128 rows and four ways); in larger ones (fbatch_plan) once by fbatch_pack_kernel into the workspace,
+// since every row group would split them again, and then take 256 rows and two ways: twice the rows halve the parts'
 // bytes a workgroup reads, which then bound it (128 rows: 1.3 GB through L2 in 94 us at 11008 x 4096 Q4_0 over 256
 // positions; 256 rows 0.83 GB).
 // Measured, whole call in a queue of calls (us, before: one 32 x 32 tile per wave and block, its workgroups one
-// per 128 rows and position tile): 256 positions 11008 x 4096 Q4_0 152 -> 83, 4096 x 4096 Q8_0 64 -> 41, 256 x 14336
-// Q8_0 195 -> 27; 64 positions 4096 x 4096 Q8_0 62 -> 18; 12 positions (the single-position kernel) 29 -> 14.
+// per 128 rows and position tile): 256 positions 11008 x 4096 Q4_0 152 -> 83, 4096 x 4096 Q8_0 64 -> 41, 256 x 8192
+// Q8_0 116 -> 16; 64 positions 4096 x 4096 Q8_0 62 -> 18; 12 positions (the single-position kernel) 29 -> 14.
 #include <algorithm>
 
 #include "device_common.hpp"
@@ -570,8 +570,15 @@ FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
     FbatchPlan p{};
     const int blocks = columns / 32;
     p.tiles = (positions + kTile - 1) / kTile;
-    p.TP = p.tiles > 1 ? 2 : 1;
-    p.fused = p.tiles <= 2;
+    // Activations converted by each workgroup for itself (fused) while that costs less than the pack launch and its
+    // bytes: measured (us, fused against packed) 256 x 14336 Q8_0 at 90 positions 17.8 against 24.2, 4096 x 1024 at 132
+    // 19.6 against 22.5, 4096 x 4096 at 132 36.0 against 37.2, 11008 x 1024 at 256 40.7 against 36.4. One position tile a
+    // unit (the weights read and converted once per tile, but twice the units to spread) for small products, and longer
+    // where two a unit would leave half a unit empty: 512 x 512 at 256 9.1 against 10.7, 608 x 9024 at 64 15.9 against
+    // 19.5, 2572 x 576 at 256 16.2 against 19.4, 4096 x 4096 at 64 19.2 against 18.9, 4580 x 1120 at 256 28.2 against 25.9.
+    const int64_t products = static_cast<int64_t>(rows) * columns * positions;
+    p.TP = products < 400000000 || (p.tiles % 2 == 1 && products < 1400000000) || p.tiles == 1 ? 1 : 2;
+    p.fused = p.tiles <= 2 || products < 2300000000;
     p.RH = p.fused ? 2 : 4;
     p.ways = 8 / p.RH;
     p.units = (p.tiles + p.TP - 1) / p.TP;
@@ -640,11 +647,13 @@ bool fbatch_pays(int rows, int columns, int positions) {
 
 size_t fbatch_workspace_bytes(int rows, int columns, int positions) {
     // The largest of this and every smaller position count, so that a buffer made for one call serves the smaller
-    // ones (each of the three forms grows with its positions).
+    // ones: the first and the last count of each number of tiles (between them the form changes at most from one of
+    // the two to the other).
     const int cus = device_cus();
-    size_t bytes = fbatch_plan(rows, columns, positions, cus).bytes;
-    for (int limit : {kTile, 2 * kTile})
-        if (positions > limit) bytes = std::max(bytes, fbatch_plan(rows, columns, limit, cus).bytes);
+    size_t bytes = 0;
+    for (int first = 1; first <= positions; first += kTile)
+        for (int n : {first, std::min(positions, first + kTile - 1)})
+            bytes = std::max(bytes, fbatch_plan(rows, columns, n, cus).bytes);
     return bytes;
 }
 

@@ -216,7 +216,7 @@ size_t kmfma_workspace_bytes(int blocks, int positions);
 
 // FP32-activation product (Q8_0 or Q4_0) over `positions` positions (at most 256) on the matrix cores
 // (gemv_fbatch.hip): the activations split into three exact bf16 parts, the product on the resident device layout
-// `w`, its partial sums (and, past 64 positions, the split activations) in `workspace` (fbatch_workspace_bytes on the
+// `w`, its partial sums (and, in large products, the split activations) in `workspace` (fbatch_workspace_bytes on the
 // current device); within 1e-5 * sum |w x| of the scalar reference like the single-position kernel. fbatch_pays: the
 // position counts it is used for.
 bool fbatch_pays(int rows, int columns, int positions);

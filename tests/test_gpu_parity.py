@@ -990,13 +990,15 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
 
 @pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
 @pytest.mark.parametrize("rows,columns,positions", [(1, 64, 32), (63, 32, 40), (129, 96, 65), (257, 4128, 129),
-                                                    (8200, 2080, 6), (513, 9056, 17), (4097, 4128, 31)])
+                                                    (8200, 2080, 6), (513, 9056, 17), (4097, 4128, 31),
+                                                    (9001, 1056, 255), (4097, 2080, 66), (3000, 4128, 120)])
 def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
     # The edges of the matrix-core batch: row groups of 128 (up to 64 positions) and 256 rows with one row more
     # or less, odd block counts, rounds past the last block, tiles cut into many partial sums, and counts below 32
     # on matrices large enough for it. The first and last positions hold an activation from which the split
     # activations give way to plain FP32 sums (2^40), and one just below it; the bound is that of
-    # test_legacy_matrix_core_batch, on the FP64 product.
+    # test_legacy_matrix_core_batch, on the FP64 product. The last three: packed activations, and the form of one and
+    # of two position tiles a unit past 64 positions.
     g = rng(515 + rows + columns + positions)
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
