@@ -772,10 +772,16 @@ template <int FORMAT>
 void launch_format(KmfmaArgs& a, hipStream_t stream) {
     long wave_tiles = 0;
     for (int i = 0; i < a.count; ++i) wave_tiles += static_cast<long>((a.m[i].rows + kTile - 1) / kTile) * a.tiles;
-    // Four ways: the kernel without staging; for the weight planes, whose bytes bound it from there on, only while each
-    // tile has a CU (280 tiles of 8960 x 1536: 12.1 against 11.0 us; 256 of 4096 x 4096: 12.1 against 15.5).
+    // Four ways (the kernel without staging) while each tile has a CU; beyond, for Q4_K, while two workgroups a CU hold
+    // most of them and the rounds of four blocks are worth their exchange, else two ways. Measured (us, four against two
+    // ways): 512 tiles of 4096 x 4096 16.0 against 20.4, 658 of 3000 x 8960 37.7 against 42.5, 376 of 3000 x 1024 8.0
+    // against 8.3; 896 of 4096 x 4096 26.0 against 24.4, 785 of 5000 x 3072 20.1 against 18.6, 560 of 8960 x 1536 (six
+    // blocks: the second round half empty) 13.1 against 11.8, 846 of 9000 x 1024 11.4 against 9.9. The weight planes,
+    // whose bytes bound them from there on: 280 tiles of 8960 x 1536 12.1 against 11.0, 256 of 4096 x 4096 12.1 against
+    // 15.5.
     const int split = choose_split(wave_tiles, a.blocks);
-    if (split == 4 && (FORMAT == kQ4_K || wave_tiles <= 256)) return launch_ways<FORMAT>(a, stream);
+    const bool more = FORMAT == kQ4_K && ((a.blocks > 6 && wave_tiles <= 700) || (a.blocks == 4 && wave_tiles <= 512));
+    if (split == 4 && (wave_tiles <= 256 || more)) return launch_ways<FORMAT>(a, stream);
     if (split == 1)
         launch_split<FORMAT, 1>(a, stream);
     else
@@ -789,13 +795,16 @@ void launch_format(KmfmaArgs& a, hipStream_t stream) {
 // Crossings measured, Q4_K: 14336 x 4096 4.2 positions, 4096 x 4096 7.7, 8960 x 1536 5.5 to 7, 1536 x 8960 9, 256 x 14336
 // about 50, 1024 x 1024 about 40; Q6_K, whose integer kernels take longer a product, from 0.75 of that. Tiles past one
 // per CU take their time in proportion. Q6_K from 16 positions on: its product reads the weight planes, which fewer
-// positions do not build. Gained (us): 14336 x 4096 at 11 positions 31.5 -> 16.1, 4096 x 4096 at 12
+// positions do not build. Past 48 positions only products as small as 512 x 512 at 100 (6.3 against 7.3) stay: the integer
+// kernels quantize every position again in each of a few rows' workgroups (297 x 2816 Q6_K at 84 15.0 against 9.4, 256 x
+// 14336 at 64 23.8 against 25.0). Gained (us): 14336 x 4096 at 11 positions 31.5 -> 16.1, 4096 x 4096 at 12
 // 13.5 -> 10.0, 1024 x 1024 at 16 7.2 -> 4.8, 256 x 14336 at 16 35.8 -> 11.8.
 bool kmfma_pays(int format, int64_t rows, int blocks, int positions) {
     if (positions < (format == kQ6_K ? kKmfmaHeldPositions : 4)) return false;
     const int64_t tiles = (rows + kTile - 1) / kTile * ((positions + kTile - 1) / kTile);
     int64_t line = std::min<int64_t>(60000 + 28000 * static_cast<int64_t>(blocks), 560000);
     if (format == kQ6_K) line = line * 4 / 5;
+    if (positions > 48) line = std::min<int64_t>(line, 110000);
     return rows * blocks * positions * 256 >= line * std::max<int64_t>(tiles, 256);
 }
 
