@@ -9,7 +9,8 @@
 //
 // Two launches. The pack kernel quantizes every (position, block) to Q8_K (the same bytes as the reference
 // quantizer) and stores the codes in the order the MFMA operands are read, with the block scales and the
-// group sums (as FP16) in separate arrays; the product kernel stages each round's blocks in LDS.
+// group sums (as FP16) in separate arrays; the product kernel stages each round's blocks in LDS, or with few tiles
+// loads them straight into registers (kmfma_ways_kernel).
 //
 // Product orientation: D = C x W^T with the positions' codes as the first operand (M = 32 positions) and the
 // weights as the second (N = 32 rows). Lane l = 32h + r then holds the 16 outputs of row r at positions
