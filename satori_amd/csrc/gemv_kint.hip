@@ -500,6 +500,20 @@ constexpr int kMultiThreads = 512;
 constexpr int kMultiPositions = 8;
 constexpr int kMultiLdsBytes = 144 * 1024;
 
+// A position's activations of a chunk of K blocks, in dwords: the codes, then the group sums, then the scales, and the
+// next position's behind them at a whole 16 bytes. Codes and sums are read and written 8 and 16 bytes at a time, and an
+// LDS access that wide has to lie on a multiple of its width. (Sums behind the scales and positions 77 K dwords apart
+// were off it for every K that is not a multiple of 4.)
+constexpr int multi_sums(int K) { return kCodeStride * K; }
+constexpr int multi_scales(int K) { return multi_sums(K) + 8 * K; }
+constexpr int multi_position(int K) { return (multi_scales(K) + K + 3) & ~3; }
+constexpr bool multi_aligned() {
+    for (int K = 1; K <= kMultiLdsBytes / (kActDwords * 4); ++K)
+        if (multi_sums(K) % 4 || multi_position(K) % 4) return false;
+    return kCodeStride % 4 == 0;
+}
+static_assert(multi_aligned(), "16-byte LDS accesses of the staged activations");
+
 template <int FORMAT, bool INLINE>
 __global__ __launch_bounds__(kMultiThreads) void gemv_kint_multi_kernel(KintMembers inline_members,
                                                                          const MatDesc* __restrict__ group,
@@ -516,14 +530,14 @@ __global__ __launch_bounds__(kMultiThreads) void gemv_kint_multi_kernel(KintMemb
     const int nb = s.blocks, K = s.chunk_blocks;
     const int tid = threadIdx.x, lane = tid & 63, c = lane % G, j16 = tid & 15;
 
-    // Per position: codes, scales and group sums of K blocks (as gemv_kint_kernel); then the terms, [position][row][block].
+    // Per position: codes, group sums and scales of K blocks; then the terms, [position][row][block].
     extern __shared__ uint32_t smem[];
     auto act_of = [&](int pp) {
-        uint32_t* base = smem + pp * (kActDwords * K);
-        return ActTile{base, reinterpret_cast<int16_t*>(base + (kCodeStride + 1) * K),
-                       reinterpret_cast<float*>(base + kCodeStride * K)};
+        uint32_t* base = smem + pp * multi_position(K);
+        return ActTile{base, reinterpret_cast<int16_t*>(base + multi_sums(K)),
+                       reinterpret_cast<float*>(base + multi_scales(K))};
     };
-    float* terms = reinterpret_cast<float*>(smem + np * (kActDwords * K));
+    float* terms = reinterpret_cast<float*>(smem + np * multi_position(K));
 
     auto load_pair = [&](int b0, int kb, int p, Raw& r) {
         const int row = row_begin + p / kb, b = b0 + p % kb;
@@ -785,10 +799,13 @@ hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_membe
     };
     while (tile < kMultiRows && workgroups(tile) > 256) ++tile;
     s.rows_per_wg = static_cast<int>(std::min<int64_t>(tile, kMultiRows));
+    // (Up to three dwords a position round its activations up to 16 bytes.)
     const int per_block = per * (kActDwords + s.rows_per_wg) * static_cast<int>(sizeof(uint32_t));
-    s.chunk_blocks = s.blocks < kMultiLdsBytes / per_block ? s.blocks : kMultiLdsBytes / per_block;
+    const int most = (kMultiLdsBytes - per * 3 * static_cast<int>(sizeof(uint32_t))) / per_block;
+    s.chunk_blocks = std::min(s.blocks, most);
     const dim3 grid((s.rows_max + s.rows_per_wg - 1) / s.rows_per_wg, count, slices);
-    const size_t lds = static_cast<size_t>(per_block) * s.chunk_blocks;
+    const size_t lds = sizeof(uint32_t) * static_cast<size_t>(per) *
+                       (multi_position(s.chunk_blocks) + s.rows_per_wg * s.chunk_blocks);
     KintMembers inline_members{};
     const bool in_arguments = count <= kKintInlineMembers;
     if (in_arguments)

@@ -1061,6 +1061,34 @@ def test_k_quantizer_special_blocks_in_every_product(context, fmt, rows, positio
                 assert np.all(same), f"row {(p0 + i) % 12}"
 
 
+@pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
+@pytest.mark.parametrize("rows,blocks,positions,members", [
+    (5000, 5, 4, 1), (5000, 6, 5, 1), (4096, 7, 4, 1), (3000, 11, 3, 1),  # every remainder of four blocks
+    (1536, 35, 5, 1), (2100, 9, 15, 1),                                    # long rows; two slices of eight positions
+    (1024, 90, 2, 32)])                                                    # a second chunk of one block (128-row tiles)
+def test_k_positions_sharing_weights_at_any_block_count(context, fmt, rows, blocks, positions, members):
+    # The integer product of a few positions keeps each position's activations in LDS one after another: whatever the
+    # block count, every member's outputs are the oracle's, bit for bit.
+    columns = 256 * blocks
+    g = rng(rows + 100 * blocks + positions)
+    data = S.quantize_weights((g.standard_normal((rows, columns), dtype=np.float32) * 0.02), rows, columns, fmt)
+    x = g.standard_normal((positions, columns), dtype=np.float32)
+    x[1, :256] = 0.0
+    want = np.stack([O.qk_matvec_quantized_avx2(data, rows, columns, int(fmt), O.q8k_quantize_row(x[p]))
+                     for p in range(positions)]).astype(np.float32)
+    dx, dy = context.alloc(x.nbytes), [context.alloc(want.nbytes) for _ in range(members)]
+    context.upload(dx, x)
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        group = S.HipGroup(context, [m] * members, [dx] * members, dy, True)
+        group.execute_batch(positions)
+        for i, p in enumerate(dy):
+            got = context.download(np.zeros_like(want), p)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"member {i}"
+        group.dispose()
+    for p in (dx, *dy):
+        context.free(p)
+
+
 @pytest.mark.parametrize("fmt,rows,blocks,positions", [
     (BQ.Q4_K, 4111, 16, 9), (BQ.Q4_K, 4111, 16, 7),     # either side of the line below 16 positions
     (BQ.Q4_K, 1300, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
