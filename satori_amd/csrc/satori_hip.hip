@@ -44,10 +44,35 @@ void check_hip(hipError_t e, const char* what) {
              std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// While it lives, this thread's allocations neither fail because of a stream capture in progress (another library's in
+// global mode, or the context's own) nor disturb it.
+struct CaptureRelaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    CaptureRelaxed() = default;
+    CaptureRelaxed(const CaptureRelaxed&) = delete;
+    ~CaptureRelaxed() {
+        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // Device buffer that only grows.
 struct DeviceBuffer {
     void* ptr = nullptr;
     size_t bytes = 0;
+    // For a call that can do without: false when the memory cannot be had (the buffer may then be gone).
+    bool try_reserve(size_t need) {
+        if (need <= bytes) return true;
+        const CaptureRelaxed relaxed;
+        release();
+        if (hipMalloc(&ptr, need) != hipSuccess) {
+            (void)hipGetLastError();
+            ptr = nullptr;
+            return false;
+        }
+        bytes = need;
+        return true;
+    }
     void reserve(size_t need) {
         if (need <= bytes) return;
         if (ptr) (void)hipFree(ptr);
@@ -252,15 +277,14 @@ void* reserve_activations(satori_hip_matrix* m, size_t need) {
 }
 
 // The context's buffer for a matrix-core product of few positions, or null where it may not be used: on another stream
-// than the context's (calls there may overlap) and in any capture (no graph holds it). A call there takes a kernel
-// that needs no workspace, as it does for a matrix's first call: a buffer of the matrix's own took 25 us of hipMalloc
-// beside a 14 us product.
+// than the context's (calls there may overlap), in any capture (no graph holds it) and when the memory cannot be had. A
+// call there takes a kernel that needs no workspace. (A buffer of the matrix's own took 25 us of hipMalloc in its first
+// call, beside a 14 us product.)
 uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t stream) {
     if (stream != c->stream || c->capturing) return nullptr;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
-    c->batch.reserve(need);
-    return static_cast<uint8_t*>(c->batch.ptr);
+    return c->batch.try_reserve(need) ? static_cast<uint8_t*>(c->batch.ptr) : nullptr;
 }
 
 // Workspace of a Q8_0 / Q4_0 batch on the matrix cores, or null where a call of fewer than 32 positions has none. A

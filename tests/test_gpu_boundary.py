@@ -386,6 +386,50 @@ def test_split_attentions_on_two_streams_do_not_share_a_workspace(context):
             context.free(p)
 
 
+def test_short_batches_while_another_stream_is_captured():
+    # Another library's capture, in the global mode that forbids allocations, neither refuses a batch of a few positions
+    # on the context stream (whose workspace is allocated, then grown, during the capture) nor is ended by it: the
+    # capture gives a graph, and the outputs are those of calls outside it.
+    g = rng(60606)
+    hip = _hip()
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    ctx = S.HipContext(0)  # fresh: its workspaces start empty
+    foreign, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(foreign), 1) == 0
+    calls = []
+    for fmt, rows, columns, positions in ((BQ.Q4_K, 4111, 4096, 9), (BQ.Q8_0, 8200, 2080, 6)):
+        data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
+        x = g.standard_normal((positions, columns)).astype(np.float32)
+        dx, dy = ctx.alloc(x.nbytes), ctx.alloc(4 * positions * rows)
+        ctx.upload(dx, x)
+        calls.append((ctx.create(data, S.QuantizedMatrixShape(rows, columns, fmt)), positions, dx, dy,
+                      np.zeros((positions, rows), np.float32)))
+    try:
+        assert hip.hipStreamBeginCapture(foreign, 0) == 0  # hipStreamCaptureModeGlobal
+        try:
+            for m, positions, dx, dy, _ in calls:
+                m.execute_batch_device(dx, positions, dy)
+        finally:
+            ended = hip.hipStreamEndCapture(foreign, ctypes.byref(graph))
+        assert ended == 0 and graph.value
+        hip.hipGraphDestroy(graph)
+        for m, positions, dx, dy, y in calls:
+            during = ctx.download(y, dy).copy()
+            ctx.upload(dy, np.full_like(y, np.nan))
+            m.execute_batch_device(dx, positions, dy)
+            after = ctx.download(y, dy)
+            assert np.array_equal(during.view(np.uint32), after.view(np.uint32))
+    finally:
+        for m, _, dx, dy, _ in calls:
+            m.dispose()
+            ctx.free(dx)
+            ctx.free(dy)
+        ctx.dispose()
+        hip.hipStreamDestroy(foreign)
+
+
 def test_attention_boundary_fixture(context):
     # VulkanAttentionTests.cs:17-29 with fixtures/operators/attention-boundaries-v1.json: 6 heads of 48 lanes at
     # 1, 2, 32, 64 and 128 tokens (across the one-workgroup form's 32-token limit), within 2e-6 + 2e-6 |e| of the
