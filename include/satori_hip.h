@@ -179,7 +179,7 @@ int satori_hip_quantize_q8k(satori_hip_context* context, const float* input, int
  * beyond shapes; the caller keeps the buffers alive until the stream has passed the work.
  * A matrix's launches share its device workspace (Ternary2: the exchange slots or partial sums of its
  * launch plan; K formats: the packed Q8_K of many-position products; Q8_0 / Q4_0: the split activations of
- * many-position products), so executions of one matrix on different streams must not overlap in time:
+ * many-position products, and off the context stream their partial sums), so executions of one matrix on different streams must not overlap in time:
  * the outputs of overlapping executions are undefined. Later executions are not affected (each Ternary2
  * launch tags its exchanges with its own number, so nothing an overlapping launch leaves behind is added
  * in), except the replays of a captured step or capture that overlapped: those reuse their recorded
@@ -313,8 +313,9 @@ int satori_hip_quantize_weights(int format, const float* weights, int rows, int 
  * groups it launches from being destroyed. While capturing, calls that synchronise, allocate or copy
  * through the host fail with SATORI_HIP_E_INVALID_OPERATION (a many-position K product must have run once
  * before, so its workspace exists), and no other thread may use the context. The step records the device
- * addresses of the workspaces it launches with (a matrix's or group's Q8_K buffer, the split attention's
- * partials): while it lives, a call that would grow one of them fails with SATORI_HIP_E_INVALID_OPERATION. */
+ * addresses of the workspaces it launches with (a matrix's activation buffer, a group's Q8_K buffer, the split
+ * attention's partials): while it lives, a call that would grow one of them fails with
+ * SATORI_HIP_E_INVALID_OPERATION. The partial sums of captured Q8_0 / Q4_0 batches are in memory of the step's own. */
 int satori_hip_capture_begin(satori_hip_context* context);
 int satori_hip_capture_end(satori_hip_context* context, satori_hip_step** step);
 

@@ -22,9 +22,9 @@
 // positions, WAYS = 8 / RH blocks a round: each wave owns 64 rows x 32 TP positions of one of the round's blocks, and
 // the ways' sums are added at the end of the tile. The tiles' rounds are dealt to one workgroup per CU in equal
 // contiguous ranges (the chip is full and ends together whatever the shape: 4096 x 4096 over 256 positions has 64
-// tiles, over 12 positions 32); a tile cut between workgroups goes through partial sums in the workspace, added by
+// tiles, over 12 positions 32); a tile cut between workgroups goes through partial sums in the scratch, added by
 // fbatch_fixup_kernel. Up to 64 positions, and in smaller products, the activations are split by the workgroups that
-// use them (FUSED, 128 rows and four ways); in larger ones (fbatch_plan) once by fbatch_pack_kernel into the workspace,
+// use them (FUSED, 128 rows and four ways); in larger ones (fbatch_plan) once by fbatch_pack_kernel into memory,
 // since every row group would split them again, and then take 256 rows and two ways: twice the rows halve the parts'
 // bytes a workgroup reads, which then bound it (128 rows: 1.3 GB through L2 in 94 us at 11008 x 4096 Q4_0 over 256
 // positions; 256 rows 0.83 GB).
@@ -51,10 +51,10 @@ constexpr int kLiftExponent = 24;
 constexpr uint32_t kFlagBits = 0x5F80u;                // a lifted part of 2^64: |x| from 2^40 on (infinite, NaN) is flagged
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// Workspace of the packed form: for 32-column block b and 32-position tile t, 6 KB at (b * tiles + t) * 6144:
+// Parts of the packed form: for 32-column block b and 32-position tile t, 6 KB at (b * tiles + t) * 6144:
 // part s (0: hi, 1: lo, 2: lolo), K step st at (2s + st) * 1024, lane l = 32h + p holding the 8 bf16 of position
-// 32t + p at columns 32b + slot_column(st, h) .. + 7. Positions past the last are zero. Then one word per (block,
-// tile, K step): the tile's flagged positions in that slot's columns. Then the partial sums.
+// 32t + p at columns 32b + slot_column(st, h) .. + 7. Positions past the last are zero. The scratch holds, beside the
+// partial sums and their flags, one word per (block, tile, K step): the tile's flagged positions in that slot's columns.
 //
 // The columns of a block are dealt to the K steps so that a lane's codes are contiguous: Q8_0 lane half h
 // holds bytes 16h .. 16h + 15 of the record, Q4_0 bytes 8h .. 8h + 7 (low nibbles in step 0, high in step 1).
@@ -563,7 +563,8 @@ struct FbatchPlan {
     int TP, RH, ways;
     bool fused;
     int tiles, units, rounds, total, workgroups;
-    size_t flags_offset, partial_offset, slot_flags_offset, tile_flags_offset, bytes;
+    size_t parts;                                                           // bytes of the split activations
+    size_t slot_flags_offset, tile_flags_offset, flags_offset, scratch;     // (the partial sums first)
 };
 
 FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
@@ -589,12 +590,11 @@ FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
     int n = std::min(p.total, cus);  // one workgroup of eight waves per CU
     if (n >= 8) n -= n % 8;
     p.workgroups = n;
-    const size_t parts = p.fused ? 0 : static_cast<size_t>(blocks) * p.tiles * kBlockTileBytes;
-    p.flags_offset = parts;
-    p.partial_offset = parts + (p.fused ? 0 : (static_cast<size_t>(blocks) * p.tiles * 8 + 255) / 256 * 256);
-    p.slot_flags_offset = p.partial_offset + static_cast<size_t>(p.workgroups) * 2 * slot_floats(p.TP, p.RH) * sizeof(float);
+    p.parts = p.fused ? 0 : static_cast<size_t>(blocks) * p.tiles * kBlockTileBytes;
+    p.slot_flags_offset = static_cast<size_t>(p.workgroups) * 2 * slot_floats(p.TP, p.RH) * sizeof(float);
     p.tile_flags_offset = p.slot_flags_offset + static_cast<size_t>(p.workgroups) * 2 * p.TP * 4;
-    p.bytes = p.tile_flags_offset + static_cast<size_t>(p.total / p.rounds) * p.TP * 4;
+    p.flags_offset = p.tile_flags_offset + static_cast<size_t>(p.total / p.rounds) * p.TP * 4;
+    p.scratch = p.flags_offset + (p.fused ? 0 : static_cast<size_t>(blocks) * p.tiles * 8);
     return p;
 }
 
@@ -620,16 +620,15 @@ hipError_t launch_product(const FbatchArgs& a, hipStream_t stream) {
 }
 
 template <int FORMAT>
-hipError_t launch_format(FbatchArgs a, const FbatchPlan& p, uint8_t* workspace, hipStream_t stream) {
+hipError_t launch_format(FbatchArgs a, const FbatchPlan& p, uint8_t* parts, uint32_t* flags, hipStream_t stream) {
     if (p.fused) return p.TP == 1 ? launch_product<FORMAT, 1, true, 2, 4>(a, stream) : launch_product<FORMAT, 2, true, 2, 4>(a, stream);
     const int64_t items = static_cast<int64_t>(a.blocks) * p.tiles * 128;
     if ((items + kThreads - 1) / kThreads > INT32_MAX) return hipErrorInvalidValue;
-    uint32_t* flags = reinterpret_cast<uint32_t*>(workspace + p.flags_offset);
     fbatch_pack_kernel<FORMAT><<<static_cast<unsigned>((items + kThreads - 1) / kThreads), kThreads, 0, stream>>>(
-        a.x, a.blocks * 32, a.positions, p.tiles, workspace, flags);
+        a.x, a.blocks * 32, a.positions, p.tiles, parts, flags);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    a.parts = workspace;
+    a.parts = parts;
     a.flags = flags;
     return launch_product<FORMAT, 2, false, 4, 2>(a, stream);
 }
@@ -645,7 +644,15 @@ bool fbatch_pays(int rows, int columns, int positions) {
     return positions >= 4 && static_cast<int64_t>(rows) * columns * (positions - 1) >= 72000000;
 }
 
-size_t fbatch_workspace_bytes(int rows, int columns, int positions) {
+// What a matrix holds for its batches: the split activations of any count of as many position tiles, and 256 bytes a tile
+// so that it grows with the tiles in every form (a matrix's first call at a count of tiles leaves a buffer, without
+// which that count may not be captured).
+size_t fbatch_held_bytes(int rows, int columns, int positions) {
+    const int tiles = (positions + kTile - 1) / kTile;
+    return fbatch_plan(rows, columns, tiles * kTile, device_cus()).parts + static_cast<size_t>(tiles) * 256;
+}
+
+size_t fbatch_scratch_bytes(int rows, int columns, int positions) {
     // The largest of this and every smaller position count, so that a buffer made for one call serves the smaller
     // ones: the first and the last count of each number of tiles (between them the form changes at most from one of
     // the two to the other).
@@ -653,12 +660,12 @@ size_t fbatch_workspace_bytes(int rows, int columns, int positions) {
     size_t bytes = 0;
     for (int first = 1; first <= positions; first += kTile)
         for (int n : {first, std::min(positions, first + kTile - 1)})
-            bytes = std::max(bytes, fbatch_plan(rows, columns, n, cus).bytes);
+            bytes = std::max(bytes, fbatch_plan(rows, columns, n, cus).scratch);
     return bytes;
 }
 
-hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* workspace, float* y, int rows,
-                              int columns, int positions, hipStream_t stream) {
+hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* parts, uint8_t* scratch, float* y,
+                              int rows, int columns, int positions, hipStream_t stream) {
     if (rows <= 0 || positions <= 0 || columns <= 0) return hipSuccess;
     if ((format != kQ8_0 && format != kQ4_0) || columns % 32 != 0) return hipErrorInvalidValue;
     const FbatchPlan p = fbatch_plan(rows, columns, positions, device_cus());
@@ -666,9 +673,11 @@ hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint
     a.w = w;
     a.x = x;
     a.y = y;
-    a.partial = reinterpret_cast<float*>(workspace + p.partial_offset);
-    a.slot_flags = reinterpret_cast<uint32_t*>(workspace + p.slot_flags_offset);
-    a.tile_flags = reinterpret_cast<uint32_t*>(workspace + p.tile_flags_offset);
+    if (!p.fused && !parts) return hipErrorInvalidValue;
+    a.partial = reinterpret_cast<float*>(scratch);
+    a.slot_flags = reinterpret_cast<uint32_t*>(scratch + p.slot_flags_offset);
+    a.tile_flags = reinterpret_cast<uint32_t*>(scratch + p.tile_flags_offset);
+    uint32_t* flags = reinterpret_cast<uint32_t*>(scratch + p.flags_offset);
     a.rows = rows;
     a.blocks = columns / 32;
     a.positions = positions;
@@ -679,7 +688,8 @@ hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint
     a.workgroups = p.workgroups;
     a.share = p.total / p.workgroups;
     a.longer = p.total % p.workgroups;
-    return format == kQ8_0 ? launch_format<kQ8_0>(a, p, workspace, stream) : launch_format<kQ4_0>(a, p, workspace, stream);
+    return format == kQ8_0 ? launch_format<kQ8_0>(a, p, parts, flags, stream)
+                           : launch_format<kQ4_0>(a, p, parts, flags, stream);
 }
 
 }  // namespace satori

@@ -215,14 +215,16 @@ hipError_t launch_gemv_kmfma(const uint8_t* w, int format, const float* x, uint8
 size_t kmfma_workspace_bytes(int blocks, int positions);
 
 // FP32-activation product (Q8_0 or Q4_0) over `positions` positions (at most 256) on the matrix cores
-// (gemv_fbatch.hip): the activations split into three exact bf16 parts, the product on the resident device layout
-// `w`, its partial sums (and, in large products, the split activations) in `workspace` (fbatch_workspace_bytes on the
-// current device); within 1e-5 * sum |w x| of the scalar reference like the single-position kernel. fbatch_pays: the
-// position counts it is used for.
+// (gemv_fbatch.hip): the activations split into three exact bf16 parts, the product on the resident device layout `w`;
+// within 1e-5 * sum |w x| of the scalar reference like the single-position kernel. fbatch_pays: the position counts it
+// is used for. `parts` (fbatch_held_bytes; may be null below 32 positions) takes the split activations of large
+// products. `scratch` (fbatch_scratch_bytes) takes partial sums, which mean nothing once the call's launches are done,
+// so launches of any matrices that run in order can share it. Both sizes are for the current device.
 bool fbatch_pays(int rows, int columns, int positions);
-size_t fbatch_workspace_bytes(int rows, int columns, int positions);
-hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* workspace, float* y, int rows,
-                              int columns, int positions, hipStream_t stream);
+size_t fbatch_held_bytes(int rows, int columns, int positions);
+size_t fbatch_scratch_bytes(int rows, int columns, int positions);
+hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* parts, uint8_t* scratch, float* y,
+                              int rows, int columns, int positions, hipStream_t stream);
 
 // The Q6_K matrix-core product reads the weights as pre-scaled int8 planes (2.02 bytes a weight, layout in
 // gemv_kmfma.hip), built once from the regrouped resident layout `w` into a buffer of kmfma_planes_bytes.

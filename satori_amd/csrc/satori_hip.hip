@@ -116,7 +116,8 @@ struct satori_hip_context {
     bool live = true;
     int matrices = 0;
     satori::DeviceBuffer x, y, q8k;
-    satori::DeviceBuffer batch;                      // partial sums of short Q8_0 / Q4_0 batches on the context stream
+    satori::DeviceBuffer batch;                      // eager batches on the context stream: partial sums of Q8_0 / Q4_0,
+                                                     // packed activations of short K ones (no graph holds it)
     satori::DeviceBuffer upload_stage, upload_flag;  // packed payloads on their way into the device layouts
     // Split-attention partials (grouped attention over long prefixes), one buffer per stream the attention
     // runs on, so attentions on different streams never share one; attentions on one stream run in order. `granted`
@@ -137,6 +138,7 @@ struct satori_hip_context {
     // Stream capture (satori_hip_capture_begin / _end): the matrices and groups launched on the context
     // stream while capturing, referenced by the step the capture becomes.
     bool capturing = false;
+    std::vector<satori::DeviceBuffer> captured_scratch;  // partial sums of the captured Q8_0 / Q4_0 batches
     std::vector<satori_hip_matrix*> captured_matrices;
     std::vector<satori_hip_group*> captured_groups;
 };
@@ -151,6 +153,7 @@ struct satori_hip_matrix {
     uint32_t t2_generation = 0;  // the last Ternary2 launch's tag in the scratch's exchange slots
     satori::DeviceBuffer q8k;    // activations of the last many-position product (K formats: packed Q8_K;
                                  // Q8_0 / Q4_0: split bf16 parts)
+    satori::DeviceBuffer partials;  // Q8_0 / Q4_0: partial sums of its batches off the context stream
     satori::DeviceBuffer planes; // Q6_K: the matrix-core weight planes, built by the first many-position product
     int groups = 0;              // live groups and captured steps that launch this matrix
     int steps = 0;               // captured steps that launch this matrix directly (they hold its q8k buffer)
@@ -187,6 +190,7 @@ struct satori_hip_step {
     satori_hip_context* context = nullptr;
     std::vector<satori_hip_group*> groups;     // in launch order (each counts this step)
     std::vector<satori_hip_matrix*> matrices;  // launched directly in a captured step (each counts it)
+    std::vector<satori::DeviceBuffer> scratch; // partial sums of its Q8_0 / Q4_0 batches
     bool attention = false;                    // the graph uses the context's split-attention workspace
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -276,24 +280,44 @@ void* reserve_activations(satori_hip_matrix* m, size_t need) {
     return m->q8k.ptr;
 }
 
-// The context's buffer for a matrix-core product of few positions, or null where it may not be used: on another stream
-// than the context's (calls there may overlap), in any capture (no graph holds it) and when the memory cannot be had. A
-// call there takes a kernel that needs no workspace. (A buffer of the matrix's own took 25 us of hipMalloc in its first
-// call, beside a 14 us product.)
-uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t stream) {
-    if (stream != c->stream || c->capturing) return nullptr;
+// Whether `stream` is being captured by the caller, not by satori_hip_capture_begin.
+bool captured_elsewhere(const satori_hip_context* c, hipStream_t stream) {
+    if (c->capturing && stream == c->stream) return false;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
+    return hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
+// The context's buffer for an eager matrix-core product of few positions, or null where it may not be used: on another
+// stream than the context's (calls there may overlap), in any capture (no graph holds it) and when the memory cannot be
+// had. A call there takes a kernel that needs no workspace. (A buffer of the matrix's own took 25 us of hipMalloc in its
+// first call, beside a 14 us product.)
+uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t stream) {
+    if (stream != c->stream || c->capturing || captured_elsewhere(c, stream)) return nullptr;
     return c->batch.try_reserve(need) ? static_cast<uint8_t*>(c->batch.ptr) : nullptr;
 }
 
-// Workspace of a Q8_0 / Q4_0 batch on the matrix cores, or null where a call of fewer than 32 positions has none. A
-// captured step may hold the matrix's own buffer (which then cannot grow).
-void* batch_workspace(satori_hip_matrix* m, int positions, size_t need, hipStream_t stream) {
+// Scratch of a Q8_0 / Q4_0 batch on the matrix cores, or null where there is none. It is up to 34 MB and holds nothing
+// once the call's launches are done, so calls that run in order share it: the eager calls on the context stream the
+// context's, the batches of a captured step the step's own. Batches elsewhere may overlap those: from 32 positions on
+// they use a buffer of the matrix's (of the largest size, so that it never moves under a graph), below it none. (In
+// every matrix's own buffer it took 40 MB instead of 6 for 4096 x 4096 over 256 positions.)
+uint8_t* batch_scratch(satori_hip_matrix* m, int positions, hipStream_t stream) {
     satori_hip_context* c = m->context;
-    if (positions >= 32) return reserve_activations(m, need);
-    if (c->capturing && stream == c->stream) return m->q8k.bytes >= need ? m->q8k.ptr : nullptr;
-    return small_batch_workspace(c, need, stream);
+    const Shape& s = m->shape;
+    constexpr int kChunk = 256;
+    const auto bytes = [&](int n) { return fbatch_scratch_bytes(s.rows, s.columns, std::min(n, kChunk)); };
+    DeviceBuffer* buffer = &c->batch;
+    size_t need = bytes(positions);
+    if (c->capturing && stream == c->stream) {
+        if (positions < 32) return nullptr;
+        if (c->captured_scratch.empty() || c->captured_scratch.back().bytes < need) c->captured_scratch.emplace_back();
+        buffer = &c->captured_scratch.back();
+    } else if (stream != c->stream || captured_elsewhere(c, stream)) {
+        if (positions < 32) return nullptr;
+        buffer = &m->partials;
+        need = bytes(kChunk);
+    }
+    return buffer->try_reserve(need) ? static_cast<uint8_t*>(buffer->ptr) : nullptr;
 }
 
 // Enqueue one FP32-activation product: x [positions][C] -> y [positions][R], all device pointers. Q8_0 and
@@ -302,12 +326,16 @@ void enqueue_float(satori_hip_matrix* m, const float* x, int positions, float* y
     const Shape& s = m->shape;
     if ((s.format == SATORI_HIP_Q8_0 || s.format == SATORI_HIP_Q4_0) && fbatch_pays(s.rows, s.columns, positions)) {
         constexpr int kChunk = 256;
-        const size_t need = fbatch_workspace_bytes(s.rows, s.columns, std::min(positions, kChunk));
-        if (void* workspace = batch_workspace(m, positions, need, stream)) {
+        void* parts = nullptr;
+        if (positions >= 32)
+            parts = reserve_activations(m, fbatch_held_bytes(s.rows, s.columns, std::min(positions, kChunk)));
+        uint8_t* scratch = batch_scratch(m, positions, stream);
+        if (!scratch && positions >= 32) fail(SATORI_HIP_E_OUT_OF_MEMORY, "hipMalloc: partial sums of a batch.");
+        if (scratch) {
             for (int p0 = 0; p0 < positions; p0 += kChunk) {
                 const int n = std::min(kChunk, positions - p0);
                 check_hip(launch_gemv_fbatch(m->payload, s.format, x + static_cast<int64_t>(p0) * s.columns,
-                                             static_cast<uint8_t*>(workspace), y + static_cast<int64_t>(p0) * s.rows,
+                                             static_cast<uint8_t*>(parts), scratch, y + static_cast<int64_t>(p0) * s.rows,
                                              s.rows, s.columns, n, stream),
                           "matrix-core gemv launch");
             }
@@ -479,6 +507,7 @@ void allocate_matrix(satori_hip_matrix* m, int64_t device_bytes) {
 
 void free_matrix(satori_hip_matrix* m) {
     m->q8k.release();
+    m->partials.release();
     m->planes.release();
     if (m->payload) (void)hipFree(m->payload);
     if (m->scratch) (void)hipFree(m->scratch);
@@ -1538,6 +1567,8 @@ int satori_hip_step_destroy(satori_hip_step* s) {
         (void)hipGraphDestroy(s->graph);
         s->exec = nullptr;
         s->graph = nullptr;
+        for (DeviceBuffer& b : s->scratch) b.release();
+        s->scratch.clear();
         for (satori_hip_group* g : s->groups) g->steps--;
         for (satori_hip_matrix* m : s->matrices) {
             m->groups--;
@@ -1581,6 +1612,13 @@ int satori_hip_capture_end(satori_hip_context* c, satori_hip_step** step) {
         std::vector<satori_hip_group*> groups;
         matrices.swap(c->captured_matrices);
         groups.swap(c->captured_groups);
+        struct Scratch {  // freed unless a step takes it
+            std::vector<DeviceBuffer> buffers;
+            ~Scratch() {
+                for (DeviceBuffer& b : buffers) b.release();
+            }
+        } scratch;
+        scratch.buffers.swap(c->captured_scratch);
         hipGraph_t graph = nullptr;
         check_hip(hipStreamEndCapture(c->stream, &graph), "graph capture");
         if (!graph) fail(SATORI_HIP_E_DEVICE, "The capture produced no graph.");
@@ -1594,6 +1632,7 @@ int satori_hip_capture_end(satori_hip_context* c, satori_hip_step** step) {
         st->context = c;
         st->graph = graph;
         st->exec = exec;
+        st->scratch.swap(scratch.buffers);
         for (satori_hip_group* g : groups) {
             if (std::find(st->groups.begin(), st->groups.end(), g) == st->groups.end()) {
                 st->groups.push_back(g);

@@ -430,6 +430,119 @@ def test_short_batches_while_another_stream_is_captured():
         hip.hipStreamDestroy(foreign)
 
 
+@pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
+def test_legacy_batches_share_their_partial_sums(fmt):
+    # The partial sums of Q8_0 / Q4_0 batches are the context's, a captured step's or, off the context stream, the
+    # matrix's: a matrix that has run 256 positions on the context stream holds no more than its split activations
+    # (2.4 MB for 1536 x 1536, in allocations of 2 MiB; the partial sums are 16.8 MB), and every route gives the bits of
+    # the first call, replays with other batches between them included. What may be captured does not depend on it: a
+    # count of position tiles that has not run is refused, and so is a larger one while a step lives.
+    g = rng(70707 + int(fmt))
+    hip = _hip()
+    P = ctypes.c_void_p
+    hip.hipStreamBeginCapture.argtypes = [P, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [P, ctypes.POINTER(P)]
+    hip.hipGraphInstantiate.argtypes = [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]
+    hip.hipGraphLaunch.argtypes = [P, P]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [P]
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    ctx = S.HipContext(0)
+    foreign = P()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(foreign), 1) == 0
+    shapes = [(1536, 1536, 256), (1536, 1536, 40), (9001, 1056, 255), (300, 9056, 70)]  # the third: packed activations
+    mats, xs, bufs, wants = [], [], [], []
+    try:
+        for rows, columns, positions in shapes:
+            data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
+            mats.append(ctx.create(data, S.QuantizedMatrixShape(rows, columns, fmt)))
+            x = g.standard_normal((positions, columns)).astype(np.float32)
+            dx, dy = ctx.alloc(x.nbytes), ctx.alloc(4 * rows * positions)
+            ctx.upload(dx, x)
+            xs.append(x)
+            bufs.append((dx, dy))
+
+        def run(i, stream=0):
+            mats[i].execute_batch_device(bufs[i][0], shapes[i][2], bufs[i][1], stream)
+
+        def check(i, what):
+            got = ctx.download(np.zeros((shapes[i][2], shapes[i][0]), np.float32), bufs[i][1])
+            assert np.array_equal(got.view(np.uint32), wants[i].view(np.uint32)), f"{what} {shapes[i]}"
+            ctx.upload(bufs[i][1], np.full_like(got, np.nan))
+
+        for i in range(4):  # nothing captured before it ran
+            ctx.capture_begin()
+            with pytest.raises(S.InvalidOperationException):
+                run(i)
+            ctx.capture_end().dispose()
+        for i, (rows, columns, positions) in enumerate(shapes):
+            run(i)
+            wants.append(ctx.download(np.zeros((positions, rows), np.float32), bufs[i][1]).copy())
+            assert np.isfinite(wants[i]).all()
+        data = S.quantize_weights((g.standard_normal((1536, 1536)) * 0.02).astype(np.float32), 1536, 1536, fmt)
+        more = [ctx.create(data, S.QuantizedMatrixShape(1536, 1536, fmt)) for _ in range(6)]
+        mats += more
+        created = free_bytes()
+        for m in more:
+            m.execute_batch_device(bufs[0][0], 256, bufs[0][1])
+        ctx.synchronize()
+        assert (created - free_bytes()) / len(more) <= 4 << 20
+
+        ctx.capture_begin()  # small, large, small again: each launch in order on the step's partial sums
+        for i in (1, 2, 0, 3):
+            run(i)
+        with pytest.raises(S.InvalidOperationException):
+            mats[1].execute_batch_device(bufs[0][0], 100, bufs[0][1])
+        step = ctx.capture_end()
+        for replay in range(3):
+            for i in range(4):
+                ctx.upload(bufs[i][1], np.full_like(wants[i], np.nan))
+            step.execute()
+            for i in range(4):
+                check(i, f"replay {replay}")
+            run(replay)
+            check(replay, "eager beside a step")
+        with pytest.raises(S.InvalidOperationException):  # (its buffer would grow)
+            mats[1].execute_batch_device(bufs[0][0], 100, bufs[0][1])
+        step.dispose()
+
+        for i in range(4):
+            run(i, foreign.value)
+            assert hip.hipStreamSynchronize(foreign) == 0
+            check(i, "another stream")
+        graph, exe = P(), P()
+        assert hip.hipStreamBeginCapture(foreign, 2) == 0  # relaxed
+        try:
+            for i in range(4):
+                run(i, foreign.value)
+        finally:
+            ended = hip.hipStreamEndCapture(foreign, ctypes.byref(graph))
+        assert ended == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for replay in range(3):
+            assert hip.hipGraphLaunch(exe, foreign) == 0
+            assert hip.hipStreamSynchronize(foreign) == 0
+            for i in range(4):
+                check(i, f"another library's graph, replay {replay}")
+                run(i)
+                check(i, "eager beside it")
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+    finally:
+        for m in mats:
+            m.dispose()
+        for pair in bufs:
+            for p in pair:
+                ctx.free(p)
+        ctx.dispose()
+        hip.hipStreamDestroy(foreign)
+
+
 def test_attention_boundary_fixture(context):
     # VulkanAttentionTests.cs:17-29 with fixtures/operators/attention-boundaries-v1.json: 6 heads of 48 lanes at
     # 1, 2, 32, 64 and 128 tokens (across the one-workgroup form's 32-token limit), within 2e-6 + 2e-6 |e| of the
