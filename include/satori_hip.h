@@ -176,7 +176,10 @@ int satori_hip_quantize_q8k(satori_hip_context* context, const float* input, int
 /* ---- MatVec, device buffers, asynchronous (resident pipelines and benchmarks) ----
  * Same arithmetic as the host-buffer calls. input/output are device pointers; the work is enqueued on
  * `stream` (NULL = the context stream) and the call returns without waiting. No input validation
- * beyond shapes; the caller keeps the buffers alive until the stream has passed the work.
+ * beyond shapes; the caller keeps the buffers alive until the stream has passed the work. Q8_0 / Q4_0 batches of 4 to
+ * 31 positions of a large matrix run on the matrix cores on the context stream (eagerly and in a captured step, with the
+ * same bits) and as single-position products on any other stream or in another library's capture: both within the
+ * FP32 bound, with last bits of their own.
  * A matrix's launches share its device workspace (Ternary2: the exchange slots or partial sums of its
  * launch plan; K formats: the packed Q8_K of many-position products; Q8_0 / Q4_0: the split activations of
  * many-position products, and off the context stream their partial sums), so executions of one matrix on different streams must not overlap in time:

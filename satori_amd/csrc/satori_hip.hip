@@ -298,9 +298,10 @@ uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t s
 
 // Scratch of a Q8_0 / Q4_0 batch on the matrix cores, or null where there is none. It is up to 34 MB and holds nothing
 // once the call's launches are done, so calls that run in order share it: the eager calls on the context stream the
-// context's, the batches of a captured step the step's own. Batches elsewhere may overlap those: from 32 positions on
-// they use a buffer of the matrix's (of the largest size, so that it never moves under a graph), below it none. (In
-// every matrix's own buffer it took 40 MB instead of 6 for 4096 x 4096 over 256 positions.)
+// context's, the batches of a captured step the step's own (a step may be replayed on any stream), so that a call and its
+// replay take the same kernel and give the same bits. Batches elsewhere may overlap those: from 32 positions on they use
+// a buffer of the matrix's (of the largest size, so that it never moves under a graph), below it none. (In every matrix's
+// own buffer it took 40 MB instead of 6 for 4096 x 4096 over 256 positions.)
 uint8_t* batch_scratch(satori_hip_matrix* m, int positions, hipStream_t stream) {
     satori_hip_context* c = m->context;
     const Shape& s = m->shape;
@@ -309,7 +310,6 @@ uint8_t* batch_scratch(satori_hip_matrix* m, int positions, hipStream_t stream) 
     DeviceBuffer* buffer = &c->batch;
     size_t need = bytes(positions);
     if (c->capturing && stream == c->stream) {
-        if (positions < 32) return nullptr;
         if (c->captured_scratch.empty() || c->captured_scratch.back().bytes < need) c->captured_scratch.emplace_back();
         buffer = &c->captured_scratch.back();
     } else if (stream != c->stream || captured_elsewhere(c, stream)) {

@@ -1145,8 +1145,8 @@ def test_k_batch_kernel_choice(context, fmt, rows, blocks, positions):
 
 
 def test_legacy_batch_captured_before_it_ran(context):
-    # A batch of fewer than 32 positions that would use the workspace is captured without one (nothing may be
-    # allocated then), replays within the FP32 bound, and the same matrix then runs eagerly with a workspace.
+    # A batch of fewer than 32 positions that uses a workspace can be captured before it ran (the workspace is then the
+    # step's), replays within the FP32 bound, and the same matrix then runs eagerly.
     rows, columns, positions = 8200, 2080, 6
     g = rng(99)
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
@@ -1168,13 +1168,44 @@ def test_legacy_batch_captured_before_it_ran(context):
             context.synchronize()
             context.download(y, dy)
             assert np.all(np.abs(y - exact) <= bound)
-        m.execute_batch_device(dx, positions, dy)  # while the step lives: still no workspace
+        m.execute_batch_device(dx, positions, dy)  # while the step lives
         assert np.all(np.abs(context.download(y, dy) - exact) <= bound)
         step.dispose()
         m.execute_batch_device(dx, positions, dy)
         assert np.all(np.abs(context.download(y, dy) - exact) <= bound)
     context.free(dx)
     context.free(dy)
+
+
+@pytest.mark.parametrize("fmt,rows,columns,positions", [(BQ.Q8_0, 8200, 2080, 6), (BQ.Q4_0, 4097, 4128, 31)])
+def test_legacy_short_batch_replays_its_eager_bits(context, fmt, rows, columns, positions):
+    # Captured before or after it ran, in one step or two of the same matrix, a batch of fewer than 32 positions on the
+    # matrix cores gives the bits of the eager call.
+    g = rng(515 + positions)
+    data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
+    x = g.standard_normal((positions, columns)).astype(np.float32)
+    dx, dy, dz = context.alloc(x.nbytes), context.alloc(4 * positions * rows), context.alloc(4 * positions * rows)
+    context.upload(dx, x)
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        steps = []
+        for out in (dy, dz):
+            context.capture_begin()
+            m.execute_batch_device(dx, positions, out)
+            steps.append(context.capture_end())
+            if len(steps) == 1:  # the second step is captured after an eager call
+                m.execute_batch_device(dx, positions, dy)
+                eager = context.download(np.zeros((positions, rows), np.float32), dy)
+        for _ in range(3):
+            for step, out in zip(steps, (dy, dz)):
+                context.upload(out, np.full_like(eager, np.nan))
+                step.execute()
+                m.execute_batch_device(dx, positions, dz if out == dy else dy)
+                got = context.download(np.zeros_like(eager), out)
+                assert np.array_equal(got.view(np.uint32), eager.view(np.uint32))
+        for step in steps:
+            step.dispose()
+    for p in (dx, dy, dz):
+        context.free(p)
 
 
 def _tiny_positions(g, positions, columns, mixed):
