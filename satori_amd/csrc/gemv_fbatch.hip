@@ -15,8 +15,8 @@
 // final scaling by 2^-24 rounds once where the result is subnormal: within 1e-5 * sum |w x| + n * 2^-149 of
 // the reference, like every FP32 path here. A lifted sum stays below 2^118 while |x| < 2^40 (2^26 blocks of the
 // largest code and scale); a position holding a larger, infinite or NaN activation is flagged while it is
-// split, and its outputs are computed by a plain FP32 loop instead (finish_flagged), which overflows and
-// propagates where the reference does.
+// split, and its tile is computed once more from activations as they are (finish_flagged), whose sums overflow and
+// propagate where the reference's do.
 //
 // Launches. fbatch_kernel: a workgroup of eight waves walks (row group, position unit) tiles of 64 RH rows x 32 TP
 // positions, WAYS = 8 / RH blocks a round: each wave owns 64 rows x 32 TP positions of one of the round's blocks, and
@@ -32,6 +32,7 @@
 // per 128 rows and position tile): 256 positions 11008 x 4096 Q4_0 152 -> 83, 4096 x 4096 Q8_0 64 -> 41, 256 x 8192
 // Q8_0 116 -> 16; 64 positions 4096 x 4096 Q8_0 62 -> 18; 12 positions (the single-position kernel) 29 -> 14.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -166,46 +167,151 @@ __device__ __forceinline__ int range_of(const FbatchArgs& a, int r) {
     return r < in_longer ? r / (a.share + 1) : a.longer + (r - in_longer) / a.share;
 }
 
-// Outputs of the flagged positions of one 32-row x 32-position tile, by 256 threads: eight per row, each the plain
-// FP32 block sums (QuantizedMatVec.cs:45-78) of every eighth block, their totals then added in order.
-template <int FORMAT>
-__device__ void finish_flagged(const FbatchArgs& a, int row0, int p0, uint32_t mask, float* totals) {
-    constexpr int kRecord = FORMAT == kQ8_0 ? 32 : 16;
-    const int tid = threadIdx.x, row = row0 + (tid & 31), share = tid >> 5;
-    const int64_t count = static_cast<int64_t>(a.rows) * a.blocks;
-    const int64_t first = static_cast<int64_t>(min(row, a.rows - 1)) * a.blocks;
-    for (; mask; mask &= mask - 1u) {
-        const int p = p0 + __builtin_ctz(mask);
-        if (p >= a.positions) break;
-        if (tid < 256) {
-            float total = 0.0f;
-            for (int b = share; b < a.blocks; b += 8) {
-                const uint8_t* rec = a.w + (first + b) * kRecord;
-                const float* xb = a.x + static_cast<int64_t>(p) * a.blocks * 32 + 32 * b;
-                const u32x4 lo = load16_a4(rec);
-                const u32x4 hi = FORMAT == kQ8_0 ? load16_a4(rec + 16) : lo;
-                const float scale = half_bits_to_float(load2_a2(a.w + count * kRecord + (first + b) * 2));
-                float sum = 0.0f;
+// Eight activations of a flagged position, in parts. Elements of 2^-80 and more are taken as they are (Q4_0: divided by 16,
+// the other factor of its codes 16 q): their parts are above 2^-126, and every sum of products overflows where the plain
+// one does. An infinite or NaN element is its first part alone. Smaller ones (SMALL) are lifted into parts of their own.
+constexpr float kSmallLine = 0x1p-80f;
+template <int FORMAT, bool SMALL>
+__device__ __forceinline__ void split8_unlifted(const float (&v)[8], u32x4 (&part)[3]) {
 #pragma unroll
-                for (int j = 0; j < 32; ++j) {
-                    float q;
-                    if constexpr (FORMAT == kQ8_0)
-                        q = sbyte_to_float(j < 16 ? lo[j >> 2] : hi[(j >> 2) - 4], j & 3);
-                    else  // bytes 16 (q - 8), the low nibbles first
-                        q = 0.0625f * sbyte_to_float((j < 16 ? lo[j >> 2] << 4 : lo[(j >> 2) - 4]) & 0xF0F0F0F0u, j & 3);
-                    sum = __fadd_rn(sum, __fmul_rn(q, load_f32(xb + j)));
-                }
-                total = __fadd_rn(total, __fmul_rn(scale, sum));
+    for (int e = 0; e < 8; e += 2) {
+        uint32_t p[3][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float x = __fmul_rn(v[e + i], SMALL ? kLift : FORMAT == kQ4_0 ? 0.0625f : 1.0f);
+            const float magnitude = __builtin_fabsf(v[e + i]);
+            if ((magnitude < kSmallLine) != SMALL) x = 0.0f;
+            p[0][i] = magnitude != magnitude ? 0x7FC00000u : __float_as_uint(x);
+            float r = __fsub_rn(x, __uint_as_float(__float_as_uint(x) & 0xFFFF0000u));
+            if (!(magnitude < INFINITY)) r = 0.0f;
+            p[1][i] = __float_as_uint(r);
+            p[2][i] = __float_as_uint(__fsub_rn(r, __uint_as_float(p[1][i] & 0xFFFF0000u)));
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s) part[s][e >> 1] = __builtin_amdgcn_perm(p[s][1], p[s][0], 0x07060302u);
+    }
+}
+
+// Whether one of the wave's elements is below 2^-80 (zeros too).
+__device__ __forceinline__ bool any_small(const u32x4 (&v)[4]) {
+    float least = INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) least = __builtin_fminf(least, __builtin_fabsf(__uint_as_float(v[j][e])));
+    return __ballot(least < kSmallLine) != 0;
+}
+
+// Outputs of the flagged positions of one 32-row x 32-position tile, by 4 G waves, each the block sums
+// (QuantizedMatVec.cs:45-78) of every 4 G-th block over the whole tile on the matrix cores, added to those of the waves
+// before it. A wave reads its block's activations in whole lines, a block ahead, and passes them through its own LDS
+// (32 rows of kFlaggedStride floats) into operand order: read in operand order, a line took four requests that the L1
+// did not hold together, and that bound it (11008 x 4096 Q4_0 over 256 positions, every one flagged, 315 us against
+// 250). Measured (us, a batch without flagged positions, with one, with all; in brackets before, when each flagged
+// position was summed in FP32 after another): 11008 x 4096 Q4_0 over 256 96, 176, 250 (144, 2,597); 4096 x 4096 Q8_0 over
+// 256 45, 101, 106 (80, 1,164), over 12 15, 35, 34 (27, 159).
+constexpr int kFlaggedStride = 36;  // padded off the banks
+template <int FORMAT, int G>
+__device__ void finish_flagged(const FbatchArgs& a, int row0, int p0, uint32_t mask, float* lds) {
+    constexpr int kRecord = FORMAT == kQ8_0 ? 32 : 16, kWaves = 4 * G;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, row = row0 + (lane & 31);
+    const uint32_t first = static_cast<uint32_t>(min(row, a.rows - 1)) * a.blocks;  // (a payload has at most 2^31 - 1 bytes)
+    const uint32_t record = first * kRecord + (FORMAT == kQ8_0 ? 16 : 8) * h;
+    const uint8_t* scales = a.w + static_cast<int64_t>(a.rows) * a.blocks * kRecord;
+    const float* x[4];  // piece lane % 8 of positions 8 j + lane / 8
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        x[j] = a.x + static_cast<int64_t>(min(p0 + 8 * j + (lane >> 3), a.positions - 1)) * a.blocks * 32 + 4 * (lane & 7);
+    float* mine = lds + wave * (32 * kFlaggedStride);
+    struct Block {
+        u32x4 x[4];
+        uint32_t raw[4];
+        uint32_t scale;
+    };
+    auto load = [&](int b, Block& o) {
+        b = min(b, a.blocks - 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o.x[j] = load16_a4(reinterpret_cast<const uint8_t*>(x[j] + 32 * b));
+        if constexpr (FORMAT == kQ8_0) {
+            const u32x4 v = load16_a4(a.w + (record + static_cast<uint32_t>(b) * kRecord));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o.raw[e] = v[e];
+        } else {
+            const uint64_t v = load8_a8(a.w + (record + static_cast<uint32_t>(b) * kRecord));
+            o.raw[0] = static_cast<uint32_t>(v);
+            o.raw[1] = static_cast<uint32_t>(v >> 32);
+        }
+        o.scale = load2_a2(scales + (first + b) * 2u);
+    };
+    auto wave_sync = [] {  // LDS written by lanes of this wave, read by others of it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    float acc[16] = {};
+    Block now;
+    load(wave, now);
+    for (int b = wave; b < a.blocks; b += kWaves) {
+        const bool small_too = any_small(now.x);
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            *reinterpret_cast<u32x4*>(mine + (8 * j + (lane >> 3)) * kFlaggedStride + 4 * (lane & 7)) = now.x[j];
+        wave_sync();
+        float v[2][8];
+        u32x4 codes[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const f32x4 q = *reinterpret_cast<const f32x4*>(mine + (lane & 31) * kFlaggedStride +
+                                                                slot_column<FORMAT>(st, h) + e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[st][e + i] = q[i];
             }
-            totals[tid] = total;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) codes[st][k] = code_pair<FORMAT>(now.raw, 4 * st + k);
+        }
+        const float scale = half_bits_to_float(now.scale);
+        load(b + kWaves, now);
+        // The sums of the block's smaller or larger elements, scaled and added up.
+        auto add = [&](auto small) {
+            f32x16 d = {};
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                u32x4 part[3];
+                split8_unlifted<FORMAT, decltype(small)::value>(v[st], part);
+#pragma unroll
+                for (int s = 0; s < 3; ++s)
+                    d = mfma_bf16(__builtin_bit_cast(bf16x8, part[s]), __builtin_bit_cast(bf16x8, codes[st]), d);
+                __builtin_amdgcn_sched_barrier(0);  // (one step's parts at a time: 128 registers, none spilled)
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float sum =
+                    decltype(small)::value ? __builtin_amdgcn_ldexpf(d[i], -kLiftExponent - (FORMAT == kQ4_0 ? 4 : 0)) : d[i];
+                acc[i] = __fadd_rn(acc[i], __fmul_rn(scale, sum));
+            }
+        };
+        add(std::false_type{});
+        if (small_too) add(std::true_type{});
+    }
+    __syncthreads();
+    for (int w = 0; w < kWaves; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if (w > 0) acc[i] = __fadd_rn(lds[64 * i + lane], acc[i]);
+                if (w + 1 < kWaves) lds[64 * i + lane] = acc[i];
+            }
         }
         __syncthreads();
-        if (tid < 32 && row < a.rows) {
-            float total = totals[tid];
-            for (int i = 1; i < 8; ++i) total = __fadd_rn(total, totals[tid + 32 * i]);
-            store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, total);
-        }
-        __syncthreads();
+    }
+    if (wave != kWaves - 1 || row >= a.rows) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int at = 8 * (i >> 2) + 4 * h + (i & 3), p = p0 + at;
+        if (p < a.positions && (mask >> at & 1u)) store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, acc[i]);
     }
 }
 
@@ -494,13 +600,16 @@ __global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a)
 // the flagged positions of any tile. Thread (g, wave q, lane) adds pieces g, g + G, ... of outputs 4q .. 4q + 3 of its
 // lane, four chains at a time, then the chains and the G sums in a fixed order: with many pieces (a few rows of many
 // columns) a single chain of their loads took longer than the product (256 x 14336 Q8_0 over 8 positions: 21.9 us
-// against 13.3) and rounded more.
+// against 13.3) and rounded more. The flags are requested beside the pieces: finish_flagged's registers leave four
+// workgroups a CU, whose round trips count (requested after the pieces' sums: 11008 x 4096 Q4_0 over 256 positions 86.2
+// us against 83.4, 4096 x 4096 Q8_0 over 12 13.5 against 13.2).
 template <int FORMAT, int TP, bool FUSED, int RH, int G>
-__global__ __launch_bounds__(kThreads * G) void fbatch_fixup_kernel(FbatchArgs a) {
-    constexpr int kGroupRows = 64 * RH, kSubs = 2 * RH * TP;
-    __shared__ uint32_t lds_flags;
-    __shared__ float lds_totals[kThreads];
-    __shared__ f32x4 lds_sums[G > 1 ? (G - 1) * kThreads : 1];
+__global__ __launch_bounds__(kThreads * G, 4) void fbatch_fixup_kernel(FbatchArgs a) {
+    constexpr int kGroupRows = 64 * RH, kSubs = 2 * RH * TP, kWaves = 4 * G;
+    __shared__ uint32_t lds_flags[kWaves];
+    __shared__ __align__(16) float lds[kWaves * 32 * kFlaggedStride];
+    f32x4* lds_sums = reinterpret_cast<f32x4*>(lds);  // (G - 1 sums a thread, read before finish_flagged)
+    static_assert((G - 1) * kThreads * sizeof(f32x4) <= sizeof(lds) && kTile * kTile * sizeof(float) <= sizeof(lds));
     const int tile = blockIdx.x / kSubs, sub = blockIdx.x - tile * kSubs;  // sub = (2 rh + rt) * TP + tp
     const int first = range_of(a, tile * a.rounds), last = range_of(a, (tile + 1) * a.rounds - 1);
     const int tid = threadIdx.x % kThreads, g = threadIdx.x / kThreads, q = tid >> 6, lane = tid & 63, h = lane >> 5;
@@ -510,6 +619,16 @@ __global__ __launch_bounds__(kThreads * G) void fbatch_fixup_kernel(FbatchArgs a
     const bool cut = first != last;
     // The piece that starts the tile is its range's last segment, the others their range's first.
     auto slot_of = [&](int i) { return 2 * i + (i == first ? 1 : 0); };
+    uint32_t word = 0u;
+    if constexpr (FUSED) {
+        if (!cut)
+            word = a.tile_flags[tile * TP + tp];
+        else
+            for (int i = first + threadIdx.x; i <= last; i += kThreads * G) word |= a.slot_flags[slot_of(i) * TP + tp];
+    } else {
+        for (int i = threadIdx.x; i < 2 * a.blocks; i += kThreads * G)
+            word |= a.flags[2 * (static_cast<int64_t>(i >> 1) * a.tiles + t) + (i & 1)];
+    }
     f32x4 sum[4] = {};  // one chain per piece in flight
     if (cut)
         for (int i0 = first + g; i0 <= last; i0 += 4 * G) {  // four pieces' loads in flight
@@ -527,22 +646,15 @@ __global__ __launch_bounds__(kThreads * G) void fbatch_fixup_kernel(FbatchArgs a
     f32x4 acc;
 #pragma unroll
     for (int k = 0; k < 4; ++k) acc[k] = __fadd_rn(__fadd_rn(sum[0][k], sum[1][k]), __fadd_rn(sum[2][k], sum[3][k]));
-    if (threadIdx.x == 0) lds_flags = 0u;
     if (G > 1 && g > 0) lds_sums[(g - 1) * kThreads + tid] = acc;
+    if (__ballot(word != 0u))
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) word |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(word), o, 64));
+    if (lane == 0) lds_flags[threadIdx.x >> 6] = word;
     __syncthreads();
-    uint32_t word = 0u;
-    if constexpr (FUSED) {
-        if (!cut)
-            word = a.tile_flags[tile * TP + tp];
-        else
-            for (int i = first + threadIdx.x; i <= last; i += kThreads * G) word |= a.slot_flags[slot_of(i) * TP + tp];
-    } else {
-        for (int i = threadIdx.x; i < 2 * a.blocks; i += kThreads * G)
-            word |= a.flags[2 * (static_cast<int64_t>(i >> 1) * a.tiles + t) + (i & 1)];
-    }
-    if (word) atomicOr(&lds_flags, word);
-    __syncthreads();
-    const uint32_t flagged = lds_flags;
+    uint32_t flagged = 0u;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) flagged |= lds_flags[w];
     if (cut && g == 0) {
 #pragma unroll
         for (int j = 0; j < G - 1; ++j)
@@ -555,7 +667,10 @@ __global__ __launch_bounds__(kThreads * G) void fbatch_fixup_kernel(FbatchArgs a
                 store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, __builtin_amdgcn_ldexpf(acc[k], -kLiftExponent));
         }
     }
-    if (flagged) finish_flagged<FORMAT>(a, row0, t * kTile, flagged, lds_totals);
+    if (flagged) {  // whole workgroup
+        __syncthreads();  // the sums are read
+        finish_flagged<FORMAT, G>(a, row0, t * kTile, flagged, lds);
+    }
 }
 
 // How a launch is cut, for the device's CU count.

@@ -10,6 +10,8 @@ Bars (the tolerance is written in each test):
 """
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 
@@ -995,8 +997,8 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
 def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
     # The edges of the matrix-core batch: row groups of 128 (up to 64 positions) and 256 rows with one row more
     # or less, odd block counts, rounds past the last block, tiles cut into many partial sums, and counts below 32
-    # on matrices large enough for it. The first and last positions hold an activation from which the split
-    # activations give way to plain FP32 sums (2^40), and one just below it; the bound is that of
+    # on matrices large enough for it. The first and last positions hold an activation from which a tile is computed once
+    # more from activations as they are (2^40), and one just below it; the bound is that of
     # test_legacy_matrix_core_batch, on the FP64 product. The last three: packed activations, and the form of one and
     # of two position tiles a unit past 64 positions.
     g = rng(515 + rows + columns + positions)
@@ -1015,6 +1017,97 @@ def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
     exact = xf @ wq.T
     for p in range(positions):
         assert_within(y[p], exact[p], bound[p], f"position {p}")
+
+
+def _large_positions(g, positions, columns):
+    """Activation rows of FP32's whole range: N(0,1) rows that hold 2^41, rows around 2^100 and 2^112, normal and
+    tiny (1e-38, subnormal) rows beside one element of 2^50 or 2^110, magnitudes spread over 2^-149..2^100. The
+    reference's block sums stay finite: 32 products of a code of at most 128 and |x| < 2^115 are below 2^127."""
+    x = g.standard_normal((positions, columns))
+    for p in range(positions):
+        kind = p % 6
+        at = int(g.integers(columns))
+        if kind == 1:
+            x[p, at] = 2.0 ** 41
+        elif kind == 2:
+            x[p] *= 2.0 ** (100 if p % 12 < 6 else 112)
+        elif kind == 3:
+            x[p, ::2] *= 1e-38
+            x[p, ::7] = g.integers(-1000, 1000, x[p, ::7].size) * TINY
+            x[p, at] = 2.0 ** 50
+        elif kind == 4:
+            x[p] *= 1e-36 if p % 12 < 6 else 1e-43
+            x[p, at] = -2.0 ** 110
+        elif kind == 5:
+            x[p] *= np.exp2(g.uniform(-149.0, 100.0, columns))
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
+@pytest.mark.parametrize("rows,columns,positions", [(70, 96, 33), (257, 4128, 40), (33, 9056, 64), (8200, 2080, 6),
+                                                    (1000, 2080, 130), (4097, 4128, 200), (1537, 9056, 250)])
+def test_legacy_batches_of_large_activations(context, fmt, rows, columns, positions):
+    # Positions with an activation of 2^40 and more, all of a batch and among others, in every form of the matrix-core
+    # batch (one and two position tiles a unit, packed activations, tiles in one piece, in a few and in many): each
+    # within the bound of test_legacy_matrix_core_batch of the FP64 product, however small the activations beside the
+    # large one; an infinity, a NaN and an activation whose products overflow give the scalar reference's specials.
+    g = rng(2 ** 16 + rows + columns + positions)
+    w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
+    w[: rows // 2, columns // 2:] = 0.0  # blocks of zero codes and of the smallest scale beside others
+    data = S.quantize_weights(w, rows, columns, fmt)
+    x = _large_positions(g, positions, columns)
+    special = (0, positions // 2, positions - 1)
+    for p, value in zip(special, (np.inf, np.nan, 2.0 ** 127)):
+        x[p] = g.standard_normal(columns)
+        x[p, p % columns] = value
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        y = np.full((positions, rows), np.nan, np.float32)
+        m.execute_batch(x.reshape(-1), positions, y.reshape(-1))
+    wq = O.decode_matrix(data, rows, columns, int(fmt)).astype(np.float64)
+    floor = (columns + columns // 32 + 2) * TINY
+    for p in range(positions):
+        if p not in special:
+            xf = x[p].astype(np.float64)
+            assert_within(y[p], wq @ xf, np.abs(wq) @ np.abs(xf) * 1e-5 + floor, f"position {p}")
+            continue
+        want = O.q_matvec_scalar(data, rows, columns, int(fmt), x[p])
+        assert np.array_equal(np.isnan(y[p]), np.isnan(want)), f"position {p}: NaN"
+        inf = np.isinf(want)
+        assert np.array_equal(np.isinf(y[p]), inf) and np.array_equal(y[p][inf], want[inf]), f"position {p}: Inf"
+
+
+@pytest.mark.parametrize("fmt,rows,columns,positions", [(BQ.Q8_0, 4096, 4096, 256), (BQ.Q8_0, 1536, 8960, 64),
+                                                        (BQ.Q4_0, 8192, 4096, 12)])
+def test_legacy_batches_of_large_activations_take_no_multiple(context, fmt, rows, columns, positions):
+    # A batch whose every position holds an activation of 2^41 (or a NaN) takes the plain batch and the tiles once more,
+    # whatever the count of such positions: at most five times the plain batch (2.1 to 2.6 measured; computed position by
+    # position it took 10 to 26 times as long).
+    g = rng(17)
+    data = S.quantize_weights((g.standard_normal((rows, columns), dtype=np.float32) * 0.02), rows, columns, fmt)
+    x = g.standard_normal((positions, columns), dtype=np.float32)
+    dx, dy = context.alloc(x.nbytes), context.alloc(4 * positions * rows)
+
+    def best(m):
+        times = []
+        for _ in range(5):
+            context.synchronize()
+            start = time.perf_counter()
+            for _ in range(20):
+                m.execute_batch_device(dx, positions, dy)
+            context.synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, fmt)) as m:
+        context.upload(dx, x)
+        m.execute_batch_device(dx, positions, dy)
+        plain = best(m)
+        for value in (2.0 ** 41, np.nan):
+            x[:, 5] = value
+            context.upload(dx, x)
+            assert best(m) <= 5 * plain
+    context.free(dx)
+    context.free(dy)
 
 
 def _q8k_special_row(columns):
