@@ -499,6 +499,16 @@ __global__ __launch_bounds__(kThreads) void gemv_kint_kernel(KintMembers inline_
 constexpr int kMultiThreads = 512;
 constexpr int kMultiPositions = 8;
 constexpr int kMultiLdsBytes = 144 * 1024;
+constexpr int kMultiMembers = 32;  // of one launch
+
+// The tiles of members of different sizes, numbered over the members: one workgroup each, so that consecutive workgroups,
+// which are dealt to the XCDs in turn, all have rows. (In a grid as wide as the largest member, with the smaller ones'
+// workgroups without rows in between, the others were dealt unevenly, and one that found no free CU in its XCD ran in a
+// second round: members of 8399, 64 and 5917 rows x 4096 Q6_K over 3 positions 26.1 us, numbered 16.0, two of 7190 15.5.)
+// Members of one size keep the grid, whose y is the member: finding it in the arguments takes 0.3 to 0.5 us more.
+struct MultiTiles {
+    int first[kMultiMembers];  // of each member; past the last member INT32_MAX
+};
 
 // A position's activations of a chunk of K blocks, in dwords: the codes, then the group sums, then the scales, and the
 // next position's behind them at a whole 16 bytes. Codes and sums are read and written 8 and 16 bytes at a time, and an
@@ -514,17 +524,27 @@ constexpr bool multi_aligned() {
 }
 static_assert(multi_aligned(), "16-byte LDS accesses of the staged activations");
 
-template <int FORMAT, bool INLINE>
+template <int FORMAT, bool INLINE, bool NUMBERED>
 __global__ __launch_bounds__(kMultiThreads) void gemv_kint_multi_kernel(KintMembers inline_members,
                                                                          const MatDesc* __restrict__ group,
-                                                                         LaunchShape s, int per) {
+                                                                         LaunchShape s, int per, MultiTiles tiles) {
     constexpr int G = 4;  // lanes per (row, block) pair
     constexpr int kSlots = kMultiThreads / G, kRows16 = kMultiThreads / 16;
     constexpr int kDepth = 2;  // pairs whose payload is in flight
     using Raw = typename std::conditional<FORMAT == kQ4_K, Q4KRaw, Q6KRaw>::type;
-    const MatDesc m = INLINE ? inline_members.m[blockIdx.y] : group[blockIdx.y];
-    const int row_begin = blockIdx.x * s.rows_per_wg;
-    if (row_begin >= m.rows) return;
+    int member = blockIdx.y, tile = blockIdx.x;
+    if constexpr (NUMBERED) {
+        int begin = 0;
+#pragma unroll
+        for (int i = 1; i < (INLINE ? kKintInlineMembers : kMultiMembers); ++i)
+            if (tile >= tiles.first[i]) {
+                member = i;
+                begin = tiles.first[i];
+            }
+        tile -= begin;
+    }
+    const MatDesc m = INLINE ? inline_members.m[member] : group[member];
+    const int row_begin = tile * s.rows_per_wg;
     const int rows = min(s.rows_per_wg, m.rows - row_begin);
     const int first = blockIdx.z * per, np = min(per, s.positions - first);
     const int nb = s.blocks, K = s.chunk_blocks;
@@ -782,9 +802,14 @@ bool multi_pays(int64_t rows, int blocks, int positions) {
            (blocks >= 8 || positions <= 6);
 }
 
-// In slices of at most kMultiPositions positions, with one workgroup per CU over all slices.
+// In slices of at most kMultiPositions positions, with one workgroup per CU over all slices; at most kMultiMembers
+// members a launch.
 hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_members, int count, LaunchShape s,
                              hipStream_t stream) {
+    for (; count > kMultiMembers; count -= kMultiMembers, members += kMultiMembers, device_members += kMultiMembers) {
+        const hipError_t e = launch_kint_multi(members, device_members, kMultiMembers, s, stream);
+        if (e != hipSuccess) return e;
+    }
     const int slices = multi_slices(s.positions);
     const int per = (s.positions + slices - 1) / slices;
     int64_t rows = 0;
@@ -803,21 +828,34 @@ hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_membe
     const int per_block = per * (kActDwords + s.rows_per_wg) * static_cast<int>(sizeof(uint32_t));
     const int most = (kMultiLdsBytes - per * 3 * static_cast<int>(sizeof(uint32_t))) / per_block;
     s.chunk_blocks = std::min(s.blocks, most);
-    const dim3 grid((s.rows_max + s.rows_per_wg - 1) / s.rows_per_wg, count, slices);
+    const bool in_arguments = count <= kKintInlineMembers;
+    KintMembers inline_members{};
+    MultiTiles tiles;
+    std::fill(tiles.first, tiles.first + kMultiMembers, INT32_MAX);
+    const auto tiles_of = [&](int rows_of) { return (rows_of + s.rows_per_wg - 1) / s.rows_per_wg; };
+    int64_t total = 0;
+    bool even = true;
+    for (int i = 0; i < count; ++i) {
+        if (in_arguments) inline_members.m[i] = members[i];
+        tiles.first[i] = static_cast<int>(std::min<int64_t>(total, INT32_MAX));
+        total += tiles_of(members[i].rows);
+        even = even && tiles_of(members[i].rows) == tiles_of(s.rows_max);
+    }
+    if (total > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid = even ? dim3(tiles_of(s.rows_max), count, slices) : dim3(static_cast<unsigned>(total), 1, slices);
     const size_t lds = sizeof(uint32_t) * static_cast<size_t>(per) *
                        (multi_position(s.chunk_blocks) + s.rows_per_wg * s.chunk_blocks);
-    KintMembers inline_members{};
-    const bool in_arguments = count <= kKintInlineMembers;
-    if (in_arguments)
-        for (int i = 0; i < count; ++i) inline_members.m[i] = members[i];
     auto go = [&](auto kernel) {
-        kernel<<<grid, kMultiThreads, lds, stream>>>(inline_members, device_members, s, per);
+        kernel<<<grid, kMultiThreads, lds, stream>>>(inline_members, device_members, s, per, tiles);
         return hipGetLastError();
     };
-    if (s.format == kQ4_K)
-        return in_arguments ? go(gemv_kint_multi_kernel<kQ4_K, true>) : go(gemv_kint_multi_kernel<kQ4_K, false>);
-    if (s.format == kQ6_K)
-        return in_arguments ? go(gemv_kint_multi_kernel<kQ6_K, true>) : go(gemv_kint_multi_kernel<kQ6_K, false>);
+    auto pick = [&](auto format) {
+        constexpr int F = decltype(format)::value;
+        if (even) return in_arguments ? go(gemv_kint_multi_kernel<F, true, false>) : go(gemv_kint_multi_kernel<F, false, false>);
+        return in_arguments ? go(gemv_kint_multi_kernel<F, true, true>) : go(gemv_kint_multi_kernel<F, false, true>);
+    };
+    if (s.format == kQ4_K) return pick(std::integral_constant<int, kQ4_K>{});
+    if (s.format == kQ6_K) return pick(std::integral_constant<int, kQ6_K>{});
     return hipErrorInvalidValue;
 }
 

@@ -1182,6 +1182,62 @@ def test_k_positions_sharing_weights_at_any_block_count(context, fmt, rows, bloc
         context.free(p)
 
 
+def _random_k(g, rows, columns, fmt):
+    """Weights of many rows from the quantized ones of 32."""
+    data = S.quantize_weights((g.standard_normal((32, columns), dtype=np.float32) * 0.02), 32, columns, fmt)
+    return np.resize(data, data.size // 32 * rows)
+
+
+@pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
+def test_k_positions_sharing_weights_over_uneven_members(context, fmt):
+    # Members of any sizes share one launch of a few positions: outputs bit for bit those of single positions (more
+    # members than travel in the kernel's arguments, than one launch takes, of a row and of many), and members of 8399, 64
+    # and 5917 rows take no longer than 1.3 times two of 7190 (1.0 measured; with workgroups dealt by the largest member's
+    # rows 1.7).
+    columns, positions = 1280, 3
+    g = rng(900 + int(fmt))
+    x = g.standard_normal((positions, 4096), dtype=np.float32)
+    dx = context.alloc(x.nbytes)
+    for rows in ((8399, 64, 5917), (1, 700, 33, 9000, 2, 1500), tuple(40 * i + 1 for i in range(35))):
+        context.upload(dx, np.ascontiguousarray(x[:, :columns]))
+        mats = [context.create(_random_k(g, r, columns, fmt), S.QuantizedMatrixShape(r, columns, fmt)) for r in rows]
+        dy = [context.alloc(4 * positions * r) for r in rows]
+        group = S.HipGroup(context, mats, [dx] * len(rows), dy, True)
+        group.execute_batch(positions)
+        for r, m, p in zip(rows, mats, dy):
+            got, single = context.download(np.zeros((positions, r), np.float32), p), np.zeros(r, np.float32)
+            for i in range(positions):
+                m.execute_batch(np.ascontiguousarray(x[i, :columns]), 1, single)
+                assert np.array_equal(got[i].view(np.uint32), single.view(np.uint32)), (rows, r, i)
+        group.dispose()
+        for m, p in zip(mats, dy):
+            m.dispose()
+            context.free(p)
+
+    context.upload(dx, x)
+    best = []
+    for rows in ((7190, 7190), (8399, 64, 5917)):
+        mats = [context.create(_random_k(g, r, 4096, fmt), S.QuantizedMatrixShape(r, 4096, fmt)) for r in rows]
+        dy = [context.alloc(4 * positions * r) for r in rows]
+        group = S.HipGroup(context, mats, [dx] * len(rows), dy, True)
+        group.execute_batch(positions)
+        times = []
+        for _ in range(10):
+            context.synchronize()
+            start = time.perf_counter()
+            for _ in range(50):
+                group.execute_batch(positions)
+            context.synchronize()
+            times.append(time.perf_counter() - start)
+        best.append(min(times))
+        group.dispose()
+        for m, p in zip(mats, dy):
+            m.dispose()
+            context.free(p)
+    assert best[1] <= 1.3 * best[0]
+    context.free(dx)
+
+
 @pytest.mark.parametrize("fmt,rows,blocks,positions", [
     (BQ.Q4_K, 4111, 16, 9), (BQ.Q4_K, 4111, 16, 7),     # either side of the line below 16 positions
     (BQ.Q4_K, 1300, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
