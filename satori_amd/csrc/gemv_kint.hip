@@ -489,7 +489,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kint_kernel(KintMembers inline_
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same product over a few positions (2 to 15). A workgroup owns a tile of rows of one member at up to
+// The same product over a few positions (multi_pays: from 2, mostly to 15). A workgroup owns a tile of rows of one member at up to
 // kMultiPositions positions: it quantizes those positions' rows, then unpacks every (row, block) pair's weights
 // once for all of them. What bounds the product at these sizes is the vector ALU (unpacking, the quantization every
 // workgroup repeats) and one latency chain, not HBM; a launch slice per position repeated all of it per position.
@@ -790,16 +790,15 @@ constexpr int kMultiRows = 128;  // two sums per thread at kMultiPositions
 int multi_slices(int positions) { return (positions + kMultiPositions - 1) / kMultiPositions; }
 
 // Whether the positions share a workgroup: where a launch slice per position would be bound by its throughput (about
-// 24 M weights x positions), and a slice's positions are not so long that quantizing all of them in every workgroup
-// costs more than reading the weights again. Measured (us, a slice per position against this): 4096 x 4096 Q4_K 7.2
-// and 5.2 at 2 positions, 10.4 and 7.5 at 5, 22.0 and 14.6 at 15; 1536 x 8960 8.4 and 7.1 at 2, 16.9 and 13.1 at 5,
-// but 16.3 and 20.6 at 8 (280 blocks a workgroup); 512 x 1024 4.4 and 5.0 at 8; 256 x 14336 8.7 and 11.3 at 5. Short
-// rows at many positions leave each pair few blocks to share (8960 x 1536 12.5 and 12.8 at 8, 1536 x 1536 6.1 and 7.0 at
-// 12; 3000 x 2048 11.0 and 7.7 at 15).
-bool multi_pays(int64_t rows, int blocks, int positions) {
-    const int slices = multi_slices(positions);
-    return rows * blocks * 256 * positions >= 24000000 && (positions + slices - 1) / slices * blocks <= 180 &&
-           (blocks >= 8 || positions <= 6);
+// 18 M weights x positions), and by more than what quantizing a slice's positions in every workgroup takes. Measured over
+// the same calls as kmfma_pays (us, a slice per position against this): 4096 x 4096 Q4_K 7.2 and 5.2 at 2 positions, 22.0
+// and 14.6 at 15; 14380 x 1280 Q6_K 31.5 and 12.0 at 12; 8000 x 768 Q4_K 5.8 and 5.1 at 6; 3088 x 10752 Q6_K 56 and 27 at
+// 12; but 742 x 4608 Q4_K 6.0 and 8.0 at 8, 721 x 2816 5.8 and 7.1 at 15, 512 x 1024 4.4 and 5.0 at 8. Q6_K, whose
+// slices take longer a product, from 0.8 of that (835 x 9728 at 4 11.1 and 8.9).
+bool multi_pays(int format, int64_t rows, int blocks, int positions) {
+    const int slices = multi_slices(positions), per = (positions + slices - 1) / slices;
+    const int64_t line = 18000000 + 150000 * static_cast<int64_t>(per) * blocks;
+    return rows * blocks * 256 * positions >= (format == kQ6_K ? line * 4 / 5 : line);
 }
 
 // In slices of at most kMultiPositions positions, with one workgroup per CU over all slices; at most kMultiMembers
@@ -867,7 +866,7 @@ hipError_t launch_gemv_kint(const MatDesc* members, const MatDesc* device_member
         if (count > kKintInlineMembers && !device_members) return hipErrorInvalidValue;
         int64_t rows = 0;
         for (int i = 0; i < count; ++i) rows += members[i].rows;
-        if (multi_pays(rows, s.blocks, s.positions)) return launch_kint_multi(members, device_members, count, s, stream);
+        if (multi_pays(s.format, rows, s.blocks, s.positions)) return launch_kint_multi(members, device_members, count, s, stream);
     }
     return launch_kint<kInputPlain>(members, device_members, count, s, InputTransform{}, stream);
 }

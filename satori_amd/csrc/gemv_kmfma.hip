@@ -791,22 +791,24 @@ void launch_format(KmfmaArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Where the matrix-core product beats the integer kernels, in rows x blocks x positions: its two launches and chain of
-// rounds (10 us for 4096 x 4096, 8 for 1536 x 1536, whatever the positions up to 32) against their time per product.
-// Crossings measured, Q4_K: 14336 x 4096 4.2 positions, 4096 x 4096 7.7, 8960 x 1536 5.5 to 7, 1536 x 8960 9, 256 x 14336
-// about 50, 1024 x 1024 about 40; Q6_K, whose integer kernels take longer a product, from 0.75 of that. Tiles past one
-// per CU take their time in proportion. Q6_K from 16 positions on: its product reads the weight planes, which fewer
-// positions do not build. Past 48 positions only products as small as 512 x 512 at 100 (6.3 against 7.3) stay: the integer
-// kernels quantize every position again in each of a few rows' workgroups (297 x 2816 Q6_K at 84 15.0 against 9.4, 256 x
-// 14336 at 64 23.8 against 25.0). Gained (us): 14336 x 4096 at 11 positions 31.5 -> 16.1, 4096 x 4096 at 12
-// 13.5 -> 10.0, 1024 x 1024 at 16 7.2 -> 4.8, 256 x 14336 at 16 35.8 -> 11.8.
+// Where the matrix-core product beats the integer kernels, in rows x columns x positions: its two launches and chain of
+// rounds (9 us for 8960 x 1536, 15 for 14336 x 4096, whatever the positions up to 32) against their time per product.
+// Measured over 130 shapes of 64 to 18,000 rows and 1 to 56 blocks at 29 counts of 2 to 256 positions (us, integer
+// against matrix cores): Q4_K 8960 x 1536 8.4 and 9.4 at 10 positions, 10.8 and 9.5 at 15; 8000 x 768 5.1 and 7.5 at 6;
+// 14380 x 1280 7.2 and 9.2 at 5; 4096 x 4096 10.0 and 10.1 at 8; 256 x 14336 9.8 and 23 at 16. Q6_K, whose integer kernels
+// take longer a product, from 0.8 of that (16805 x 256 at 17 8.7 and 6.8). Tiles past one per CU take half of their share
+// more (30000 x 1792 at 6 15.5 and 12.9), a second position tile less than its share of the launches. Q6_K from 16 positions on: its product
+// reads the weight planes, which fewer positions do not build. Past 48 positions only small products stay: the integer
+// kernels quantize every position again in each of a few rows' workgroups (256 x 14336 at 64 24 and 25). Against the
+// best of the kernels at each of those 3,900 calls the rule loses 1.0% on average, against the kernels before this choice
+// more than 5% only within the 4 to 6 us of a launch.
 bool kmfma_pays(int format, int64_t rows, int blocks, int positions) {
     if (positions < (format == kQ6_K ? kKmfmaHeldPositions : 4)) return false;
     const int64_t tiles = (rows + kTile - 1) / kTile * ((positions + kTile - 1) / kTile);
-    int64_t line = std::min<int64_t>(60000 + 28000 * static_cast<int64_t>(blocks), 560000);
+    int64_t line = std::min<int64_t>((positions > kTile ? 100000 : 200000) + 28000 * static_cast<int64_t>(blocks), 800000);
     if (format == kQ6_K) line = line * 4 / 5;
-    if (positions > 48) line = std::min<int64_t>(line, 110000);
-    return rows * blocks * positions * 256 >= line * std::max<int64_t>(tiles, 256);
+    if (positions > 48) line = std::min<int64_t>(line, 300000);
+    return rows * blocks * positions * 256 >= line * (256 + std::max<int64_t>(tiles - 256, 0) / 2);
 }
 
 size_t kmfma_workspace_bytes(int blocks, int positions) {

@@ -1238,6 +1238,37 @@ def test_k_positions_sharing_weights_over_uneven_members(context, fmt):
     context.free(dx)
 
 
+@pytest.mark.parametrize("rows,columns,few,more,limit", [((8000,), 768, 5, 6, 1.3), ((2400,) * 6, 1280, 3, 5, 1.7),
+                                                         ((14380,), 1280, 4, 5, 1.3)])
+def test_k_batch_time_has_no_step(context, rows, columns, few, more, limit):
+    # Where the choice of the kernel changes with the positions, more of them take at most their share longer (1.03, 1.22
+    # and 1.08 measured; on the matrix cores, too early, 1.5, 2.4 and 1.6).
+    g = rng(2)
+    mats = [context.create(_random_k(g, r, columns, BQ.Q4_K), S.QuantizedMatrixShape(r, columns, BQ.Q4_K)) for r in rows]
+    x = g.standard_normal((more, columns), dtype=np.float32)
+    dx, dy = context.alloc(x.nbytes), [context.alloc(4 * more * r) for r in rows]
+    context.upload(dx, x)
+    group = S.HipGroup(context, mats, [dx] * len(rows), dy, True)
+    best = []
+    for positions in (few, more):
+        group.execute_batch(positions)
+        times = []
+        for _ in range(10):
+            context.synchronize()
+            start = time.perf_counter()
+            for _ in range(100):
+                group.execute_batch(positions)
+            context.synchronize()
+            times.append(time.perf_counter() - start)
+        best.append(min(times))
+    assert best[1] <= limit * best[0]
+    group.dispose()
+    for m, p in zip(mats, dy):
+        m.dispose()
+        context.free(p)
+    context.free(dx)
+
+
 @pytest.mark.parametrize("fmt,rows,blocks,positions", [
     (BQ.Q4_K, 4111, 16, 9), (BQ.Q4_K, 4111, 16, 7),     # either side of the line below 16 positions
     (BQ.Q4_K, 1300, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
