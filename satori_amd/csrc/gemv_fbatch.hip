@@ -27,7 +27,7 @@
 // use them (FUSED, 128 rows and four ways); in larger ones (fbatch_plan) once by fbatch_pack_kernel into memory,
 // since every row group would split them again, and then take 256 rows and two ways: twice the rows halve the parts'
 // bytes a workgroup reads, which then bound it (128 rows: 1.3 GB through L2 in 94 us at 11008 x 4096 Q4_0 over 256
-// positions; 256 rows 0.83 GB).
+// positions; 256 rows 0.83 GB). Short rows under many outputs take whole tiles instead (fbatch_tiles_kernel).
 // Measured, whole call in a queue of calls (us, before: one 32 x 32 tile per wave and block, its workgroups one
 // per 128 rows and position tile): 256 positions 11008 x 4096 Q4_0 152 -> 83, 4096 x 4096 Q8_0 64 -> 41, 256 x 8192
 // Q8_0 116 -> 16; 64 positions 4096 x 4096 Q8_0 62 -> 18; 12 positions (the single-position kernel) 29 -> 14.
@@ -151,8 +151,8 @@ struct FbatchArgs {
     float* y;               // [positions][rows]
     int rows, blocks, positions, tiles;
     int units;              // position units: ceil(tiles / TP)
-    int rounds;             // rounds per tile: ceil(blocks / 2)
-    int total;              // tiles x rounds
+    int rounds;             // rounds per tile: ceil(blocks / ways)
+    int total;              // tiles x rounds (fbatch_tiles_kernel: tiles)
     int workgroups;         // ranges: the first total % workgroups hold total / workgroups + 1 rounds, the others one less
     int share, longer;      // total / workgroups, total % workgroups
 };
@@ -353,8 +353,8 @@ __global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a)
         const int group = tile / a.units, t0 = (tile - group * a.units) * TP;  // row group, first position tile
         const int row0 = group * kGroupRows;
 
-        // ---- staging: this thread's pieces of a round (blocks 2r and 2r + 1; a second block past the last reads the
-        // first again, and is not computed). Addresses are a uniform base per round and a fixed 32-bit offset (a
+        // ---- staging: this thread's pieces of a round (WAYS blocks from WAYS r on; a block past the last reads the last
+        // again, and is not computed). Addresses are a uniform base per round and a fixed 32-bit offset (a
         // payload is at most 2^31 - 1 bytes). ----
         u32x4 wregs[kAhead][kPieces];
         uint32_t woff[kPieces];
@@ -425,9 +425,9 @@ __global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a)
                 for (int j = 0; j < kXLoads; ++j) *reinterpret_cast<u32x4*>(buf + 16 * (tid + kThreads * j)) = xreg[j];
             }
         };
-        // The rows' scales of eight blocks (four rounds) at a time, 16 bytes a row (2-byte aligned; up to 14 bytes past
-        // the last row's end, inside the payload's slack): one line read per row and four rounds, where two bytes a lane
-        // and round took half of the kernel's L2 requests.
+        // The rows' scales of eight blocks (kScaleRounds rounds) at a time, 16 bytes a row (2-byte aligned; up to 14 bytes
+        // past the last row's end, inside the payload's slack): one line read per row and eight blocks, where two bytes a
+        // lane and round took half of the kernel's L2 requests.
         u32x4 sreg;
         const uint8_t* ssrc = scales + static_cast<uint32_t>(min(row0 + tid % kGroupRows, a.rows - 1)) * blocks * 2u;
         auto load_scales = [&](int g) { sreg = *(const SATORI_GLOBAL u32x4_a2*)(ssrc + 16 * min(g, (blocks - 1) >> 3)); };
@@ -596,6 +596,148 @@ __global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a)
     }
 }
 
+// Short rows under many outputs: a workgroup is one tile of 128 rows x 32 positions, W blocks a round, with as many of them
+// on a CU as fit, so that one's loads and stores pass behind another's products. (What bounds fbatch_kernel there is its
+// chain: a tile has one to nine rounds, and one workgroup a CU waits for each tile's first loads, 2.4 us a round in all.
+// A product of three tiles a workgroup, 13771 x 288 Q8_0 over 224 positions, took it 23 us, 15 with tiles twice as large, 9
+// here: whole_tiles.) Wave
+// (way, row tile) multiplies block W k + way of round k for 32 rows; the split activations of a round go through the LDS,
+// double-buffered, the weights straight into registers, both requested two rounds ahead. The ways' sums are added in order.
+template <int FORMAT, int W>
+__global__ __launch_bounds__(256 * W) void fbatch_tiles_kernel(FbatchArgs a) {
+    constexpr int kRecord = FORMAT == kQ8_0 ? 32 : 16;
+    constexpr int kThreads = 256 * W, kRoundBytes = W * kBlockTileBytes, kPieces = kRoundBytes / 16;
+    constexpr int kLoads = (kPieces + kThreads - 1) / kThreads, kSumBytes = (W - 1) * 4 * 64 * 16 * 4;
+    __shared__ __align__(16) uint8_t lds[2 * kRoundBytes > kSumBytes ? 2 * kRoundBytes : kSumBytes];
+    const int per_xcd = gridDim.x >> 3;
+    const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (u >= a.total) return;  // whole workgroup
+    const int group = u / a.tiles, t = u - group * a.tiles;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, rt = (tid >> 6) & 3, way = tid >> 8;
+    const int row = group * 128 + 32 * rt + (lane & 31), blocks = a.blocks, rounds = a.rounds;
+    const uint32_t first = static_cast<uint32_t>(min(row, a.rows - 1)) * blocks;  // (a payload has at most 2^31 - 1 bytes)
+    const uint32_t record = first * kRecord + (FORMAT == kQ8_0 ? 16 : 8) * h;
+    const uint8_t* scales = a.w + static_cast<int64_t>(a.rows) * blocks * kRecord;
+    const uint8_t* parts = a.parts + static_cast<int64_t>(t) * kBlockTileBytes;
+    const int64_t stride = static_cast<int64_t>(a.tiles) * kBlockTileBytes;
+
+    struct Weights {
+        uint32_t raw[4];
+        uint32_t scale;
+    };
+    auto load_weights = [&](int r, Weights& o) {  // (a block past the last reads the last, and is not computed)
+        const uint32_t b = min(W * r + way, blocks - 1);
+        if constexpr (FORMAT == kQ8_0) {
+            const u32x4 v = load16_a4(a.w + (record + b * kRecord));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o.raw[e] = v[e];
+        } else {
+            const uint64_t v = load8_a8(a.w + (record + b * kRecord));
+            o.raw[0] = static_cast<uint32_t>(v);
+            o.raw[1] = static_cast<uint32_t>(v >> 32);
+        }
+        o.scale = load2_a2(scales + (first + b) * 2u);
+    };
+    u32x4 staged[kLoads];
+    auto load_parts = [&](int r) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int c = min(tid + kThreads * j, kPieces - 1), b = min(W * r + c / 384, blocks - 1);
+            staged[j] = *(const SATORI_GLOBAL u32x4*)(parts + b * stride + 16 * (c % 384));
+        }
+    };
+    auto store_parts = [&](int r) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j)
+            if (tid + kThreads * j < kPieces)
+                *reinterpret_cast<u32x4*>(lds + (r & 1) * kRoundBytes + 16 * (tid + kThreads * j)) = staged[j];
+    };
+
+    float acc[16] = {};
+    Weights w[2];
+    load_parts(0);
+    load_weights(0, w[0]);
+    load_weights(1, w[1]);
+    store_parts(0);
+    load_parts(1);
+    __syncthreads();  // round 0 staged
+    for (int r0 = 0; r0 < rounds; r0 += 2)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int r = r0 + n;
+            if (r >= rounds) break;
+            const uint8_t* mine = lds + n * kRoundBytes + way * kBlockTileBytes + 16 * lane;
+            if (W * r + way < blocks) {
+                float scale = half_bits_to_float(w[n].scale);
+                if (FORMAT == kQ4_0) scale *= 0.0625f;  // (codes 16 q)
+                f32x16 d = {};
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {
+                    u32x4 codes;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) codes[k] = code_pair<FORMAT>(w[n].raw, 4 * st + k);
+#pragma unroll
+                    for (int s = 0; s < 3; ++s)
+                        d = mfma_bf16(*reinterpret_cast<const bf16x8*>(mine + (2 * s + st) * kPartBytes),
+                                      __builtin_bit_cast(bf16x8, codes), d);
+                }
+                load_weights(r + 2, w[n]);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[i] = __builtin_fmaf(scale, d[i], acc[i]);
+            }
+            if (r + 1 < rounds) {
+                store_parts(r + 1);
+                load_parts(r + 2);
+            }
+            __syncthreads();  // round r + 1 staged, round r's buffer read
+        }
+    if constexpr (W > 1) {
+        f32x4* sums = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (way > 0)
+                sums[(((way - 1) * 4 + rt) * 4 + q) * 64 + lane] = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        __syncthreads();
+        if (way > 0) return;
+#pragma unroll
+        for (int n = 1; n < W; ++n)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 v = sums[(((n - 1) * 4 + rt) * 4 + q) * 64 + lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[4 * q + e] = __fadd_rn(acc[4 * q + e], v[e]);
+            }
+    }
+    if (row >= a.rows) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int p = t * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (p < a.positions) store_f32(a.y + static_cast<int64_t>(p) * a.rows + row, __builtin_amdgcn_ldexpf(acc[i], -kLiftExponent));
+    }
+}
+
+// The flagged positions of fbatch_tiles_kernel's product, over what it stored there: every workgroup looks at all flags and,
+// where there are any, computes its share of the 32 x 32 tiles that hold some.
+template <int FORMAT>
+__global__ __launch_bounds__(kThreads) void fbatch_flagged_kernel(FbatchArgs a) {
+    __shared__ uint32_t flagged[8];  // (256 positions at most)
+    __shared__ __align__(16) float lds[4 * 32 * kFlaggedStride];
+    if (threadIdx.x < 8) flagged[threadIdx.x] = 0u;
+    __syncthreads();
+    bool any = false;
+    for (int i = threadIdx.x; i < 2 * a.blocks * a.tiles; i += kThreads) {
+        const uint32_t word = a.flags[i];
+        if (word) atomicOr(&flagged[(i >> 1) % a.tiles], word);
+        any |= word != 0u;
+    }
+    if (!__syncthreads_or(any)) return;
+    const int row_tiles = (a.rows + kTile - 1) / kTile;
+    for (int u = blockIdx.x; u < row_tiles * a.tiles; u += gridDim.x) {
+        const int t = u % a.tiles;
+        if (flagged[t]) finish_flagged<FORMAT, 1>(a, u / a.tiles * kTile, t * kTile, flagged[t], lds);
+    }
+}
+
 // One workgroup per 32 x 32 tile of every (row group, position unit) tile: adds the pieces of a cut tile and computes
 // the flagged positions of any tile. Thread (g, wave q, lane) adds pieces g, g + G, ... of outputs 4q .. 4q + 3 of its
 // lane, four chains at a time, then the chains and the G sums in a fixed order: with many pieces (a few rows of many
@@ -676,11 +818,20 @@ __global__ __launch_bounds__(kThreads * G, 4) void fbatch_fixup_kernel(FbatchArg
 // How a launch is cut, for the device's CU count.
 struct FbatchPlan {
     int TP, RH, ways;
-    bool fused;
+    bool fused, whole;  // whole: fbatch_tiles_kernel
     int tiles, units, rounds, total, workgroups;
     size_t parts;                                                           // bytes of the split activations
     size_t slot_flags_offset, tile_flags_offset, flags_offset, scratch;     // (the partial sums first)
 };
+
+// Short rows under many outputs go to fbatch_tiles_kernel: it needs a workgroup for half of the CUs at least, and past 36
+// blocks an even deal and more rows a workgroup are worth more. Measured over 60 shapes at 14 counts of 33 to 256 positions
+// (us, fbatch_kernel against this): 13771 x 288 at 224 29.7 and 16.3, 9132 x 160 at 256 21.5 and 13.2, 7429 x 1120 at 128
+// Q4_0 24.7 and 20.9, 3798 x 576 at 256 20.7 and 15.0, but 7227 x 1760 at 64 23.2 and 24.8, 1772 x 8000 at 64 22 and 90,
+// 372 x 192 at 110 8.2 and 9.6.
+bool whole_tiles(int rows, int blocks, int tiles) {
+    return tiles > 1 && blocks <= 36 && static_cast<int64_t>((rows + 127) / 128) * tiles >= 128;
+}
 
 FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
     FbatchPlan p{};
@@ -691,12 +842,29 @@ FbatchPlan fbatch_plan(int rows, int columns, int positions, int cus) {
     // 19.6 against 22.5, 4096 x 4096 at 132 36.0 against 37.2, 11008 x 1024 at 256 40.7 against 36.4. One position tile a
     // unit (the weights read and converted once per tile, but twice the units to spread) for small products, and longer
     // where two a unit would leave half a unit empty: 512 x 512 at 256 9.1 against 10.7, 608 x 9024 at 64 15.9 against
-    // 19.5, 2572 x 576 at 256 16.2 against 19.4, 4096 x 4096 at 64 19.2 against 18.9, 4580 x 1120 at 256 28.2 against 25.9.
+    // 19.5, 2572 x 576 at 256 16.2 against 19.4, 4096 x 4096 at 64 19.2 against 18.9, 4580 x 1120 at 256 28.2 against 25.9,
+    // 9880 x 1984 at 82 29.1 against 31.8.
     const int64_t products = static_cast<int64_t>(rows) * columns * positions;
-    p.TP = products < 400000000 || (p.tiles % 2 == 1 && products < 1400000000) || p.tiles == 1 ? 1 : 2;
+    p.TP = products < 400000000 || (p.tiles % 2 == 1 && products < 1800000000) || p.tiles == 1 ? 1 : 2;
     p.fused = p.tiles <= 2 || products < 2300000000;
     p.RH = p.fused ? 2 : 4;
     p.ways = 8 / p.RH;
+    if (whole_tiles(rows, blocks, p.tiles)) {
+        const int64_t n = static_cast<int64_t>((rows + 127) / 128) * p.tiles;
+        p.whole = true;
+        p.fused = false;
+        p.TP = 1;
+        p.RH = 2;
+        // As many ways as keep every workgroup on the chip at once (two of 16 waves a CU, four of eight or eight of four).
+        p.ways = n <= 2 * cus ? 4 : n <= 4 * cus ? 2 : 1;
+        p.units = p.tiles;
+        p.rounds = (blocks + p.ways - 1) / p.ways;
+        p.total = static_cast<int>(n);
+        p.parts = static_cast<size_t>(blocks) * p.tiles * kBlockTileBytes;
+        p.workgroups = static_cast<int>(std::min<int64_t>(cus, 4 * n));  // of fbatch_flagged_kernel
+        p.scratch = static_cast<size_t>(blocks) * p.tiles * 8;           // (flags_offset 0)
+        return p;
+    }
     p.units = (p.tiles + p.TP - 1) / p.TP;
     p.tiles = p.units * p.TP;  // whole units: the packed form's last tile may be all zero
     p.rounds = (blocks + p.ways - 1) / p.ways;
@@ -745,7 +913,18 @@ hipError_t launch_format(FbatchArgs a, const FbatchPlan& p, uint8_t* parts, uint
     if (e != hipSuccess) return e;
     a.parts = parts;
     a.flags = flags;
-    return launch_product<FORMAT, 2, false, 4, 2>(a, stream);
+    if (!p.whole) return launch_product<FORMAT, 2, false, 4, 2>(a, stream);
+    const unsigned grid = (static_cast<unsigned>(a.total) + 7) / 8 * 8;
+    if (p.ways == 4)
+        fbatch_tiles_kernel<FORMAT, 4><<<grid, 1024, 0, stream>>>(a);
+    else if (p.ways == 2)
+        fbatch_tiles_kernel<FORMAT, 2><<<grid, 512, 0, stream>>>(a);
+    else
+        fbatch_tiles_kernel<FORMAT, 1><<<grid, 256, 0, stream>>>(a);
+    const hipError_t launched = hipGetLastError();
+    if (launched != hipSuccess) return launched;
+    fbatch_flagged_kernel<FORMAT><<<static_cast<unsigned>(a.workgroups), kThreads, 0, stream>>>(a);
+    return hipGetLastError();
 }
 
 }  // namespace

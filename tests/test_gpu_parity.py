@@ -993,14 +993,17 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
 @pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
 @pytest.mark.parametrize("rows,columns,positions", [(1, 64, 32), (63, 32, 40), (129, 96, 65), (257, 4128, 129),
                                                     (8200, 2080, 6), (513, 9056, 17), (4097, 4128, 31),
-                                                    (9001, 1056, 255), (4097, 2080, 66), (3000, 4128, 120)])
+                                                    (9001, 1056, 255), (4097, 2080, 66), (3000, 4128, 120),
+                                                    (1537, 9056, 250), (9001, 1184, 255), (2100, 1120, 250),
+                                                    (9001, 288, 255), (18001, 96, 256)])
 def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
     # The edges of the matrix-core batch: row groups of 128 (up to 64 positions) and 256 rows with one row more
     # or less, odd block counts, rounds past the last block, tiles cut into many partial sums, and counts below 32
     # on matrices large enough for it. The first and last positions hold an activation from which a tile is computed once
     # more from activations as they are (2^40), and one just below it; the bound is that of
-    # test_legacy_matrix_core_batch, on the FP64 product. The last three: packed activations, and the form of one and
-    # of two position tiles a unit past 64 positions.
+    # test_legacy_matrix_core_batch, on the FP64 product. By the plan: packed activations of (9001, 1184) and, in
+    # tiles of many pieces, (1537, 9056); one and two position tiles a unit past 64 positions, (4097, 2080) and (3000, 4128);
+    # whole tiles of short rows in four, two and one ways, (2100, 1120), (9001, 288 and 1056) and (18001, 96).
     g = rng(515 + rows + columns + positions)
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
@@ -1045,7 +1048,8 @@ def _large_positions(g, positions, columns):
 
 @pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
 @pytest.mark.parametrize("rows,columns,positions", [(70, 96, 33), (257, 4128, 40), (33, 9056, 64), (8200, 2080, 6),
-                                                    (1000, 2080, 130), (4097, 4128, 200), (1537, 9056, 250)])
+                                                    (1000, 2080, 130), (4097, 4128, 200), (1537, 9056, 250),
+                                                    (5001, 1120, 130), (9001, 96, 250), (20001, 64, 256)])
 def test_legacy_batches_of_large_activations(context, fmt, rows, columns, positions):
     # Positions with an activation of 2^40 and more, all of a batch and among others, in every form of the matrix-core
     # batch (one and two position tiles a unit, packed activations, tiles in one piece, in a few and in many): each
@@ -1074,6 +1078,63 @@ def test_legacy_batches_of_large_activations(context, fmt, rows, columns, positi
         assert np.array_equal(np.isnan(y[p]), np.isnan(want)), f"position {p}: NaN"
         inf = np.isinf(want)
         assert np.array_equal(np.isinf(y[p]), inf) and np.array_equal(y[p][inf], want[inf]), f"position {p}: Inf"
+
+
+@pytest.mark.parametrize("rows,columns", [(5001, 1120), (9001, 1024), (1537, 9056), (4097, 4128)])
+def test_legacy_batch_buffer_serves_fewer_positions(context, rows, columns):
+    # What a matrix holds after 256 positions serves every smaller count, whatever form it takes: none is refused while a
+    # step holds the buffer, and the step's replay gives the bits of the eager call.
+    g = rng(31 + rows)
+    data = S.quantize_weights((g.standard_normal((rows, columns), dtype=np.float32) * 0.02), rows, columns, BQ.Q8_0)
+    x = g.standard_normal((256, columns), dtype=np.float32)
+    dx, dy = context.alloc(x.nbytes), context.alloc(4 * 256 * rows)
+    context.upload(dx, x)
+    with context.create(data, S.QuantizedMatrixShape(rows, columns, BQ.Q8_0)) as m:
+        m.execute_batch_device(dx, 256, dy)
+        want = context.download(np.zeros((256, rows), np.float32), dy)
+        context.capture_begin()
+        m.execute_batch_device(dx, 256, dy)
+        step = context.capture_end()
+        for positions in (32, 33, 65, 100, 128, 129, 161, 200, 225, 255):
+            context.upload(dy, np.full((256, rows), np.nan, np.float32))
+            m.execute_batch_device(dx, positions, dy)
+            got = context.download(np.zeros((256, rows), np.float32), dy)
+            bound = 1e-5 * (np.abs(x[positions - 1]).astype(np.float64).sum() * 0.1)  # |w| < 0.1
+            assert np.all(np.isfinite(got[:positions])) and np.all(np.isnan(got[positions:]))
+            assert np.all(np.abs(got[positions - 1] - want[positions - 1]) <= bound)
+            step.execute()
+            again = context.download(np.zeros((256, rows), np.float32), dy)
+            assert np.array_equal(again.view(np.uint32), want.view(np.uint32))
+        step.dispose()
+    context.free(dx)
+    context.free(dy)
+
+
+@pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
+def test_legacy_batch_of_short_rows_takes_no_longer_a_weight(context, fmt):
+    # 13771 x 288 over 224 positions: at most 1.9 times 6886 x 288 over 112, a quarter of the products (1.4 to 1.6 measured;
+    # 2.2 where one workgroup a CU waited for each short tile's loads).
+    g = rng(9)
+    times = []
+    for rows, positions in ((6886, 112), (13771, 224)):
+        data = S.quantize_weights((g.standard_normal((rows, 288), dtype=np.float32) * 0.02), rows, 288, fmt)
+        x = g.standard_normal((positions, 288), dtype=np.float32)
+        dx, dy = context.alloc(x.nbytes), context.alloc(4 * positions * rows)
+        context.upload(dx, x)
+        with context.create(data, S.QuantizedMatrixShape(rows, 288, fmt)) as m:
+            m.execute_batch_device(dx, positions, dy)
+            best = []
+            for _ in range(10):
+                context.synchronize()
+                start = time.perf_counter()
+                for _ in range(50):
+                    m.execute_batch_device(dx, positions, dy)
+                context.synchronize()
+                best.append(time.perf_counter() - start)
+            times.append(min(best))
+        context.free(dx)
+        context.free(dy)
+    assert times[1] <= 1.9 * times[0]
 
 
 @pytest.mark.parametrize("fmt,rows,columns,positions", [(BQ.Q8_0, 4096, 4096, 256), (BQ.Q8_0, 1536, 8960, 64),
