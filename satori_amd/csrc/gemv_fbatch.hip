@@ -930,12 +930,17 @@ hipError_t launch_format(FbatchArgs a, const FbatchPlan& p, uint8_t* parts, uint
 }  // namespace
 
 // From 32 positions on always; below, where the weights the single-position kernel would read again outweigh the second
-// launch. Measured against that kernel (us, FP32 activations): 4096 x 4096 Q8_0 14 at any count to 32, against 10 at 2
-// positions, 16 at 4, 29 at 12; 11008 x 4096 Q4_0 23 against 16 at 2, 24 at 4, 39 at 8; 1135 x 3808 Q4_0 11 against
-// 9.4 at 8, 15 at 16; 4096 x 1024 Q4_0 10 against 8.4 at 16, 13 at 31; 512 x 1024 8.5 against 3.8 at 31.
-bool fbatch_pays(int rows, int columns, int positions) {
+// launch and, a row, its share of the partial sums; Q4_0, whose weights are half as many bytes, from 1.1 of that. Measured
+// against that kernel over 90 shapes at 11 counts of 4 to 31 positions (us, FP32 activations, this against that kernel):
+// Q8_0 4096 x 4096 14.2 and 10.4 at 4, 14.0 and 26.1 at 12; 8175 x 2176 16.0 and 12.6 at 6, 16.3 and 18.2 at 12; 10460 x
+// 736 13.2 and 9.8 at 12; 4096 x 1024 10.4 and 9.1 at 20; Q4_0 11008 x 4096 22.5 and 21.5 at 4, 22.6 and 36.6 at 8; 1135 x
+// 3808 11.6 and 8.5 at 8, 11.7 and 12.3 at 16. At 11 of those 1,980 calls the rule takes this product where the other
+// kernel is more than 3% faster.
+bool fbatch_pays(int format, int rows, int columns, int positions) {
     if (positions >= kTile) return true;
-    return positions >= 4 && static_cast<int64_t>(rows) * columns * (positions - 1) >= 72000000;
+    const int64_t line = 60000000 + 4000 * static_cast<int64_t>(rows);
+    return positions >= 4 &&
+           static_cast<int64_t>(rows) * columns * (positions - 1) >= (format == kQ4_0 ? line + line / 10 : line);
 }
 
 // What a matrix holds for its batches: the split activations of any count of as many position tiles, and 256 bytes a tile

@@ -220,7 +220,7 @@ size_t kmfma_workspace_bytes(int blocks, int positions);
 // is used for. `parts` (fbatch_held_bytes; may be null below 32 positions) takes the split activations of large
 // products. `scratch` (fbatch_scratch_bytes) takes partial sums, which mean nothing once the call's launches are done,
 // so launches of any matrices that run in order can share it. Both sizes are for the current device.
-bool fbatch_pays(int rows, int columns, int positions);
+bool fbatch_pays(int format, int rows, int columns, int positions);
 size_t fbatch_held_bytes(int rows, int columns, int positions);
 size_t fbatch_scratch_bytes(int rows, int columns, int positions);
 hipError_t launch_gemv_fbatch(const uint8_t* w, int format, const float* x, uint8_t* parts, uint8_t* scratch, float* y,

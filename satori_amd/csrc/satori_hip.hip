@@ -333,7 +333,7 @@ uint8_t* batch_scratch(satori_hip_matrix* m, int positions, hipStream_t stream) 
 // Q4_0 over as many positions as fbatch_pays says run on the matrix cores, 256 positions at a time.
 void enqueue_float(satori_hip_matrix* m, const float* x, int positions, float* y, hipStream_t stream) {
     const Shape& s = m->shape;
-    if ((s.format == SATORI_HIP_Q8_0 || s.format == SATORI_HIP_Q4_0) && fbatch_pays(s.rows, s.columns, positions)) {
+    if ((s.format == SATORI_HIP_Q8_0 || s.format == SATORI_HIP_Q4_0) && fbatch_pays(s.format, s.rows, s.columns, positions)) {
         constexpr int kChunk = 256;
         void* parts = nullptr;
         if (positions >= 32)

@@ -399,7 +399,7 @@ def test_short_batches_while_another_stream_is_captured():
     foreign, graph = ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamCreateWithFlags(ctypes.byref(foreign), 1) == 0
     calls = []
-    for fmt, rows, columns, positions in ((BQ.Q4_K, 4111, 4096, 9), (BQ.Q8_0, 8200, 2080, 6)):
+    for fmt, rows, columns, positions in ((BQ.Q4_K, 4111, 4096, 9), (BQ.Q8_0, 4100, 6176, 6)):
         data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
         x = g.standard_normal((positions, columns)).astype(np.float32)
         dx, dy = ctx.alloc(x.nbytes), ctx.alloc(4 * positions * rows)

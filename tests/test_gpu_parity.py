@@ -992,7 +992,7 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
 
 @pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
 @pytest.mark.parametrize("rows,columns,positions", [(1, 64, 32), (63, 32, 40), (129, 96, 65), (257, 4128, 129),
-                                                    (8200, 2080, 6), (513, 9056, 17), (4097, 4128, 31),
+                                                    (4100, 6176, 6), (513, 9056, 17), (4097, 4128, 31),
                                                     (9001, 1056, 255), (4097, 2080, 66), (3000, 4128, 120),
                                                     (1537, 9056, 250), (9001, 1184, 255), (2100, 1120, 250),
                                                     (9001, 288, 255), (18001, 96, 256)])
@@ -1047,7 +1047,7 @@ def _large_positions(g, positions, columns):
 
 
 @pytest.mark.parametrize("fmt", [BQ.Q8_0, BQ.Q4_0])
-@pytest.mark.parametrize("rows,columns,positions", [(70, 96, 33), (257, 4128, 40), (33, 9056, 64), (8200, 2080, 6),
+@pytest.mark.parametrize("rows,columns,positions", [(70, 96, 33), (257, 4128, 40), (33, 9056, 64), (4100, 6176, 6),
                                                     (1000, 2080, 130), (4097, 4128, 200), (1537, 9056, 250),
                                                     (5001, 1120, 130), (9001, 96, 250), (20001, 64, 256)])
 def test_legacy_batches_of_large_activations(context, fmt, rows, columns, positions):
@@ -1388,7 +1388,7 @@ def test_k_batch_kernel_choice(context, fmt, rows, blocks, positions):
 def test_legacy_batch_captured_before_it_ran(context):
     # A batch of fewer than 32 positions that uses a workspace can be captured before it ran (the workspace is then the
     # step's), replays within the FP32 bound, and the same matrix then runs eagerly.
-    rows, columns, positions = 8200, 2080, 6
+    rows, columns, positions = 4100, 6176, 6
     g = rng(99)
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, BQ.Q8_0)
@@ -1418,7 +1418,7 @@ def test_legacy_batch_captured_before_it_ran(context):
     context.free(dy)
 
 
-@pytest.mark.parametrize("fmt,rows,columns,positions", [(BQ.Q8_0, 8200, 2080, 6), (BQ.Q4_0, 4097, 4128, 31)])
+@pytest.mark.parametrize("fmt,rows,columns,positions", [(BQ.Q8_0, 4100, 6176, 6), (BQ.Q4_0, 4097, 4128, 31)])
 def test_legacy_short_batch_replays_its_eager_bits(context, fmt, rows, columns, positions):
     # Captured before or after it ran, in one step or two of the same matrix, a batch of fewer than 32 positions on the
     # matrix cores gives the bits of the eager call.
