@@ -144,14 +144,14 @@ def test_legacy_batch_nonfinite_inputs_propagate(context, fmt):
 
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
-@pytest.mark.parametrize("positions", [1, 3, 20])
-def test_k_batch_nonfinite_inputs_match_the_reference_bits(context, fmt, positions):
+@pytest.mark.parametrize("rows,positions", [(200, 1), (200, 3), (200, 20), (6000, 20), (6000, 200)])
+def test_k_batch_nonfinite_inputs_match_the_reference_bits(context, fmt, rows, positions):
     # Q8KCodec.QuantizeBlock with infinities and NaNs (Q8KCodec.cs:44-76): NaN never wins the maximum, an
     # all-NaN-or-zero block quantizes to zero and is skipped, an infinite maximum gives inverse -0, codes 0
-    # and scale -Inf, whose block term is NaN. The integer kernel (1-15 positions) and the matrix-core
-    # kernel (16+) both follow it.
+    # and scale -Inf, whose block term is NaN. The integer kernels (200 rows) and the matrix-core
+    # products (6000) all follow it.
     g = rng(77 + 10 * int(fmt) + positions)
-    rows, columns = 200, 2048
+    columns = 2048
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
     x = g.standard_normal((positions, columns)).astype(np.float32)
@@ -184,10 +184,11 @@ def test_k_batch_nonfinite_inputs_match_the_reference_bits(context, fmt, positio
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
 @pytest.mark.parametrize("rows,columns,positions", [(300, 29696, 1), (300, 29696, 3), (130, 29696, 16),
-                                                    (70, 65536, 1), (33, 57344, 2)])
+                                                    (70, 65536, 1), (33, 57344, 2), (1030, 29696, 16)])
 def test_k_batch_wide_rows_are_bit_exact(context, fmt, rows, columns, positions):
     # Rows wider than one staging of the Q8_K row (112 blocks = 28,672 columns) are summed chunk by chunk in
-    # block order; 29,696 (116 blocks), 57,344 (two whole chunks) and 65,536 (256 blocks, a ragged last chunk).
+    # block order; 29,696 (116 blocks), 57,344 (two whole chunks) and 65,536 (256 blocks, a ragged last chunk); 16
+    # positions of 1030 rows on the matrix cores.
     g = rng(5150 + columns + rows + int(fmt))
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
@@ -399,7 +400,7 @@ def test_short_batches_while_another_stream_is_captured():
     foreign, graph = ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamCreateWithFlags(ctypes.byref(foreign), 1) == 0
     calls = []
-    for fmt, rows, columns, positions in ((BQ.Q4_K, 4111, 4096, 9), (BQ.Q8_0, 4100, 6176, 6)):
+    for fmt, rows, columns, positions in ((BQ.Q4_K, 4111, 4096, 14), (BQ.Q8_0, 4100, 6176, 6)):
         data = S.quantize_weights((g.standard_normal((rows, columns)) * 0.02).astype(np.float32), rows, columns, fmt)
         x = g.standard_normal((positions, columns)).astype(np.float32)
         dx, dy = ctx.alloc(x.nbytes), ctx.alloc(4 * positions * rows)

@@ -579,13 +579,15 @@ def test_k_integer_batch_is_bit_exact(context, fmt, rows, columns):
 
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
-def test_k_integer_product_quantizer_edge_cases(context, fmt):
+@pytest.mark.parametrize("rows,repeat", [(70, 4), (4200, 4), (4200, 50)])
+def test_k_integer_product_quantizer_edge_cases(context, fmt, rows, repeat):
     # Q8KCodec.QuantizeBlock (Q8KCodec.cs:44-76) inside the integer products: ties of the largest magnitude
     # (the lowest index wins, and its sign sets the scale), the maximum in every lane position of a block,
-    # subnormal and huge blocks, zero blocks; outputs bit-exact against the oracle, for the single-position
-    # kernel (which quantizes in-kernel) and the matrix-core batch (which quantizes in its pack kernel).
+    # subnormal and huge blocks, zero blocks; outputs bit-exact against the oracle, for the single-position kernel and
+    # batches: 20 positions of 70 rows quantize in the integer kernel, 20 and 250 of 4200 in the matrix cores' pack kernel
+    # (the product without staging, and the staged one).
     g = rng(4711)
-    rows, columns = 70, 4096
+    columns = 4096
     w = (g.standard_normal((rows, columns)) * 0.05).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
     cases = []
@@ -610,16 +612,19 @@ def test_k_integer_product_quantizer_edge_cases(context, fmt):
     x[1024:1280] = 0.0
     cases.append(x)
     m = context.create(data, S.QuantizedMatrixShape(rows, columns, fmt))
+    want = []
     for i, x in enumerate(cases):
         y = np.zeros(rows, np.float32)
         m.execute_batch(x, 1, y)
-        expected = O.qk_matvec_quantized_avx2(data, rows, columns, int(fmt), O.q8k_quantize_row(x))
-        assert np.array_equal(y.view(np.uint32), expected.view(np.uint32)), f"case {i}"
-    xs = np.stack(cases * 4).astype(np.float32)  # 20 positions: the matrix-core path
-    y = np.zeros(xs.shape[0] * rows, np.float32)
-    m.execute_batch(xs.reshape(-1), xs.shape[0], y)
-    expected = O.q_matvec_batch(data, rows, columns, int(fmt), xs.reshape(-1), xs.shape[0])
-    assert np.array_equal(y.view(np.uint32), expected.view(np.uint32))
+        want.append(O.qk_matvec_quantized_avx2(data, rows, columns, int(fmt), O.q8k_quantize_row(x)))
+        assert np.array_equal(y.view(np.uint32), want[i].view(np.uint32)), f"case {i}"
+    xs = np.stack(cases * repeat).astype(np.float32)
+    y = np.zeros((xs.shape[0], rows), np.float32)
+    m.execute_batch(xs.reshape(-1), xs.shape[0], y.reshape(-1))
+    for i in range(xs.shape[0]):
+        assert np.array_equal(y[i].view(np.uint32), want[i % len(cases)].view(np.uint32)), f"position {i}"
+    assert np.array_equal(O.q_matvec_batch(data, rows, columns, int(fmt), xs[:5].reshape(-1), 5).view(np.uint32),
+                          y[:5].reshape(-1).view(np.uint32))
     m.dispose()
 
 
@@ -642,11 +647,12 @@ def test_k_integer_batch_multi_position_on_fixture_blocks(context, fmt, fixture)
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
 @pytest.mark.parametrize("rows,columns,positions", [(17, 512, 16), (129, 768, 37), (300, 1536, 64),
-                                                    (1536, 1536, 100), (8960, 1536, 256), (256, 8960, 65)])
+                                                    (1536, 1536, 100), (8960, 1536, 256), (256, 8960, 65),
+                                                    (9000, 2048, 17)])
 def test_k_matrix_core_batch_equals_per_position(context, fmt, rows, columns, positions):
-    # BatchedMatVecTests.cs:45-113: a batch equals its positions run one at a time. Sixteen positions and
-    # more take the matrix-core kernel, one position the single-position integer kernel (bit-exact against
-    # the oracle above), so the two must agree bit for bit. Ragged row and position counts, a zero
+    # BatchedMatVecTests.cs:45-113: a batch equals its positions run one at a time. The last four take the matrix
+    # cores, the small ones the integer kernels, one position the single-position integer kernel (bit-exact against
+    # the oracle above), so all must agree bit for bit. Ragged row and position counts, a zero
     # position, a zero block inside a position and a position of large magnitude are included.
     g = rng(7 + rows + columns + positions)
     w = (g.standard_normal((rows, columns), dtype=np.float32) * 0.02).astype(np.float32)
@@ -688,11 +694,13 @@ def _q6k_extreme_blocks(g, rows: int, blocks: int) -> np.ndarray:
     return np.ascontiguousarray(out.reshape(-1))
 
 
-@pytest.mark.parametrize("rows,columns,positions", [(70, 1536, 33), (33, 8960, 64)])
+@pytest.mark.parametrize("rows,columns,positions", [(70, 1536, 33), (33, 8960, 64), (3001, 1536, 33), (1030, 8960, 64),
+                                                    (9001, 1536, 64)])
 def test_k_matrix_core_q6k_extreme_products(context, rows, columns, positions):
     # The Q6_K matrix-core product reads pre-scaled weight planes: its extremes (the largest |sc * (q - 32)|
-    # against activation codes of +-127, |Dot| near 2^27) must give the reference's outputs bit for bit, as
-    # must the single-position kernel on the resident layout.
+    # against activation codes of +-127, |Dot| near 2^27) must give the reference's outputs bit for bit, in the product
+    # without staging (3001 and 1030 rows) and the staged one (9001), as must the integer kernels on the resident layout
+    # (one position; 70 and 33 rows).
     g = rng(31337 + rows + columns)
     data = _q6k_extreme_blocks(g, rows, columns // 256)
     x = g.standard_normal((positions, columns), dtype=np.float32)
@@ -805,7 +813,7 @@ def test_randomized_shapes_sweep(context):
     # A seeded sweep over every MatVec path and random shapes (rows 1-3000, so rows end inside panels and
     # tiles; ragged Ternary2 columns; odd block counts; long and short rows): the FP32 paths within the
     # 1e-5 * sum|w*x| gate of the oracle's scalar restatement of ExecuteScalarCore / ExecuteScalar, the
-    # integer K path (1-15 positions: in-kernel quantization; 16 and more: the matrix-core product) equal to
+    # integer K path (any of its kernels) equal to
     # the oracle's ExecuteQuantizedTiled bit for bit.
     g = rng(20261201)
     for case in range(45):
@@ -1191,10 +1199,12 @@ def _q8k_special_row(columns):
 
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
-@pytest.mark.parametrize("rows,positions", [(40, 1), (3000, 3), (3001, 11), (64, 17)])
+@pytest.mark.parametrize("rows,positions", [(40, 1), (3000, 3), (3001, 11), (64, 17), (8001, 11), (6001, 17), (9001, 40),
+                                            (9001, 100)])
 def test_k_quantizer_special_blocks_in_every_product(context, fmt, rows, positions):
-    # The activation quantizer inside the single-position, few-position and matrix-core integer products, on rows whose
-    # blocks take its special cases, against the oracle's quantizer and integer product, bit for bit; one block at a
+    # The activation quantizer inside the single-position and few-position integer products (3001 rows and fewer) and in
+    # the matrix cores' pack kernel (from 6001 on; Q6_K from 16 positions; its product without staging at 17 positions, Q4_K's
+    # to 40, the staged one beyond), on rows whose blocks take its special cases, against the oracle's quantizer and integer product, bit for bit; one block at a
     # time (the others plain), so that a NaN or infinity of one does not hide another.
     columns = 12 * 256
     special = _q8k_special_row(columns)
@@ -1331,10 +1341,10 @@ def test_k_batch_time_has_no_step(context, rows, columns, few, more, limit):
 
 
 @pytest.mark.parametrize("fmt,rows,blocks,positions", [
-    (BQ.Q4_K, 4111, 16, 9), (BQ.Q4_K, 4111, 16, 7),     # either side of the line below 16 positions
-    (BQ.Q4_K, 1300, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
-    (BQ.Q4_K, 33, 3, 40), (BQ.Q4_K, 33, 1, 256),        # small products from 16 positions on
-    (BQ.Q6_K, 3001, 6, 16), (BQ.Q6_K, 1300, 4, 50), (BQ.Q6_K, 200, 9, 40)])
+    (BQ.Q4_K, 4111, 16, 14), (BQ.Q4_K, 4111, 16, 7),    # either side of the line below 16 positions
+    (BQ.Q4_K, 4000, 5, 31), (BQ.Q4_K, 1000, 7, 65),      # rounds, rows and positions with a remainder
+    (BQ.Q4_K, 33, 3, 40), (BQ.Q4_K, 33, 1, 256),        # small products from 16 positions on: integer
+    (BQ.Q6_K, 5001, 6, 16), (BQ.Q6_K, 1300, 4, 50), (BQ.Q6_K, 200, 9, 40)])
 def test_k_batch_kernel_choice(context, fmt, rows, blocks, positions):
     # The matrix-core product of few tiles and the integer kernels, each where the other ran before: the bits of
     # single-position products, from a matrix and from a group of two. Captured before it ran, a call of fewer than 16
@@ -1516,13 +1526,15 @@ def test_legacy_tiny_activations_within_reference_floor(context, fmt, mixed):
 
 
 @pytest.mark.parametrize("fmt", [BQ.Q4_K, BQ.Q6_K])
-def test_k_tiny_activations_float_and_integer_paths(context, fmt):
+@pytest.mark.parametrize("rows", [256, 3001])
+def test_k_tiny_activations_float_and_integer_paths(context, fmt, rows):
     # The K formats with the same tiny positions: the FP32-activation MatVec (IQuantizedMatrix.Execute,
     # QuantizedMatVec.ExecuteScalar's DotBlock, QuantizedMatVec.cs:56-65) within 1e-5 * sum|w x| + n *
     # float.Epsilon of the scalar reference, and the Q8_K integer path (ExecuteBatch) bit-identical to the
-    # reference's ExecuteQuantizedTiled composition, at one position and as a 40-position matrix-core batch.
+    # reference's ExecuteQuantizedTiled composition, at one position and as a batch of 40 (256 rows: the integer kernels;
+    # 3001: the matrix cores).
     g = rng(5151 + int(fmt))
-    rows, columns, positions = 256, 1536, 40
+    columns, positions = 1536, 40
     w = (g.standard_normal((rows, columns)) * 0.02).astype(np.float32)
     data = S.quantize_weights(w, rows, columns, fmt)
     x, kinds = _tiny_positions(g, positions, columns, True)
@@ -1873,7 +1885,7 @@ def _gguf_with(tmp_path, tensors):
 def test_gguf_tensors_upload_to_resident_matrices(context, tmp_path):
     # GgufQuantizedMatrix.CreateExecution (GgufQuantizedMatrix.cs:31-36): the device matrix made from the
     # mapped tensor equals the one made from the same bytes through the factory, for every format, on the
-    # FP32 path and on the integer K path (single position and the matrix-core batch).
+    # FP32 path and on the integer K path (a single position and a batch).
     g = rng(99)
     specs = [("blk.0.attn_q.weight", 300, 512, BQ.Q4_K, 12), ("blk.0.ffn_down.weight", 129, 768, BQ.Q6_K, 14),
              ("blk.0.attn_k.weight", 70, 256, BQ.Q8_0, 8), ("blk.0.attn_v.weight", 33, 320, BQ.Q4_0, 2)]
