@@ -813,7 +813,7 @@ hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_membe
     const int per = (s.positions + slices - 1) / slices;
     int64_t rows = 0;
     for (int i = 0; i < count; ++i) rows += members[i].rows;
-    int64_t tile = std::max<int64_t>(4, (rows * slices + 255) / 256);
+    int64_t tile = std::max<int64_t>(4, (rows * slices + kCus - 1) / kCus);
     // No more than one workgroup per CU where the rounding of each slice's and member's last tile made a few more: they
     // run in a second round (297 x 2816 Q6_K over 48 positions, 258 workgroups: 16.0 us; 40 positions 9.5).
     auto workgroups = [&](int64_t t) {
@@ -821,7 +821,7 @@ hipError_t launch_kint_multi(const MatDesc* members, const MatDesc* device_membe
         for (int i = 0; i < count; ++i) n += (members[i].rows + t - 1) / t;
         return n * slices;
     };
-    while (tile < kMultiRows && workgroups(tile) > 256) ++tile;
+    while (tile < kMultiRows && workgroups(tile) > kCus) ++tile;
     s.rows_per_wg = static_cast<int>(std::min<int64_t>(tile, kMultiRows));
     // (Up to three dwords a position round its activations up to 16 bytes.)
     const int per_block = per * (kActDwords + s.rows_per_wg) * static_cast<int>(sizeof(uint32_t));

@@ -332,7 +332,7 @@ __device__ __forceinline__ void block_terms(PlaneRegs& r, const uint8_t* next, c
     }
 }
 
-// Blocks of one row tile are split over S waves ("ways"): way w computes blocks w, w + S, ... and, per round
+// Blocks of one row tile are split over S waves ("ways"), one or two of them (four: kmfma_ways_kernel): way w computes blocks w, w + S, ... and, per round
 // of S blocks, hands its 16 terms per lane to the others through LDS; the wave that owns an output adds the
 // round's S terms in block order, so every (row, position) sum is formed exactly as the sequential one.
 // A workgroup holds R = 4 / S row tiles x S ways of one position tile; the S blocks of a round are staged
@@ -340,6 +340,7 @@ __device__ __forceinline__ void block_terms(PlaneRegs& r, const uint8_t* next, c
 // the scales) into registers while the current round is computed, and writes them to LDS after it.
 template <int S>
 struct Split {
+    static_assert(S == 1 || S == 2);
     static constexpr int R = 4 / S;
     static constexpr int kOwned = 16 / S;  // outputs per lane each way adds up (whole quads)
 };
@@ -487,7 +488,7 @@ __global__ __launch_bounds__(256, S == 1 ? 3 : 2) void kmfma_kernel(KmfmaArgs a)
         if (k < rounds) round(k, ra, rb);
     } else {
         // The row tile's plane records (a tile past the last computes on the last one and stores nothing).
-        // With two ways (two waves per SIMD, 256 VGPRs; launch_format caps the planes at two) two plane register
+        // With two ways (two waves per SIMD, 256 VGPRs) two plane register
         // sets alternate: round k (this way's block k S + way) reads set k mod 2 and refills it with block
         // (k + 2) S + way while it runs, so each block's planes are requested two rounds ahead, after the next
         // round's codes (a wait for those leaves the planes in flight). One way (three workgroups per CU) keeps
@@ -774,15 +775,15 @@ void launch_format(KmfmaArgs& a, hipStream_t stream) {
     long wave_tiles = 0;
     for (int i = 0; i < a.count; ++i) wave_tiles += static_cast<long>((a.m[i].rows + kTile - 1) / kTile) * a.tiles;
     // Four ways (the kernel without staging) while each tile has a CU; beyond, for Q4_K, while two workgroups a CU hold
-    // most of them and the rounds of four blocks are worth their exchange, else two ways. Measured (us, four against two
-    // ways): 512 tiles of 4096 x 4096 16.0 against 20.4, 658 of 3000 x 8960 37.7 against 42.5, 376 of 3000 x 1024 8.0
-    // against 8.3; 896 of 4096 x 4096 26.0 against 24.4, 785 of 5000 x 3072 20.1 against 18.6, 560 of 8960 x 1536 (six
-    // blocks: the second round half empty) 13.1 against 11.8, 846 of 9000 x 1024 11.4 against 9.9. The weight planes,
-    // whose bytes bound them from there on: 280 tiles of 8960 x 1536 12.1 against 11.0, 256 of 4096 x 4096 12.1 against
-    // 15.5.
+    // most of them and rounds of four blocks save at least two of the rounds of two (from seven blocks on: the exchange of
+    // a round among four ways costs more than among two). Measured over 168 calls, four ways' time over two's: 280 to 512
+    // tiles 0.72 to 0.80 at 20 blocks and more, 0.77 to 0.96 at 7 to 16 (0.91 to 0.96 at 9 and 10, whose last round is
+    // nearly empty), 0.97 to 1.01 at 4, 1.01 to 1.07 at 5 and 6; 560 to 688 tiles 0.83 to 1.05 from 7 blocks on, 1.08 to
+    // 1.12 at 5 and 6; 896 tiles of 4096 x 4096 26.0 us against 24.4, 785 of 5000 x 3072 20.1 against 18.6. The weight
+    // planes, whose bytes bound them from there on: 280 tiles 0.97 to 1.15, 256 of 4096 x 4096 12.1 us against 15.5.
     const int split = choose_split(wave_tiles, a.blocks);
-    const bool more = FORMAT == kQ4_K && ((a.blocks > 6 && wave_tiles <= 700) || (a.blocks == 4 && wave_tiles <= 512));
-    if (split == 4 && (wave_tiles <= 256 || more)) return launch_ways<FORMAT>(a, stream);
+    const bool more = FORMAT == kQ4_K && wave_tiles <= 700 && (a.blocks + 1) / 2 - (a.blocks + 3) / 4 >= 2;
+    if (split == 4 && (wave_tiles <= kCus || more)) return launch_ways<FORMAT>(a, stream);
     if (split == 1)
         launch_split<FORMAT, 1>(a, stream);
     else
@@ -808,7 +809,7 @@ bool kmfma_pays(int format, int64_t rows, int blocks, int positions) {
     int64_t line = std::min<int64_t>((positions > kTile ? 100000 : 200000) + 28000 * static_cast<int64_t>(blocks), 800000);
     if (format == kQ6_K) line = line * 4 / 5;
     if (positions > 48) line = std::min<int64_t>(line, 300000);
-    return rows * blocks * positions * 256 >= line * (256 + std::max<int64_t>(tiles - 256, 0) / 2);
+    return rows * blocks * positions * 256 >= line * (kCus + std::max<int64_t>(tiles - kCus, 0) / 2);
 }
 
 size_t kmfma_workspace_bytes(int blocks, int positions) {

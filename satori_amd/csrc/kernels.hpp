@@ -15,6 +15,8 @@ enum Format : int { kQ8_0 = 0, kQ4_0 = 1, kQ4_K = 2, kQ6_K = 3, kTernary2 = 16 }
 constexpr int kQ8KBlockBytes = 292;
 
 // One matrix of a launch. Row-major payload: row r starts at w + r * row_bytes.
+constexpr int kCus = 256;  // of an MI355X: what the measured lines between kernels are drawn for
+
 struct MatDesc {
     const uint8_t* w;   // weights (device; the payload, or its regrouped device layout)
     const float* x;     // FP32 activations [positions][columns]
