@@ -659,7 +659,8 @@ __global__ __launch_bounds__(THREADS) void attention_split_kernel(const float* _
     const double m = split_reduce<THREADS>(local_max, red, true);
     double part = 0;
     for (int t = t0 + threadIdx.x; t < t1; t += THREADS) {
-        const double e = exp(es[t - t0] - m);
+        const double score = es[t - t0];
+        const double e = score == -INFINITY ? 0.0 : exp(score - m);  // (a split of nothing else: 0, not NaN)
         es[t - t0] = e;
         part = part + e;
     }

@@ -655,6 +655,25 @@ def test_attention_decode_equals_inputs_then_attention(context, position, heads,
             context.free(p)
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,tokens", [(6, 6, 48, 300), (18, 2, 64, 257), (224, 32, 128, 96),
+                                                            (4, 1, 256, 2000)])
+def test_attention_split_of_scores_of_minus_infinity(context, heads, kv_heads, head_dim, tokens):
+    # A workgroup's tokens may all score -infinity where others do not (the general split form, at head widths, groups and
+    # counts that the shared one does not take): they weigh nothing. All tokens at -infinity give NaN, as in the reference.
+    g = rng(heads + tokens)
+    q = np.abs(g.standard_normal(heads * head_dim)).astype(np.float32)
+    k = (g.standard_normal((tokens, kv_heads * head_dim)) * 0.3).astype(np.float32)
+    v = g.standard_normal(k.shape).astype(np.float32)
+    out = np.zeros(q.size, np.float32)
+    k[:tokens - 7] = -np.inf
+    S.TransformerOps.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens, out, context)
+    _within_ulp(out, O.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens), "masked")
+    k[:] = -np.inf
+    S.TransformerOps.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens, out, context)
+    want = O.grouped_attention(q, k.ravel(), v.ravel(), heads, kv_heads, head_dim, tokens)
+    assert np.array_equal(np.isnan(out), np.isnan(want))
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,tokens", [
     (1, 1, 32, 33), (2, 1, 64, 63), (6, 2, 96, 64), (4, 1, 128, 65),   # the edges of one 32-token split
     (5, 1, 128, 97), (35, 5, 32, 255), (48, 8, 96, 257), (64, 8, 64, 300),  # 1 .. 8 query heads, divided and whole
