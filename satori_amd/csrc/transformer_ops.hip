@@ -1338,10 +1338,12 @@ namespace {
 // Splits of the shared form, or 0 where it does not apply: 32 tokens each (one pass of the workgroup: a token's key by
 // eight threads), at most 512 workgroups over the key/value heads (two per CU; more would run in a second round) and,
 // partials within kStaticAttentionBytes, the no-allocation entry point's buffer and the least of any other; at most
-// kSharedMaxTokens tokens a split, what a
-// split's terms take of the LDS. Past that, and for other heads, the general split attention.
+// kSharedMaxTokens tokens a split, what a split's terms take of the LDS. Past that, and for other heads, the general split
+// attention; also up to 128 tokens under more than 512 combine workgroups of 512 threads, which then take longer than the
+// splits save (224 / 32 heads of 128 lanes at 96 tokens 14.3 us, the general form 10.6; at 192 13.3 and 14.7 for 256 / 32).
 int shared_splits(int query_heads, int kv_heads, int head_dim, int tokens) {
     if (tokens <= 32 || head_dim % 32 != 0 || head_dim > 128 || query_heads / kv_heads > kSharedHeads) return 0;
+    if (tokens <= 128 && static_cast<int64_t>(query_heads) * (head_dim / 32) > 512) return 0;
     const int64_t fit = static_cast<int64_t>(kStaticAttentionBytes - static_cast<size_t>(query_heads) * head_dim * sizeof(float)) /
                         (static_cast<int64_t>(query_heads) * (2 + head_dim) * static_cast<int64_t>(sizeof(double)));
     const int most = static_cast<int>(std::min<int64_t>({512 / kv_heads, kSharedCombineThreads, fit}));
@@ -1359,11 +1361,16 @@ hipError_t launch_shared(const float* q, float* q_out, const float* k, const flo
     const int per = ((tokens + splits - 1) / splits + kSharedTile - 1) / kSharedTile * kSharedTile;
     // Query heads per workgroup: all of the key/value head's once their splits fill the chip (512 workgroups, two per
     // CU); a shorter prefix divides them evenly over more workgroups, each of whose chains is then shorter (12 / 2 heads
-    // of 128 lanes at 300 tokens 10.7 -> 8.0 us, 48 / 8 10.6 -> 8.6; at 1,500, two heads a workgroup, 10.7 -> 9.1).
+    // of 128 lanes at 300 tokens 10.7 -> 8.0 us, 48 / 8 10.6 -> 8.6; at 1,500, two heads a workgroup, 10.7 -> 9.1). Three
+    // per CU are faster where the cache is warm (256 / 32 at 300 17.1 -> 15.7) and slower in a token, whose other launches
+    // have passed through it (12 / 2 at 1,501 1.4 us a layer). Five and seven heads, which would stay together on too few
+    // workgroups, take them: 112 / 16 at 192 12.2 -> 10.2 (one workgroup per query head: 10.8), 56 / 8 at 300 11.3 -> 9.2,
+    // 20 / 4 at 1,000 10.5 -> 9.4.
     const int all = query_heads / kv_heads, dp = head_dim / 8;
     int group = all;
     for (int n : {4, 2, 1})
         if (n < all && all % n == 0 && kv_heads * splits * (all / n) <= 512) group = n;
+    if (group == all && (all == 5 || all == 7) && kv_heads * splits * all <= 768) group = 1;
     const size_t lds = sizeof(double) * (static_cast<size_t>(group) * (8 * (dp + 2) + per) +
                                          static_cast<size_t>(kSharedThreads / head_dim - 1) * group * head_dim) +
                        sizeof(float) * 2 * head_dim;

@@ -47,8 +47,10 @@ def decode_attention_launches(tokens: int, head_dim: int) -> int:
 def shares_attention(tokens: int, heads: int, kv_heads: int, head_dim: int) -> bool:
     """Whether the library attends with one workgroup per key/value head and split for all of its query heads (the
     inputs of a decoded position always inside it): heads of 32, 64, 96 or 128 lanes, at most eight per key/value
-    head, past 32 tokens, while splits of at most 256 tokens suffice."""
+    head, past 32 tokens (128 for more than 512 heads x 32 lanes), while splits of at most 256 tokens suffice."""
     if tokens <= 32 or head_dim % 32 or head_dim > 128 or heads // kv_heads > 8:
+        return False
+    if tokens <= 128 and heads * (head_dim // 32) > 512:
         return False
     fit = ((4 << 20) - 4 * heads * head_dim) // (heads * (2 + head_dim) * 8)
     most = min(512 // kv_heads, 512, fit)

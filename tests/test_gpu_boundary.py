@@ -10,6 +10,7 @@ other output the same 32 bits); attention within one unit in the last place of t
 from __future__ import annotations
 
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -674,11 +675,40 @@ def test_attention_split_of_scores_of_minus_infinity(context, heads, kv_heads, h
     assert np.array_equal(np.isnan(out), np.isnan(want))
 
 
+@pytest.mark.parametrize("few,more,kv_heads,head_dim,tokens", [(192, 224, 32, 128, 96), (96, 112, 16, 96, 192)])
+def test_attention_of_seven_heads_takes_no_step(context, few, more, kv_heads, head_dim, tokens):
+    # Seven query heads to a key/value head, which divide into no smaller groups than one: at most their share of six's time
+    # and a tenth (1.0 to 1.1 of six's measured; left whole, on too few workgroups, 1.3).
+    g = rng(7)
+    kv = g.standard_normal((tokens, kv_heads * head_dim)).astype(np.float32)
+    q = g.standard_normal(more * head_dim).astype(np.float32)
+    dq, dk, dv, out = (context.alloc(n) for n in (q.nbytes, kv.nbytes, kv.nbytes, q.nbytes))
+    context.upload(dq, q)
+    context.upload(dk, kv)
+    context.upload(dv, kv)
+    ops, best = S.DeviceOps(context), []
+    for heads in (few, more):
+        ops.grouped_attention(dq, dk, dv, heads, kv_heads, head_dim, tokens, out)
+        times = []
+        for _ in range(10):
+            context.synchronize()
+            start = time.perf_counter()
+            for _ in range(100):
+                ops.grouped_attention(dq, dk, dv, heads, kv_heads, head_dim, tokens, out)
+            context.synchronize()
+            times.append(time.perf_counter() - start)
+        best.append(min(times))
+    for p in (dq, dk, dv, out):
+        context.free(p)
+    assert best[1] <= 1.1 * 7 / 6 * best[0], best
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,tokens", [
     (1, 1, 32, 33), (2, 1, 64, 63), (6, 2, 96, 64), (4, 1, 128, 65),   # the edges of one 32-token split
     (5, 1, 128, 97), (35, 5, 32, 255), (48, 8, 96, 257), (64, 8, 64, 300),  # 1 .. 8 query heads, divided and whole
     (12, 2, 128, 2079), (7, 1, 128, 16385),   # two and three heads a workgroup; 64 tokens a split, its last partial
-    (16, 2, 128, 8129), (3, 3, 96, 40000)])   # all eight heads a workgroup; 256 tokens a split
+    (16, 2, 128, 8129), (3, 3, 96, 40000),    # all eight heads a workgroup; 256 tokens a split
+    (224, 32, 128, 96), (224, 32, 96, 129), (112, 16, 96, 192), (56, 8, 128, 300)])  # many heads: the general form, then shared
 def test_attention_shared_by_query_heads(context, heads, kv_heads, head_dim, tokens):
     # One workgroup per key/value head and split for several of its query heads: within one unit in the last place of
     # the oracle (sums in FP64, one rounding to FP32), the decode form with the same bits as its two calls, a whole
