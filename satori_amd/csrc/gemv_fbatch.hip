@@ -599,8 +599,8 @@ __global__ __launch_bounds__(64 * RH * WAYS, 2) void fbatch_kernel(FbatchArgs a)
 // Short rows under many outputs: a workgroup is one tile of 128 rows x 32 positions, W blocks a round, with as many of them
 // on a CU as fit, so that one's loads and stores pass behind another's products. (What bounds fbatch_kernel there is its
 // chain: a tile has one to nine rounds, and one workgroup a CU waits for each tile's first loads, 2.4 us a round in all.
-// A product of three tiles a workgroup, 13771 x 288 Q8_0 over 224 positions, took it 23 us, 15 with tiles twice as large, 9
-// here: whole_tiles.) Wave
+// A product of three tiles a workgroup, 13771 x 288 Q8_0 over 224 positions, took it 25.7 us, 16.4 with tiles four times as
+// large, 14.0 here.) Wave
 // (way, row tile) multiplies block W k + way of round k for 32 rows; the split activations of a round go through the LDS,
 // double-buffered, the weights straight into registers, both requested two rounds ahead. The ways' sums are added in order.
 template <int FORMAT, int W>

@@ -302,10 +302,11 @@ uint8_t* small_batch_workspace(satori_hip_context* c, size_t need, hipStream_t s
 // Scratch of a Q8_0 / Q4_0 batch on the matrix cores, or null where there is none. It is up to 34 MB and holds nothing
 // once the call's launches are done, so calls that run in order share it (two buffers in turn: partial sums written over
 // those the call before has just read took 1.5 us longer, 20.3 us and 18.7 in turn for 4096 x 4096 Q8_0 over 64
-// positions, 18.1 and 16.4 for 256 x 8192 over 256): the eager calls on the context stream the context's, the batches of a captured step the step's own (a step may be replayed on any stream), so that a call and its
-// replay take the same kernel and give the same bits. Batches elsewhere may overlap those: from 32 positions on they use
-// a buffer of the matrix's (of the largest size, so that it never moves under a graph), below it none. (In every matrix's
-// own buffer it took 40 MB instead of 6 for 4096 x 4096 over 256 positions.)
+// positions, 18.1 and 16.4 for 256 x 8192 over 256): the eager calls on the context stream the context's, the batches of
+// a captured step the step's own (a step may be replayed on any stream), so that a call and its replay take the same
+// kernel and give the same bits. Batches elsewhere may overlap those: from 32 positions on they use a buffer of the
+// matrix's (of the largest size, so that it never moves under a graph), below it none. (In every matrix's own buffer it
+// took 40 MB instead of 6 for 4096 x 4096 over 256 positions.)
 uint8_t* batch_scratch(satori_hip_matrix* m, int positions, hipStream_t stream) {
     satori_hip_context* c = m->context;
     const Shape& s = m->shape;
