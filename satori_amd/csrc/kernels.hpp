@@ -220,7 +220,7 @@ size_t kmfma_workspace_bytes(int blocks, int positions);
 // (gemv_fbatch.hip): the activations split into three exact bf16 parts, the product on the resident device layout `w`;
 // within 1e-5 * sum |w x| of the scalar reference like the single-position kernel. fbatch_pays: the position counts it
 // is used for. `parts` (fbatch_held_bytes; may be null below 32 positions) takes the split activations of large
-// products. `scratch` (fbatch_scratch_bytes) takes partial sums, which mean nothing once the call's launches are done,
+// products and of short rows under many outputs. `scratch` (fbatch_scratch_bytes) takes partial sums, which mean nothing once the call's launches are done,
 // so launches of any matrices that run in order can share it. Both sizes are for the current device.
 bool fbatch_pays(int format, int rows, int columns, int positions);
 size_t fbatch_held_bytes(int rows, int columns, int positions);
