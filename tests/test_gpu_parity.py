@@ -1005,7 +1005,7 @@ def test_legacy_matrix_core_batch(context, fmt, rows, columns, positions):
                                                     (1537, 9056, 250), (9001, 1184, 255), (2100, 1120, 250),
                                                     (9001, 288, 255), (18001, 96, 256)])
 def test_legacy_matrix_core_tiles(context, fmt, rows, columns, positions):
-    # The edges of the matrix-core batch: row groups of 128 (up to 64 positions) and 256 rows with one row more
+    # The edges of the matrix-core batch: row groups of 128 and, packed, 256 rows with one row more
     # or less, odd block counts, rounds past the last block, tiles cut into many partial sums, and counts below 32
     # on matrices large enough for it. The first and last positions hold an activation from which a tile is computed once
     # more from activations as they are (2^40), and one just below it; the bound is that of
